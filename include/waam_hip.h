@@ -530,9 +530,10 @@ typedef struct waam_step_fields {
     /* waam_quiet_bytes(nx, ny, nz, layout) bytes: per row segment (the 64 cells of one
      * wavefront along the contiguous axis) whether it ended the last two steps quiet (all GAS,
      * phi 0) or cold (SOLID below the solidus and the HAZ thresholds), the list of the segments
-     * a steady step sweeps and which of them the flag-update and stream sweeps visit, and the
-     * pull's per-lane cell masks; written by every step, contents need no initial value (the
-     * size is queried, not a layout) */
+     * a steady step sweeps and which of them the flag-update and stream sweeps visit, the
+     * full pull's per-lane cell masks, and which directions of which segments the last write
+     * into each population buffer changed, with the steady pull's list; written by every step,
+     * contents need no initial value (the size is queried, not a layout) */
     uint8_t *quiet;
     /* temperature-dependent material (params.use_tables; NULL otherwise): cp_rho_prev holds
      * the previous step's refresh_thermal_properties cp*rho (kernels.py:1710-1772), read by the
@@ -569,7 +570,9 @@ typedef struct waam_step_params {
     /* 1: run the cell sweeps of kernels 2, 4 and 7 only on the row segments whose results can
      * change: a segment is left out when every cell its stencils reach ended the previous step
      * GAS with phi exactly 0 and the segment itself ended the step before so too (both buffers
-     * of every pair then hold its results already). Honoured only on steady steps
+     * of every pair then hold its results already); and pull only the directions of the row
+     * segments whose populations can change (f_src and f_dst are then the two buffers of the
+     * step before, swapped). Honoured only on steady steps
      * (pending_stream 1, thermal_list_ready 1 or 2, arc_applied 0, forces_from_fields 0,
      * force_reset_all 0), which a caller may pass only when nothing was written between this
      * step and the waam_step_fused call before. 0: every segment is swept and the quiet record

@@ -18,8 +18,9 @@
 //   7 k_step_stream          every other cell: the previous step's pull stream, force reset;
 //                            every cell: remelt, trailing-pool and cooled-metal solidification
 // On steady steps (the row-segment record below) 2, 4 and 7 walk a list of the row segments
-// whose results can change (k_step_quiet_list builds it after 1), the pull runs ahead of 7 in
-// two launches of its own (k_step_pull_x2), and in the ZYX layout the plate's cold segments are
+// whose results can change (k_step_quiet_list builds it after 1), the pull runs after 7 over the
+// directions and segments whose populations do not stand still (k_step_pull_seg; other steps
+// pull everything ahead of 7 in launches of its own), and in the ZYX layout the plate's cold segments are
 // marched along z by k_step_thermal_plate instead of being listed.
 // Every cell value is produced by the same fp32 expression sequence as the one-kernel-per-
 // reference-kernel path, so both paths give identical bits.
@@ -312,9 +313,16 @@ __host__ __device__ inline size_t quiet_pull_offset(const Dims &d)
 {
     return (quiet_need_offset(d) + quiet_segments(d) + 255) / 256 * 256;
 }
+/* then, 256-aligned, the pull's own record (PullRec): its count on a line of its own, the change
+ * and edge words of both population buffers, and its list (every segment once, and once more by
+ * kernel 7) */
+__host__ __device__ inline size_t quiet_still_offset(const Dims &d)
+{
+    return (quiet_pull_offset(d) + (d.n() + 1) / 2 + 255) / 256 * 256;
+}
 __host__ __device__ inline size_t quiet_bytes(const Dims &d)
 {
-    return quiet_pull_offset(d) + (d.n() + 1) / 2;
+    return quiet_still_offset(d) + 256 + 4 * 4 * quiet_segments(d) + 2 * 8 * quiet_segments(d);
 }
 
 /* slices of the plate that kernel 2p marches (ZYX layout with constant material; 0 in the XYZ
@@ -379,6 +387,92 @@ __device__ __forceinline__ bool segment_active(const QuietRec &q, int bx, int j,
     return !((own == 3u) && (all & 1u));
 }
 
+/* Still populations. Most of a grid's gas populations stand still: a pull writes the words its
+ * destination buffer holds already (on 768x384x192 the words of 1 % of the gas cells change in a
+ * step: those on the lines the pool's outgoing populations travel along). A word of segment S in
+ * direction q at step n is the pull of the row at (j - e_y, k - e_z) of A(n-1), the source buffer;
+ * the destination buffer holds A(n-2), pulled from A(n-3), which is what the source buffer held
+ * before step n-1 wrote it. So direction q of S has to be pulled at step n only if step n-1
+ * changed that direction's words of the source row, or a flag the pull reads changed (between
+ * n-1 and n-3 on S and its neighbours, between n and n-2 on S). Two words per segment and
+ * population buffer hold what the last write into that buffer changed: bit q of `chg`, some word
+ * of direction q of the segment; bit q of `edge`, the word at the segment's end that the
+ * neighbouring segment along the row pulls (the last cell for a direction of positive e_x, the
+ * first for a negative one). A segment that holds a collided cell, or
+ * whose stream flags differ from those two steps before, counts as changed in every direction
+ * (kPullFull, set by kernel 7, which pulls the latter whole as well). A step that is not steady
+ * leaves every word unknown (kPullUnknown): the next steady step pulls every segment and calls
+ * every one changed, since the destination it compares with may not be a pull of A(n-1)'s
+ * predecessor; the one after pulls every segment and compares. The buffer at the lower address
+ * owns the first pair of words. */
+constexpr uint32_t kPullDirs = (1u << Q) - 1u;
+constexpr uint32_t kPullFull = 0x7fffffffu;  // bit 30: pull the segment itself whole as well
+constexpr uint32_t kPullUnknown = 0xffffffffu;
+
+struct PullRec {
+    uint32_t *chg_src, *edge_src, *chg_dst, *edge_dst;
+    int *count;
+    uint2 *list;  // (segment, directions)
+};
+
+__device__ __forceinline__ PullRec pull_rec(const waam_step_fields &f, const Dims &d)
+{
+    const size_t nseg = quiet_segments(d);
+    uint8_t *base = f.quiet + quiet_still_offset(d);
+    uint32_t *w = reinterpret_cast<uint32_t *>(base + 256);
+    const bool lower = f.f_src < f.f_dst;
+    PullRec r;
+    r.count = reinterpret_cast<int *>(base);
+    r.chg_src = w + (lower ? 0 : 2) * nseg;
+    r.edge_src = r.chg_src + nseg;
+    r.chg_dst = w + (lower ? 2 : 0) * nseg;
+    r.edge_dst = r.chg_dst + nseg;
+    r.list = reinterpret_cast<uint2 *>(w + 4 * nseg);
+    return r;
+}
+
+/* whether a steady step keeps the change words and pulls by them: rows along x only. A row
+ * segment along z crosses the plate and the film over it, so nearly all of them hold a collided
+ * cell and would be pulled whole (40x24x66: 1932 entries for 1920 segments); the full pull moves
+ * those in wider words */
+__host__ __device__ inline bool pulls_by_record(const Dims &d) { return d.layout == kLayoutZYX; }
+
+/* the directions that pull from the row at (j - dj, k - dk), and of those the ones whose step
+ * along x is sh (2: any) */
+__host__ __device__ constexpr uint32_t row_dirs(int dj, int dk, int sh)
+{
+    uint32_t m = 0;
+    for (int q = 0; q < Q; ++q)
+        if (ey(q) == dj && ez(q) == dk && (sh == 2 || ex(q) == sh)) m |= 1u << q;
+    return m;
+}
+
+/* the directions of segment (bx, j, k) that this step has to pull (x wraps, y and z clamp) */
+__device__ __forceinline__ uint32_t pull_dirs(const PullRec &r, const QuietRec &q, int bx, int j,
+                                              int k, const Dims &d)
+{
+    const int xl = bx > 0 ? bx - 1 : q.nbx - 1;
+    const int xr = bx < q.nbx - 1 ? bx + 1 : 0;
+    uint32_t m = 0, own = 0;
+#pragma unroll
+    for (int dk = -1; dk <= 1; ++dk) {
+#pragma unroll
+        for (int dj = -1; dj <= 1; ++dj) {
+            const uint32_t any = row_dirs(dj, dk, 2);
+            const uint32_t up = row_dirs(dj, dk, 1), dn = row_dirs(dj, dk, -1);
+            if (any == 0u) continue;
+            const size_t row = seg_index(q, 0, imax(0, imin(j - dj, d.ny - 1)),
+                                         imax(0, imin(k - dk, d.nz - 1)), d);
+            const uint32_t w = r.chg_src[row + bx];
+            if (dj == 0 && dk == 0) own = w;
+            m |= w & any;
+            if (up != 0u) m |= r.edge_src[row + xl] & up;
+            if (dn != 0u) m |= r.edge_src[row + xr] & dn;
+        }
+    }
+    return (own & ~kPullDirs) != 0u ? kPullDirs : m;
+}
+
 /* 1b — the active segments of a steady step, one thread per segment, appended to the list a
  * block at a time (one atomic per block; the block's segments in index order, blocks in
  * arrival order: each segment's results depend only on the sweeps' inputs, so the order is
@@ -400,22 +494,42 @@ __global__ void __launch_bounds__(kBlock) k_step_quiet_list(waam_step_fields f, 
          * which lists it only if it is no longer cold */
         if (b < KP && (q.bits[sg] & 12u) == 12u) act = false;
     }
-    __shared__ int s_cnt[kBlock / 64];
-    __shared__ int s_base;
-    const unsigned long long m = __ballot(act);
+    /* the directions the pull has to move, and the segment's change words of the buffer this
+     * step writes, started afresh */
+    const PullRec r = pull_rec(f, d);
+    uint32_t dirs = 0;
+    if (sg < nseg && pulls_by_record(d)) {
+        const int bx = (int)(sg % (size_t)q.nbx);
+        const size_t row = sg / (size_t)q.nbx;
+        dirs = pull_dirs(r, q, bx, (int)(row % (size_t)d.ny), (int)(row / (size_t)d.ny), d);
+        const uint32_t fresh = r.chg_src[sg] == kPullUnknown ? kPullFull : 0u;
+        r.chg_dst[sg] = fresh;
+        r.edge_dst[sg] = fresh;
+    }
+    __shared__ int s_cnt[2][kBlock / 64];
+    __shared__ int s_base[2];
+    const unsigned long long m = __ballot(act), mp = __ballot(dirs != 0u);
     const int lane = (int)__lane_id();
     const int wave = (int)threadIdx.x >> 6;
-    if (lane == 0) s_cnt[wave] = __popcll(m);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int tot = 0;
-        for (int w = 0; w < kBlock / 64; ++w) tot += s_cnt[w];
-        s_base = tot ? atomicAdd(q.count, tot) : 0;
+    if (lane == 0) {
+        s_cnt[0][wave] = __popcll(m);
+        s_cnt[1][wave] = __popcll(mp);
     }
     __syncthreads();
-    int base = s_base;
-    for (int w = 0; w < wave; ++w) base += s_cnt[w];
-    if (act) q.list[base + __popcll(m & ((1ull << lane) - 1ull))] = (int32_t)sg;
+    if (threadIdx.x < 2) {
+        int tot = 0;
+        for (int w = 0; w < kBlock / 64; ++w) tot += s_cnt[threadIdx.x][w];
+        s_base[threadIdx.x] = tot ? atomicAdd(threadIdx.x == 0 ? q.count : r.count, tot) : 0;
+    }
+    __syncthreads();
+    int base = s_base[0], pbase = s_base[1];
+    for (int w = 0; w < wave; ++w) {
+        base += s_cnt[0][w];
+        pbase += s_cnt[1][w];
+    }
+    const unsigned long long below = (1ull << lane) - 1ull;
+    if (act) q.list[base + __popcll(m & below)] = (int32_t)sg;
+    if (dirs != 0u) r.list[pbase + __popcll(mp & below)] = make_uint2((uint32_t)sg, dirs);
 }
 
 /* the cell of this lane in segment seg (block3() blocks: the lanes along the contiguous axis,
@@ -491,6 +605,14 @@ __device__ __forceinline__ void record_quiet(const QuietRec &q, size_t seg, bool
     }
 }
 
+/* a step that is not steady leaves the pull's record unknown for both buffers */
+__device__ __forceinline__ void forget_pull(const PullRec &r, size_t seg)
+{
+    if (threadIdx.x != 0) return;
+    r.chg_src[seg] = r.edge_src[seg] = kPullUnknown;
+    r.chg_dst[seg] = r.edge_dst[seg] = kPullUnknown;
+}
+
 /* below the solidus and both HAZ thresholds: no freeze rule and no HAZ clock acts on the cell */
 __device__ __forceinline__ float cold_limit(const waam_step_params &p)
 {
@@ -541,7 +663,10 @@ __global__ void __launch_bounds__(kBlock) k_step_begin(waam_step_fields f, StepC
     if (blockIdx.x == 0) {
         if (!p.thermal_list_ready) cell_list(f, s.d.n(), 0).count(threadIdx.x) = 0;
         cell_list(f, s.d.n(), 1).count(threadIdx.x) = 0;
-        if (p.quiet_skip && threadIdx.x == 0) *quiet_rec(f, d).count = 0;
+        if (p.quiet_skip && threadIdx.x == 0) {
+            *quiet_rec(f, d).count = 0;
+            *pull_rec(f, d).count = 0;
+        }
     }
     int best = -1;
     for (int k = threadIdx.x; k < d.nz; k += blockDim.x) {
@@ -1708,8 +1833,9 @@ __global__ void __launch_bounds__(256) k_step_stream(waam_step_fields f, StepCon
         if (j >= d.ny) return;  // the wavefront's whole row is past the grid
         bool quiet = true;
         if (in) quiet = stream_cell<E, true>(f, s, i, j, k);
-        record_quiet(q, seg_index(q, (int)blockIdx.x, j, (int)blockIdx.z, d), quiet, false,
-                     false);
+        const size_t seg = seg_index(q, (int)blockIdx.x, j, (int)blockIdx.z, d);
+        record_quiet(q, seg, quiet, false, false);
+        forget_pull(pull_rec(f, d), seg);
         return;
     }
     const int a = (int)(blockIdx.x * blockDim.x + threadIdx.x);
@@ -1744,15 +1870,20 @@ __global__ void __launch_bounds__(256) k_step_stream(waam_step_fields f, StepCon
         if (in)
             quiet = stream_rest_cell(f, s, zyx ? a : b, j, zyx ? b : a, c[t], fc[t], fp[t], T[t],
                                      phi[t], fl[t]);
-        record_quiet(q, seg_index(q, (int)blockIdx.x, j, b, d), quiet, false, false);
+        const size_t seg = seg_index(q, (int)blockIdx.x, j, b, d);
+        record_quiet(q, seg, quiet, false, false);
+        forget_pull(pull_rec(f, d), seg);
     }
 }
 
-/* 7 over the segments kernel 2 left in (the pull ran in its own launch) */
+/* 7 over the segments kernel 2 left in (the pull runs in its own launch). A segment
+ * that holds a collided cell, or whose stream flags are not those of two steps before, counts as
+ * changed in every direction; the latter is pulled whole */
 __global__ void __launch_bounds__(256) k_step_stream_seg(waam_step_fields f, StepConsts s)
 {
     const Dims &d = s.d;
     const QuietRec q = quiet_rec(f, d);
+    const PullRec r = pull_rec(f, d);
     const float T_cold = cold_limit(s.p);
     for_needed_segments(q, *q.count, [&](size_t seg) {
         int i, j, k;
@@ -1760,6 +1891,7 @@ __global__ void __launch_bounds__(256) k_step_stream_seg(waam_step_fields f, Ste
         const size_t c = in ? d.idx(i, j, k) : 0;
         const uint8_t fc = in ? f.flags_out[c] : (uint8_t)GAS;
         const uint8_t fp = in ? f.sflags_prev[c] : (uint8_t)GAS;
+        const uint8_t fpp = in ? f.sflags_next[c] : (uint8_t)GAS;  // two steps before
         const float phi = in ? f.phi[c] : 0.0f;
         /* the freeze inputs, and the cold test's */
         const bool fr = in && fc != GAS;
@@ -1771,6 +1903,14 @@ __global__ void __launch_bounds__(256) k_step_stream_seg(waam_step_fields f, Ste
          * changes it (the cooled rule rewrites the same values), so it ends the step SOLID */
         const bool cold = !in || (fc == SOLID && phi == 1.0f && fl == 0.0f && T < T_cold);
         record_quiet(q, seg, quiet, cold, true);
+        if (!pulls_by_record(d)) return;
+        const bool turned = __ballot(fc != fpp) != 0ull;
+        if (turned || __ballot(is_surface_class(fc)) != 0ull) {
+            if (threadIdx.x == 0) {
+                r.chg_dst[seg] = r.edge_dst[seg] = kPullFull;
+                if (turned) r.list[atomicAdd(r.count, 1)] = make_uint2((uint32_t)seg, kPullDirs);
+            }
+        }
     });
 }
 
@@ -2023,6 +2163,119 @@ __global__ void __launch_bounds__(256) k_step_pull_x2(waam_step_fields f, StepCo
 #pragma unroll
             for (int h = 0; h < CPL; ++h)
                 if (need[h]) o[h] = (Elem)((v[q] >> (EB * h)) & kMask);
+        }
+    }
+}
+
+/* direction tables as bit fields, two bits a direction (component + 1), for a direction known
+ * only at run time (scalar shifts instead of a table in memory) */
+__host__ __device__ constexpr uint64_t dir_bits(int axis)
+{
+    uint64_t t = 0;
+    for (int q = 0; q < Q; ++q)
+        t |= (uint64_t)((axis == 0 ? ex(q) : (axis == 1 ? ey(q) : ez(q))) + 1) << (2 * q);
+    return t;
+}
+__device__ __forceinline__ int dir_of(int axis, int q)
+{
+    constexpr uint64_t tx = dir_bits(0), ty = dir_bits(1), tz = dir_bits(2);
+    return (int)(((axis == 0 ? tx : (axis == 1 ? ty : tz)) >> (2 * q)) & 3ull) - 1;
+}
+
+/* 7b — the pull of a steady step: the listed directions of the listed segments, a wavefront per
+ * segment, kPullGroup directions' loads in flight (a whole gas segment far above the pool moves
+ * its five upward directions, so one round of loads); only words that change are stored, and
+ * what changed goes into the destination buffer's change words. 768x384x192 (fp16, 885 k
+ * segments, about 75 k listed): 43 us, and 13 us more of kernel 1b, where the full pull took 700;
+ * 512x256x128 fp32: 20 + 6 against 378. Bound by the latency of its two rounds of loads (entry
+ * and flags, then the rows) per segment. Runs after kernel 7, which leaves the step's flags
+ * before the freeze rules in sflags_next. Values are those of the full pulls (the words they
+ * would rewrite unchanged are left alone). A segment may be on the list twice: both wavefronts
+ * form the same words, and the one that finds a word different records it. */
+constexpr int kPullGroup = 5;
+
+template <class E>
+__global__ void __launch_bounds__(256) k_step_pull_seg(waam_step_fields f, StepConsts s)
+{
+    const Dims &d = s.d;
+    const QuietRec q = quiet_rec(f, d);
+    const PullRec r = pull_rec(f, d);
+    const E *src = static_cast<const E *>(f.f_src);
+    E *dst = static_cast<E *>(f.f_dst);
+    const size_t N = d.n();
+    const int nx = d.nx;
+    const int n = *r.count;
+    const int nw = (int)(gridDim.x * blockDim.y);
+    const int w0 = (int)(blockIdx.x * blockDim.y + threadIdx.y);
+    const int lane = (int)threadIdx.x;
+    for (long long t0 = w0; t0 < n; t0 += 64LL * nw) {
+        const long long tl = t0 + (long long)lane * nw;
+        const uint2 mine = tl < n ? r.list[tl] : make_uint2(0u, 0u);
+        const int cnt = (int)std::min<long long>(64, (n - t0 + nw - 1) / nw);
+        for (int it = 0; it < cnt; ++it) {
+            const uint32_t seg = (uint32_t)__builtin_amdgcn_readlane((int)mine.x, it);
+            uint32_t dirs = (uint32_t)__builtin_amdgcn_readlane((int)mine.y, it);
+            const uint32_t rowi = seg / (uint32_t)q.nbx;
+            const int bx = (int)(seg - rowi * (uint32_t)q.nbx);
+            const int k = (int)(rowi / (uint32_t)d.ny), j = (int)(rowi - (uint32_t)k * (uint32_t)d.ny);
+            const int i = imin(bx * kTileFast + lane, nx - 1);
+            const bool in = bx * kTileFast + lane < nx;
+            const size_t c = d.idx(i, j, k);
+            const uint8_t fc = f.sflags_next[c], fp = f.sflags_prev[c];
+            const bool need = in && !is_surface_class(fc) && fp != SOLID;
+            if (__ballot(need) == 0ull) continue;
+            const bool bounce = need && fp != GAS;
+            const bool any_bounce = __ballot(bounce) != 0ull;
+            /* the segment's end cells that the neighbouring segments pull */
+            const int last = imin(kTileFast, nx - bx * kTileFast) - 1;
+            uint32_t chg = 0, edge = 0;
+            while (dirs != 0u) {
+                int qs[kPullGroup];
+                E v[kPullGroup], old[kPullGroup];
+                size_t at[kPullGroup];
+#pragma unroll
+                for (int u = 0; u < kPullGroup; ++u) {
+                    qs[u] = dirs != 0u ? __builtin_ctz(dirs) : -1;
+                    dirs &= dirs - 1u;
+                }
+#pragma unroll
+                for (int u = 0; u < kPullGroup; ++u) {
+                    if (qs[u] < 0) continue;
+                    const int dq = qs[u];
+                    int ni = i - dir_of(0, dq);
+                    ni = ni < 0 ? ni + nx : (ni >= nx ? ni - nx : ni);
+                    const int nj = imax(0, imin(j - dir_of(1, dq), d.ny - 1));
+                    const int nk = imax(0, imin(k - dir_of(2, dq), d.nz - 1));
+                    at[u] = d.idx(ni, nj, nk);
+                    v[u] = src[(size_t)dq * N + at[u]];
+                    old[u] = dst[(size_t)dq * N + c];
+                }
+                if (any_bounce) {
+                    /* bounce-back off SOLID neighbours for a destination that was not GAS at
+                     * the step whose stream this is */
+#pragma unroll
+                    for (int u = 0; u < kPullGroup; ++u) {
+                        if (qs[u] <= 0) continue;
+                        const int oq = ((qs[u] - 1) ^ 1) + 1;
+                        if (bounce && f.sflags_prev[at[u]] == SOLID) v[u] = src[(size_t)oq * N + c];
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < kPullGroup; ++u) {
+                    if (qs[u] < 0) continue;
+                    const bool ch = need && v[u] != old[u];
+                    const unsigned long long m = __ballot(ch);
+                    if (m == 0ull) continue;
+                    if (ch) dst[(size_t)qs[u] * N + c] = v[u];
+                    const int sh = dir_of(0, qs[u]);
+                    chg |= 1u << qs[u];
+                    if (sh > 0 ? (m >> last) & 1ull : (sh < 0 && (m & 1ull))) edge |= 1u << qs[u];
+                }
+            }
+            if (chg != 0u && lane == 0) {
+                atomicOr(&r.chg_dst[seg], chg);
+                if (edge != 0u) atomicOr(&r.edge_dst[seg], edge);
+            }
         }
     }
 }
@@ -2377,7 +2630,8 @@ static void launch_step(const StepConsts &s, const waam_step_fields &f, hipStrea
      * faster: 727 against 718 us for the 16-bit pull of 768x384x192) */
     const bool wide = kWidePull && (f32 ? d.fast() % 2 == 0 : d.fast() % 4 == 0);
     const bool separate = seg || pair16 || (f32 ? kSeparatePull32 : kSeparatePull16);
-    if (separate && p.pending_stream)
+    const bool by_record = seg && pulls_by_record(d);
+    if (!by_record && separate && p.pending_stream)
         timed_launch(WAAM_K_PULL, [&](hipEvent_t a, hipEvent_t b) {
             if (wide) {
                 dim3 gp, bp;
@@ -2410,6 +2664,18 @@ static void launch_step(const StepConsts &s, const waam_step_fields &f, hipStrea
         else
             launch_k(capture, k_step_stream<uint16_t, true>, g3, block3(), st, a, b, f, s);
     });
+    /* a steady step pulls what does not stand still, after kernel 7 */
+    if (by_record)
+        timed_launch(WAAM_K_PULL, [&](hipEvent_t a, hipEvent_t b) {
+            if (f32)
+                launch_k(capture, k_step_pull_seg<uint32_t>,
+                         dim3(resident_blocks(k_step_pull_seg<uint32_t>, kBlock)), block3(), st, a,
+                         b, f, s);
+            else
+                launch_k(capture, k_step_pull_seg<uint16_t>,
+                         dim3(resident_blocks(k_step_pull_seg<uint16_t>, kBlock)), block3(), st, a,
+                         b, f, s);
+        });
 }
 
 }  // namespace waam
