@@ -17,27 +17,32 @@ struct ArcParams {
     int enable;
 };
 
-/* Returns false for cells the reference skips (w_dep < 1e-6); otherwise the shape weight wg
- * (Gaussian exp or Goldak pdf) and the surface weight wdep, whose product is the pass-1 term and
- * (epw*wg)*wdep the pass-2 increment. */
-__device__ __forceinline__ bool arc_cell_weights(const ArcParams &p, int i, int j, int k, float fl,
-                                                 float &wg, float &wdep)
+/* the shape weight of cell (i, j, k): Gaussian exp or Goldak pdf */
+__device__ __forceinline__ float arc_shape(const ArcParams &p, int i, int j, int k)
 {
-    wdep = arc_deposition_weight(k, p.arc_k, fl, p.pen, p.enable);
-    if (wdep < 1e-6f) return false;
     float di = (float)i - p.arc_i, dj = (float)j - p.arc_j, dk = (float)k - p.arc_k;
     if (p.kind == 0) {
         float r2 = di * di + dj * dj + dk * dk * 0.25f;
-        wg = waam_expf(-r2 * p.inv2s2);
-        return true;
+        return waam_expf(-r2 * p.inv2s2);
     }
     const float eps = 1e-6f;
     float x = di * p.sgn;
     bool front = x >= 0.0f;
     float a = front ? p.af : p.ar;
     float frac = front ? p.ff : p.fr;
-    wg = frac * waam_expf(-3.0f * ((x * x) / (a * a + eps) + (dj * dj) / (p.b * p.b + eps) +
-                                   (dk * dk) / (p.cax * p.cax + eps)));
+    return frac * waam_expf(-3.0f * ((x * x) / (a * a + eps) + (dj * dj) / (p.b * p.b + eps) +
+                                     (dk * dk) / (p.cax * p.cax + eps)));
+}
+
+/* Returns false for cells the reference skips (w_dep < 1e-6); otherwise the shape weight wg and
+ * the surface weight wdep, whose product is the pass-1 term and (epw*wg)*wdep the pass-2
+ * increment. */
+__device__ __forceinline__ bool arc_cell_weights(const ArcParams &p, int i, int j, int k, float fl,
+                                                 float &wg, float &wdep)
+{
+    wdep = arc_deposition_weight(k, p.arc_k, fl, p.pen, p.enable);
+    if (wdep < 1e-6f) return false;
+    wg = arc_shape(p, i, j, k);
     return true;
 }
 

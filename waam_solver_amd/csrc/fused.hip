@@ -221,17 +221,19 @@ __device__ __forceinline__ void list_append(bool want, size_t c, const CellList 
  * of the block calls it. Returns the list length. */
 __device__ __forceinline__ int list_prefix(const CellList &l, int *s_pref)
 {
-    int t = threadIdx.y * blockDim.x + threadIdx.x;
+    __shared__ int s_wave[kListSegments / 64];
+    const int t = threadIdx.y * blockDim.x + threadIdx.x, lane = t & 63;
     int v = imin(l.count(t), (int)l.cap(t));
+    for (int off = 1; off < 64; off <<= 1) {
+        const int add = __shfl_up(v, off);
+        if (lane >= off) v += add;
+    }
+    if (lane == 63) s_wave[t >> 6] = v;
+    __syncthreads();
+    for (int w = 0; w < (t >> 6); ++w) v += s_wave[w];
     s_pref[t + 1] = v;
     if (t == 0) s_pref[0] = 0;
     __syncthreads();
-    for (int off = 1; off < kListSegments; off <<= 1) {
-        int add = t + 1 > off ? s_pref[t + 1 - off] : 0;
-        __syncthreads();
-        s_pref[t + 1] += add;
-        __syncthreads();
-    }
     return s_pref[kListSegments];
 }
 
@@ -320,9 +322,15 @@ __host__ __device__ inline size_t quiet_still_offset(const Dims &d)
 {
     return (quiet_pull_offset(d) + (d.n() + 1) / 2 + 255) / 256 * 256;
 }
+/* then, 256-aligned, the step's arc depth weights (kernel 1): one float per slice */
+__host__ __device__ inline size_t quiet_depth_offset(const Dims &d)
+{
+    return (quiet_still_offset(d) + 256 + 4 * 4 * quiet_segments(d) + 2 * 8 * quiet_segments(d) +
+            255) / 256 * 256;
+}
 __host__ __device__ inline size_t quiet_bytes(const Dims &d)
 {
-    return quiet_still_offset(d) + 256 + 4 * 4 * quiet_segments(d) + 2 * 8 * quiet_segments(d);
+    return quiet_depth_offset(d) + 4 * (size_t)d.nz;
 }
 
 /* slices of the plate that kernel 2p marches (ZYX layout with constant material; 0 in the XYZ
@@ -695,6 +703,12 @@ __global__ void __launch_bounds__(kBlock) k_step_begin(waam_step_fields f, StepC
     ap.arc_i = at.arc_i;
     ap.arc_j = at.arc_j;
     ap.arc_k = p.use_arc_k_override ? p.arc_k_override : s_arck;
+    if (do_sums && blockIdx.x == 0) {
+        /* the surface weight of a cell that is not liquid, by slice (HView) */
+        float *depth = reinterpret_cast<float *>(f.quiet + quiet_depth_offset(d));
+        for (int k = threadIdx.x; k < d.nz; k += blockDim.x)
+            depth[k] = arc_deposition_weight(k, ap.arc_k, 0.0f, ap.pen, ap.enable);
+    }
     double sum = 0.0, comp = 0.0;
     size_t N = d.n();
     /* the arc's weights are exactly zero outside its (i, j) box (exp underflows to 0 there), so
@@ -868,6 +882,9 @@ struct HView {
     /* temperature-dependent material: the ceiling's cp*rho per cell, from the previous step's
      * refresh (clamp_enthalpy_ceiling_variable_cp, kernels.py:1987-2010) */
     const float *cp_prev;
+    /* the arc's surface weight of a cell that is not liquid, by slice: kernel 1 evaluates it once
+     * a slice, where a surface cell would form thirteen of its exponentials */
+    const float *depth;
     Dims d;
     ArcParams ap;
     float epw, H_liq, cap_l, cap_s, T_cap, T_l;
@@ -880,11 +897,14 @@ struct HView {
     {
         return arc_on && i >= box_i0 && i <= box_i1 && j >= box_j0 && j <= box_j1;
     }
-    __device__ __forceinline__ float value(float h, float fl, float cp, int i, int j, int k) const
+    /* arc heat (reference kernels.py:497-510) and the ceiling; wk: depth[k] */
+    __device__ __forceinline__ float value(float h, float fl, float cp, float wk, int i, int j,
+                                           int k) const
     {
         if (heated(i, j)) {
-            float wg, wdep;
-            if (arc_cell_weights(ap, i, j, k, fl, wg, wdep)) h += epw * wg * wdep;
+            const float wdep = fl > 0.55f ? 1.0f : wk;
+            const float hot = h + epw * arc_shape(ap, i, j, k) * wdep;
+            h = wdep < 1e-6f ? h : hot;
         }
         if (cap_on) {
             if (tab) h = ceiling_clamp(h, H_liq, H_liq + cp * (T_cap - T_l), cp * T_cap);
@@ -895,20 +915,18 @@ struct HView {
     /* f_l is read only where the arc heats */
     __device__ __forceinline__ float at(size_t c, int i, int j, int k) const
     {
-        return value(H_in[c], heated(i, j) ? fl_in[c] : 0.0f, tab ? cp_prev[c] : 0.0f, i, j, k);
+        return value(H_in[c], heated(i, j) ? fl_in[c] : 0.0f, tab ? cp_prev[c] : 0.0f,
+                     arc_on ? depth[k] : 0.0f, i, j, k);
     }
-    /* _masked_at on the enthalpy view: clamped index, GAS neighbours give the fallback (loads
-     * first, select last, so the loads are not sunk behind the flag test) */
-    __device__ __forceinline__ float masked(int i, int j, int k, float fallback) const
+    /* operand t of the upwind stencil of cell (i, j, k): axis t / 4, offsets -1, 1, -2, 2,
+     * clamped to the grid */
+    __device__ __forceinline__ void operand(int t, int i, int j, int k, int &ii, int &jj,
+                                            int &kk) const
     {
-        int ii = imax(0, imin(i, d.nx - 1));
-        int jj = imax(0, imin(j, d.ny - 1));
-        int kk = imax(0, imin(k, d.nz - 1));
-        size_t c = d.idx(ii, jj, kk);
-        uint8_t fg = flags_in[c];
-        float v = value(H_in[c], heated(ii, jj) ? fl_in[c] : 0.0f, tab ? cp_prev[c] : 0.0f, ii,
-                        jj, kk);
-        return fg == GAS ? fallback : v;
+        const int o = (t & 1 ? 1 : -1) * (t & 2 ? 2 : 1), axis = t >> 2;
+        ii = imax(0, imin(i + (axis == 0 ? o : 0), d.nx - 1));
+        jj = imax(0, imin(j + (axis == 1 ? o : 0), d.ny - 1));
+        kk = imax(0, imin(k + (axis == 2 ? o : 0), d.nz - 1));
     }
 };
 
@@ -919,6 +937,7 @@ __device__ __forceinline__ HView make_hview(const waam_step_fields &f, const Ste
     hv.H_in = f.H_in;
     hv.fl_in = f.fl_in;
     hv.flags_in = f.flags_in;
+    hv.depth = reinterpret_cast<const float *>(f.quiet + quiet_depth_offset(s.d));
     hv.d = s.d;
     const ArcStep at = arc_step(s);
     hv.ap = s.arc;
@@ -1048,18 +1067,36 @@ __device__ __forceinline__ float2 thermal_cell(const waam_step_fields &f, const 
     float H_c = hv.at(c, i, j, k);
     if (ADV && flag != SOLID) {
         float u = f.ux[c], v = f.uy[c], w = f.uz[c];
-        float H_im = hv.masked(i - 1, j, k, H_c);
-        float H_ip = hv.masked(i + 1, j, k, H_c);
-        float H_imm = hv.masked(i - 2, j, k, H_im);
-        float H_ipp = hv.masked(i + 2, j, k, H_ip);
-        float H_jm = hv.masked(i, j - 1, k, H_c);
-        float H_jp = hv.masked(i, j + 1, k, H_c);
-        float H_jmm = hv.masked(i, j - 2, k, H_jm);
-        float H_jpp = hv.masked(i, j + 2, k, H_jp);
-        float H_km = hv.masked(i, j, k - 1, H_c);
-        float H_kp = hv.masked(i, j, k + 1, H_c);
-        float H_kmm = hv.masked(i, j, k - 2, H_km);
-        float H_kpp = hv.masked(i, j, k + 2, H_kp);
+        /* the twelve operands along the axes: every load first. One masked read at a time left
+         * each behind the previous one's branches on the arc box. A list that fits the chip is
+         * bound by this chain of one lane: 20.7 us on 64x40x32, 19.0 with the loads together,
+         * 14.8 with the depth weights by slice and exps without branches (768x384x192: 47, 41) */
+        float h[12], fl[12], cp[12], wk[12];
+        uint8_t fg[12];
+#pragma unroll
+        for (int t = 0; t < 12; ++t) {
+            int ii, jj, kk;
+            hv.operand(t, i, j, k, ii, jj, kk);
+            const size_t n = d.idx(ii, jj, kk);
+            fg[t] = f.flags_in[n];
+            h[t] = f.H_in[n];
+            fl[t] = hv.arc_on ? f.fl_in[n] : 0.0f;
+            cp[t] = TAB ? f.cp_rho_prev[n] : 0.0f;
+            wk[t] = hv.arc_on ? hv.depth[kk] : 0.0f;
+        }
+#pragma unroll
+        for (int t = 0; t < 12; ++t) {
+            int ii, jj, kk;
+            hv.operand(t, i, j, k, ii, jj, kk);
+            h[t] = hv.value(h[t], fl[t], cp[t], wk[t], ii, jj, kk);
+        }
+        /* GAS operands give the next nearer one */
+        const float H_im = fg[0] == GAS ? H_c : h[0], H_ip = fg[1] == GAS ? H_c : h[1];
+        const float H_imm = fg[2] == GAS ? H_im : h[2], H_ipp = fg[3] == GAS ? H_ip : h[3];
+        const float H_jm = fg[4] == GAS ? H_c : h[4], H_jp = fg[5] == GAS ? H_c : h[5];
+        const float H_jmm = fg[6] == GAS ? H_jm : h[6], H_jpp = fg[7] == GAS ? H_jp : h[7];
+        const float H_km = fg[8] == GAS ? H_c : h[8], H_kp = fg[9] == GAS ? H_c : h[9];
+        const float H_kmm = fg[10] == GAS ? H_km : h[10], H_kpp = fg[11] == GAS ? H_kp : h[11];
         float gx = upwind_grad(u, H_imm, H_im, H_c, H_ip, H_ipp);
         float gy = upwind_grad(v, H_jmm, H_jm, H_c, H_jp, H_jpp);
         float gz = upwind_grad(w, H_kmm, H_km, H_c, H_kp, H_kpp);
@@ -1107,7 +1144,7 @@ __global__ void __launch_bounds__(256) k_step_thermal(waam_step_fields f, StepCo
     float phi_new = (in && s.p.enable_vof) ? vof_advect_cell(f, d, i, j, k, flag) : 0.0f;
     if (LIST) list_append(in && is_surface_class(flag), c, cell_list(f, s.d.n(), 0));
     if (!in || is_surface_class(flag)) return;
-    thermal_cell<TAB>(f, s, i, j, k, c, flag, h_in);
+    thermal_cell<TAB, false>(f, s, i, j, k, c, flag, h_in);
     if (s.p.enable_vof) f.phi_tmp[c] = phi_new;
 }
 
@@ -1193,6 +1230,7 @@ __global__ void __launch_bounds__(kTileFast * kPlateRows) k_step_thermal_plate(w
             tp = f.T_prev[c];
         }
     };
+    float WK = hv.arc_on && k0 < k1 ? hv.depth[k0] : 0.0f;
     if (k0 < k1) load_k(k0, hist_at(k0), Th, Fh, Tr, Fr, H, FL, TX, TP);
     for (int k = k0; k < k1; ++k) {
         const bool hist = hist_at(k);
@@ -1201,6 +1239,7 @@ __global__ void __launch_bounds__(kTileFast * kPlateRows) k_step_thermal_plate(w
         Fn = f.flags_in[idx(ic, jc, k + 2)];
         float Th1 = 0.0f, Tr1 = 0.0f, H1 = 0.0f, FL1 = 0.0f, TX1 = 0.0f, TP1 = 0.0f;
         uint8_t Fh1 = GAS, Fr1 = GAS;
+        const float WK1 = hv.arc_on && k + 1 < k1 ? hv.depth[k + 1] : 0.0f;
         if (k + 1 < k1) load_k(k + 1, hist_at(k + 1), Th1, Fh1, Tr1, Fr1, H1, FL1, TX1, TP1);
         sT[r][lane] = Tc;
         sF[r][lane] = Fc;
@@ -1251,7 +1290,7 @@ __global__ void __launch_bounds__(kTileFast * kPlateRows) k_step_thermal_plate(w
                                             (int)(i - 1 >= 0 && Fim == GAS)
                                       : 0;
                 const size_t c = d.idx(i, j, k);
-                const float H_c = hv.value(H, FL, 0.0f, i, j, k);
+                const float H_c = hv.value(H, FL, 0.0f, WK, i, j, k);
                 const float dH = conduction_dH(pr, Tc, m_im, m_ip, m_jm, m_jp, m_km, m_kp);
                 const float2 tf = thermal_finish<false>(f, s, c, Tc, H_c, dH, n_exp, pr, TX, TP,
                                                         true);
@@ -1277,6 +1316,7 @@ __global__ void __launch_bounds__(kTileFast * kPlateRows) k_step_thermal_plate(w
         Fr = Fr1;
         H = H1;
         FL = FL1;
+        WK = WK1;
         TX = TX1;
         TP = TP1;
     }

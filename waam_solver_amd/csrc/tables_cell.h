@@ -18,15 +18,25 @@ __device__ __forceinline__ float lookup_table_1d(float T, const float *t_arr, co
         } else if (T >= t_arr[n - 1]) {
             result = v_arr[n - 1];
         } else {
+            /* the last interval that holds T (as the reference's loop leaves it), then one
+             * division: a division per interval under its own branch made four lookups of a
+             * cell cost more than its thermal update */
+            float t0 = 0.0f, t1 = 0.0f, v0 = 0.0f, v1 = 0.0f;
+            bool hit = false;
 #pragma unroll
             for (int idx = 0; idx < WAAM_MAX_KNOTS - 1; ++idx) {
                 if (idx < n - 1) {
-                    float t0 = t_arr[idx], t1 = t_arr[idx + 1];
-                    if (T >= t0 && T <= t1) {
-                        float w = (T - t0) / (t1 - t0 + 1e-8f);
-                        result = v_arr[idx] + w * (v_arr[idx + 1] - v_arr[idx]);
-                    }
+                    const bool in = T >= t_arr[idx] && T <= t_arr[idx + 1];
+                    t0 = in ? t_arr[idx] : t0;
+                    t1 = in ? t_arr[idx + 1] : t1;
+                    v0 = in ? v_arr[idx] : v0;
+                    v1 = in ? v_arr[idx + 1] : v1;
+                    hit = hit || in;
                 }
+            }
+            if (hit) {
+                const float w = (T - t0) / (t1 - t0 + 1e-8f);
+                result = v0 + w * (v1 - v0);
             }
         }
     }

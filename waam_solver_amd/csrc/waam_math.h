@@ -6,8 +6,9 @@
  * (reference: kernels.py:436, :489, :510, :3082, :1173). Cell flags are decided by
  * fp32 threshold tests on fields that these exponentials feed, so a GPU kernel and a
  * CPU implementation only agree bit for bit if they evaluate exp() identically. This
- * header is that one evaluation, compiled unchanged as plain C (gcc) and as HIP device
- * code (hipcc); every other operation on the path is a single IEEE-754 operation
+ * header is that one evaluation, compiled as plain C (gcc) and as HIP device
+ * code (hipcc; the device's last scaling takes another form, equal on every one of the 2^32 words);
+ * every other operation on the path is a single IEEE-754 operation
  * (+ - * / sqrt, all correctly rounded on both targets when FMA contraction is off).
  *
  * Method (Cody & Waite, "Software Manual for the Elementary Functions", 1980):
@@ -52,9 +53,13 @@ WAAM_HD float waam_pow2i(int n)
 
 WAAM_HD float waam_expf(float x)
 {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const int in_range = x <= WAAM_EXP_INF_ABOVE && x >= WAAM_EXP_ZERO_BELOW;
+#else
     if (!(x == x)) return x + x;                         /* NaN in, NaN out */
     if (x > WAAM_EXP_INF_ABOVE) return waam_f32_from_bits(0x7f800000u);
     if (x < WAAM_EXP_ZERO_BELOW) return 0.0f;
+#endif
 
     const float LOG2E  = 1.44269502f;                     /* 1/ln2 rounded to fp32 */
     const float LN2_HI = 0.693145751953125f;              /* 45426 / 65536 */
@@ -73,9 +78,19 @@ WAAM_HD float waam_expf(float x)
     p = p * r + 1.0f;
     p = p * r + 1.0f;
 
+#if defined(__HIP_DEVICE_COMPILE__)
+    /* the same values without a branch: p * 2^n rounded once by the scaling instruction (p lies
+     * in [0.7, 1.5], so the plain form's two scalings round once too), the ends selected after.
+     * A lane's exp then costs about 20 instructions in one block; four branches around 30
+     * instructions each let no two of a cell's exps overlap */
+    const float y = __builtin_amdgcn_ldexpf(p, n);
+    const float end = x == x ? (x > 0.0f ? waam_f32_from_bits(0x7f800000u) : 0.0f) : x + x;
+    return in_range ? y : end;
+#else
     if (n > 127) return (p * waam_pow2i(127)) * waam_pow2i(n - 127);
     if (n < -126) return (p * waam_pow2i(n + 64)) * waam_pow2i(-64);
     return p * waam_pow2i(n);
+#endif
 }
 
 #endif /* WAAM_MATH_H */
