@@ -18,9 +18,11 @@
 //   7 k_step_stream          every other cell: the previous step's pull stream, force reset;
 //                            every cell: remelt, trailing-pool and cooled-metal solidification
 // On steady steps (the row-segment record below) 2, 4 and 7 walk a list of the row segments
-// whose results can change (k_step_quiet_list builds it after 1), the pull runs after 7 over the
-// directions and segments whose populations do not stand still (k_step_pull_seg; other steps
-// pull everything ahead of 7 in launches of its own), and in the ZYX layout the plate's cold segments are
+// whose results can change (k_step_quiet_list builds it after 1, with the arc total in its last
+// block), the pull runs after 5 over the directions and segments whose populations do not stand
+// still (k_step_pull_seg, with the tracers; other steps pull everything ahead of 7 in launches of
+// its own), 2 and 3 share a launch on grids that do not fill the chip (k_step_thermal_steady: a
+// steady step is then seven launches), and in the ZYX layout the plate's cold segments are
 // marched along z by k_step_thermal_plate instead of being listed.
 // Every cell value is produced by the same fp32 expression sequence as the one-kernel-per-
 // reference-kernel path, so both paths give identical bits.
@@ -290,6 +292,7 @@ __device__ __forceinline__ void cell_ijk(size_t c, const Dims &d, int &i, int &j
 struct QuietRec {
     uint8_t *bits;
     int *count;
+    int *warm;      // segments kernel 2p lists, from the list's end backwards
     int32_t *list;
     uint8_t *need;  // per list position: kernels 4 and 7 visit the segment
     int nbx;        // segments per row
@@ -348,6 +351,7 @@ __device__ __forceinline__ QuietRec quiet_rec(const waam_step_fields &f, const D
     q.nbx = quiet_nbx(d);
     q.bits = f.quiet;
     q.count = reinterpret_cast<int *>(f.quiet + quiet_count_offset(d));
+    q.warm = q.count + 1;
     q.list = reinterpret_cast<int32_t *>(f.quiet + quiet_count_offset(d) + 256);
     q.need = f.quiet + quiet_need_offset(d);
     return q;
@@ -485,7 +489,7 @@ __device__ __forceinline__ uint32_t pull_dirs(const PullRec &r, const QuietRec &
  * block at a time (one atomic per block; the block's segments in index order, blocks in
  * arrival order: each segment's results depend only on the sweeps' inputs, so the order is
  * free). One atomic per wavefront, on the one counter, took 36 against 20 us at 768x384x192. */
-__global__ void __launch_bounds__(kBlock) k_step_quiet_list(waam_step_fields f, StepConsts s)
+__device__ __forceinline__ void quiet_list(const waam_step_fields &f, const StepConsts &s)
 {
     const Dims &d = s.d;
     const QuietRec q = quiet_rec(f, d);
@@ -558,12 +562,14 @@ __device__ __forceinline__ bool seg_cell(const QuietRec &q, size_t seg, const Di
 /* a wavefront's walk over the active-segment list (entries w, w + nw, ... of a grid of nw
  * wavefronts): the entries and their segments' record bytes are loaded 64 at a time, one per
  * lane, and handed out by shuffles, so those loads drop out of each segment's chain of memory
- * round trips. body(segment, list position, record byte). */
+ * round trips; block `block` of `nblocks` walks. body(segment, list position, record byte). */
 template <class Body>
-__device__ __forceinline__ void for_listed_segments(const QuietRec &q, int n, Body &&body)
+__device__ __forceinline__ void for_listed_segments(const QuietRec &q, int block, int nblocks,
+                                                    Body &&body)
 {
-    const int nw = (int)(gridDim.x * blockDim.y);
-    const int w = (int)(blockIdx.x * blockDim.y + threadIdx.y);
+    const int n = *q.count;
+    const int nw = nblocks * (int)blockDim.y;
+    const int w = block * (int)blockDim.y + (int)threadIdx.y;
     const int lane = (int)threadIdx.x;
     for (long long t0 = w; t0 < n; t0 += 64LL * nw) {
         const long long tl = t0 + (long long)lane * nw;
@@ -576,18 +582,21 @@ __device__ __forceinline__ void for_listed_segments(const QuietRec &q, int n, Bo
     }
 }
 
-/* the same walk over the list positions kernel 2 marked needed (the cold plate left out) */
+/* the same walk over the list positions kernel 2 marked needed (the cold plate left out), then
+ * over the plate segments that warmed up this step, which kernel 2p lists from the list's end */
 template <class Body>
-__device__ __forceinline__ void for_needed_segments(const QuietRec &q, int n, Body &&body)
+__device__ __forceinline__ void for_needed_segments(const QuietRec &q, const Dims &d, Body &&body)
 {
+    const int n1 = *q.count, n = n1 + *q.warm;
+    const int tail = (int)quiet_segments(d) - 1 + n1;
     const int nw = (int)(gridDim.x * blockDim.y);
     const int w = (int)(blockIdx.x * blockDim.y + threadIdx.y);
     const int lane = (int)threadIdx.x;
     for (long long t0 = w; t0 < n; t0 += 64LL * nw) {
         const long long tl = t0 + (long long)lane * nw;
-        const bool in = tl < n;
-        const int mine = in ? q.list[tl] : 0;
-        const bool nd = in && q.need[tl] != 0;
+        const bool in = tl < n, warm = tl >= n1;
+        const int mine = in ? q.list[warm ? tail - (int)tl : (int)tl] : 0;
+        const bool nd = in && (warm || q.need[tl] != 0);
         unsigned long long m = __ballot(nd);
         while (m != 0ull) {
             const int it = __builtin_ctzll(m);
@@ -673,6 +682,7 @@ __global__ void __launch_bounds__(kBlock) k_step_begin(waam_step_fields f, StepC
         cell_list(f, s.d.n(), 1).count(threadIdx.x) = 0;
         if (p.quiet_skip && threadIdx.x == 0) {
             *quiet_rec(f, d).count = 0;
+            *quiet_rec(f, d).warm = 0;
             *pull_rec(f, d).count = 0;
         }
     }
@@ -849,7 +859,7 @@ __global__ void __launch_bounds__(kBlock) k_step_begin(waam_step_fields f, StepC
 
 /* 1b — fixed-order total of the block sums and the energy per unit weight (reference
  *      kernels.py:493-496); one block */
-__global__ void __launch_bounds__(kBlock) k_step_arc_total(waam_step_fields f, StepConsts s)
+__device__ __forceinline__ void arc_total(const waam_step_fields &f, const StepConsts &s)
 {
     __shared__ double sh_s[kBlock], sh_c[kBlock];
     const double *parts = reinterpret_cast<const double *>((char *)f.scratch + kScratchPartials);
@@ -870,6 +880,20 @@ __global__ void __launch_bounds__(kBlock) k_step_arc_total(waam_step_fields f, S
         tot[0] = w_total;
         tot[1] = epw;
     }
+}
+
+__global__ void __launch_bounds__(kBlock) k_step_arc_total(waam_step_fields f, StepConsts s)
+{
+    arc_total(f, s);
+}
+
+/* the segment list of a steady step and, in the last block, the arc total (TOTAL: the step has
+ * sums): neither needs the other, and a launch of its own cost the total 4.5 us */
+template <bool TOTAL>
+__global__ void __launch_bounds__(kBlock) k_step_quiet_list(waam_step_fields f, StepConsts s)
+{
+    if (TOTAL && blockIdx.x == gridDim.x - 1) arc_total(f, s);
+    else quiet_list(f, s);
 }
 
 /* Enthalpy of a non-GAS cell as the thermal kernel reads it: after this step's arc injection
@@ -1158,15 +1182,21 @@ __global__ void __launch_bounds__(256) k_step_thermal(waam_step_fields f, StepCo
  * are loaded), the i neighbours come from the adjacent lanes, and every load of slice k+1
  * (k+2 for T and flags) is issued before slice k's arithmetic; the slices are split into
  * kPlateChunks ranges, one per block of a column. The arithmetic is kernel 2's
- * (conduction_dH, thermal_finish). Kernel 1b leaves these segments out of the list; this
- * kernel records each cold again (12) or, visited and no longer cold, records 28 and appends it
- * to the list (kernel 2's walk then marks it for kernels 4 and 7, and kernel 7's record drops
- * bit 4). */
+ * (conduction_dH, thermal_finish). Kernel 1b leaves these segments out of the list; the march
+ * records each cold again or, no longer cold, lists it for kernels 4 and 7 at the list's end. */
 constexpr int kPlateRows = 4;
 constexpr int kPlateChunks = 3;  // slice ranges per block column (1: 77 us, 3: 72 us)
 
-__global__ void __launch_bounds__(kTileFast * kPlateRows) k_step_thermal_plate(waam_step_fields f,
-                                                                              StepConsts s)
+static_assert(kTileFast == 64 && kPlateRows == kTileJ, "the plate march takes block3() blocks");
+
+__host__ __device__ inline int plate_row_blocks(const Dims &d) { return (d.ny + kPlateRows - 1) / kPlateRows; }
+__host__ __device__ inline int plate_blocks(const Dims &d)
+{
+    return quiet_nbx(d) * plate_row_blocks(d) * kPlateChunks;
+}
+
+__device__ __forceinline__ void plate_march(const waam_step_fields &f, const StepConsts &s,
+                                            int block)
 {
     __shared__ float sT[kPlateRows][kTileFast];
     __shared__ uint8_t sF[kPlateRows][kTileFast];
@@ -1177,8 +1207,10 @@ __global__ void __launch_bounds__(kTileFast * kPlateRows) k_step_thermal_plate(w
     const float T_cold = cold_limit(p);
     const int KP = plate_slices(p, d);
     const int lane = (int)threadIdx.x, r = (int)threadIdx.y;
-    const int bx = (int)blockIdx.x;
-    const int j = (int)blockIdx.y * kPlateRows + r;
+    const int bx = block % q.nbx;
+    const int rest = block / q.nbx;
+    const int chunk = rest / plate_row_blocks(d);
+    const int j = (rest - chunk * plate_row_blocks(d)) * kPlateRows + r;
     const int i = bx * kTileFast + lane;
     const bool row_in = j < d.ny;
     const bool in = row_in && i < d.nx;
@@ -1199,9 +1231,9 @@ __global__ void __launch_bounds__(kTileFast * kPlateRows) k_step_thermal_plate(w
      * halo row's T and flag at k (and k+1 in flight), the cell's H, f_l, T_max and T_prev at k
      * (and k+1 in flight) */
     auto idx = [&](int ii, int jj, int kk) { return d.idx(ii, jj, imax(0, imin(kk, d.nz - 1))); };
-    /* the block's slices: chunk blockIdx.z of kPlateChunks */
+    /* the block's slices: one of kPlateChunks ranges */
     const int kc = (KP + kPlateChunks - 1) / kPlateChunks;
-    const int k0 = (int)blockIdx.z * kc, k1 = imin(KP, k0 + kc);
+    const int k0 = chunk * kc, k1 = imin(KP, k0 + kc);
     float Tm, Tc, Tp, Tn;
     uint8_t Fm, Fc, Fp, Fn;
     Tm = f.T_in[idx(ic, jc, k0 - 1)];
@@ -1299,8 +1331,9 @@ __global__ void __launch_bounds__(kTileFast * kPlateRows) k_step_thermal_plate(w
             const bool all_cold = __ballot(!cold) == 0ull;
             if (first && row_in) {
                 const size_t seg = seg_index(q, bx, j, k, d);
-                q.bits[seg] = all_cold ? 12u : 28u;
-                if (!all_cold) q.list[atomicAdd(q.count, 1)] = (int32_t)seg;
+                q.bits[seg] = 12u;
+                if (!all_cold)
+                    q.list[quiet_segments(d) - 1 - (size_t)atomicAdd(q.warm, 1)] = (int32_t)seg;
             }
         }
         __syncthreads();
@@ -1325,14 +1358,13 @@ __global__ void __launch_bounds__(kTileFast * kPlateRows) k_step_thermal_plate(w
 /* 2 over the active segments of a steady step (the surface cells go to kernel 3); marks which
  * of them kernels 4 and 7 visit: all but the segments that stay cold plate */
 template <bool TAB>
-__global__ void __launch_bounds__(256) k_step_thermal_seg(waam_step_fields f, StepConsts s)
+__device__ __forceinline__ void thermal_walk(const waam_step_fields &f, const StepConsts &s,
+                                             int block, int nblocks)
 {
     const Dims &d = s.d;
     const QuietRec q = quiet_rec(f, d);
     const float T_cold = cold_limit(s.p);
-    const int KP = plate_slices(s.p, d);
-    const size_t plate_row = (size_t)q.nbx * (size_t)d.ny;  // segments per slice
-    for_listed_segments(q, *q.count, [&](size_t seg, long long pos, unsigned bits) {
+    for_listed_segments(q, block, nblocks, [&](size_t seg, long long pos, unsigned bits) {
         int i, j, k;
         const bool in = seg_cell(q, seg, d, i, j, k);
         const size_t c = in ? d.idx(i, j, k) : 0;
@@ -1341,12 +1373,6 @@ __global__ void __launch_bounds__(256) k_step_thermal_seg(waam_step_fields f, St
          * both f_l buffers hold 0 */
         const bool hist = (bits & 12u) == 12u;
         bool cold = !in;
-        /* a plate slice's cold segment: kernel 2p ran it and recorded whether it is still
-         * cold (12) or not (28) */
-        if (hist && (int)(seg / plate_row) < KP) {
-            if (threadIdx.x == 0) q.need[pos] = (bits & 16u) ? 1 : 0;
-            return;
-        }
         if (hist) {
             if (in) {
                 const float2 tf = thermal_cell<TAB, false>(f, s, i, j, k, c, SOLID, 0.0f, true);
@@ -1377,6 +1403,19 @@ __global__ void __launch_bounds__(256) k_step_thermal_seg(waam_step_fields f, St
     });
 }
 
+/* the march in a launch of its own (a plate past kTogetherBlocks) */
+__global__ void __launch_bounds__(256) k_step_thermal_plate(waam_step_fields f, StepConsts s)
+{
+    plate_march(f, s, (int)blockIdx.x);
+}
+
+/* the walk in a launch of its own (temperature-dependent material, or a plate of that size) */
+template <bool TAB>
+__global__ void __launch_bounds__(256) k_step_thermal_seg(waam_step_fields f, StepConsts s)
+{
+    thermal_walk<TAB>(f, s, (int)blockIdx.x, (int)gridDim.x);
+}
+
 /* thermal chain (with enthalpy advection) and VOF advection of the listed FLUID/IFACE cells;
  * worker b of nb, 256 threads each */
 template <bool TAB>
@@ -1401,6 +1440,19 @@ template <bool TAB>
 __global__ void __launch_bounds__(256) k_step_thermal_surface(waam_step_fields f, StepConsts s)
 {
     thermal_surface_list<TAB>(f, s, blockIdx.x, gridDim.x);
+}
+
+/* 2, 2p and 3 of a steady step in one launch: the first `surface` blocks take the listed
+ * FLUID/IFACE cells (the longest chain, so first), the next `walk` the active segments, the rest
+ * the plate's cold segments. Constant material: with the tables the two inlined copies of the
+ * cell routine make the compiler copy the argument structs to private memory */
+__global__ void __launch_bounds__(256) k_step_thermal_steady(waam_step_fields f, StepConsts s,
+                                                             int surface, int walk)
+{
+    const int b = (int)blockIdx.x;
+    if (b < surface) thermal_surface_list<false>(f, s, b, surface);
+    else if (b < surface + walk) thermal_walk<false>(f, s, b - surface, walk);
+    else plate_march(f, s, b - surface - walk);
 }
 
 /* 2+3 in one launch, when the previous step's kernel 7 has listed this step's FLUID/IFACE
@@ -1541,19 +1593,32 @@ __global__ void __launch_bounds__(256) k_step_vof_flags(waam_step_fields f, Step
     list_append(in && is_surface_class(nf), c, cell_list(f, s.d.n(), 1));
 }
 
-/* 4 over the segments kernel 2 left in */
+/* 4 over the segments kernel 2 left in; writes the step's stream flags as well (they are the
+ * updated flags, which the freeze rules of kernel 7 change afterwards). A segment that holds a
+ * cell to be collided, or whose stream flags are not those of two steps before, counts as changed
+ * in every direction for the pull; the latter is pulled whole */
 __global__ void __launch_bounds__(256) k_step_vof_flags_seg(waam_step_fields f, StepConsts s)
 {
     const Dims &d = s.d;
     if (blockIdx.x == 0)  // kernel 2 has consumed the list
         cell_list(f, d.n(), 0).count(threadIdx.y * blockDim.x + threadIdx.x) = 0;
     const QuietRec q = quiet_rec(f, d);
-    for_needed_segments(q, *q.count, [&](size_t seg) {
+    const PullRec r = pull_rec(f, d);
+    for_needed_segments(q, d, [&](size_t seg) {
         int i, j, k;
         const bool in = seg_cell(q, seg, d, i, j, k);
         const size_t c = in ? d.idx(i, j, k) : 0;
+        const uint8_t fpp = in ? f.sflags_next[c] : (uint8_t)GAS;  // two steps before
         const uint8_t nf = in ? vof_flags_cell<true>(f, s, i, j, k, c) : (uint8_t)GAS;
-        list_append(in && is_surface_class(nf), c, cell_list(f, d.n(), 1));
+        if (nf != fpp) f.sflags_next[c] = nf;
+        const bool surface = is_surface_class(nf);
+        list_append(surface, c, cell_list(f, d.n(), 1));
+        if (!pulls_by_record(d)) return;
+        const bool turned = __ballot(nf != fpp) != 0ull;
+        if ((turned || __ballot(surface) != 0ull) && threadIdx.x == 0) {
+            r.chg_dst[seg] = r.edge_dst[seg] = kPullFull;
+            if (turned) r.list[atomicAdd(r.count, 1)] = make_uint2((uint32_t)seg, kPullDirs);
+        }
     });
 }
 
@@ -1840,13 +1905,14 @@ __device__ __forceinline__ bool stream_cell(const waam_step_fields &f, const Ste
  * dependent memory round trips of each cell */
 constexpr int kStreamSlices = 4;
 
+template <bool SFLAGS>  // whether it writes the stream flags (kernel 4 has, on steady steps)
 __device__ __forceinline__ bool stream_rest_cell(const waam_step_fields &f, const StepConsts &s,
                                                  int i, int j, int k, size_t c, uint8_t fc,
                                                  uint8_t fp, float T, float phi, float fl)
 {
     const waam_step_params &p = s.p;
     bool surface = is_surface_class(fc);
-    f.sflags_next[c] = fc;
+    if (SFLAGS) f.sflags_next[c] = fc;
     if (!surface && p.store_forces && !p.forces_from_fields &&
         (p.force_reset_all || is_surface_class(fp))) {
         f.Fx[c] = 0.0f;
@@ -1908,7 +1974,7 @@ __global__ void __launch_bounds__(256) k_step_stream(waam_step_fields f, StepCon
         if (b >= d.slow()) break;
         bool quiet = true;
         if (in)
-            quiet = stream_rest_cell(f, s, zyx ? a : b, j, zyx ? b : a, c[t], fc[t], fp[t], T[t],
+            quiet = stream_rest_cell<true>(f, s, zyx ? a : b, j, zyx ? b : a, c[t], fc[t], fp[t], T[t],
                                      phi[t], fl[t]);
         const size_t seg = seg_index(q, (int)blockIdx.x, j, b, d);
         record_quiet(q, seg, quiet, false, false);
@@ -1916,41 +1982,30 @@ __global__ void __launch_bounds__(256) k_step_stream(waam_step_fields f, StepCon
     }
 }
 
-/* 7 over the segments kernel 2 left in (the pull runs in its own launch). A segment
- * that holds a collided cell, or whose stream flags are not those of two steps before, counts as
- * changed in every direction; the latter is pulled whole */
+/* 7 over the segments kernel 2 left in (the pull runs in its own launch, kernel 4 has written the
+ * stream flags) */
 __global__ void __launch_bounds__(256) k_step_stream_seg(waam_step_fields f, StepConsts s)
 {
     const Dims &d = s.d;
     const QuietRec q = quiet_rec(f, d);
-    const PullRec r = pull_rec(f, d);
     const float T_cold = cold_limit(s.p);
-    for_needed_segments(q, *q.count, [&](size_t seg) {
+    for_needed_segments(q, d, [&](size_t seg) {
         int i, j, k;
         const bool in = seg_cell(q, seg, d, i, j, k);
         const size_t c = in ? d.idx(i, j, k) : 0;
         const uint8_t fc = in ? f.flags_out[c] : (uint8_t)GAS;
         const uint8_t fp = in ? f.sflags_prev[c] : (uint8_t)GAS;
-        const uint8_t fpp = in ? f.sflags_next[c] : (uint8_t)GAS;  // two steps before
         const float phi = in ? f.phi[c] : 0.0f;
         /* the freeze inputs, and the cold test's */
         const bool fr = in && fc != GAS;
         const float T = fr ? f.T_out[c] : 0.0f;
         const float fl = fr ? f.fl_out[c] : 0.0f;
         bool quiet = true;
-        if (in) quiet = stream_rest_cell(f, s, i, j, k, c, fc, fp, T, phi, fl);
+        if (in) quiet = stream_rest_cell<false>(f, s, i, j, k, c, fc, fp, T, phi, fl);
         /* SOLID after the flag update with phi 1, f_l 0 and T below the limit: no freeze rule
          * changes it (the cooled rule rewrites the same values), so it ends the step SOLID */
         const bool cold = !in || (fc == SOLID && phi == 1.0f && fl == 0.0f && T < T_cold);
         record_quiet(q, seg, quiet, cold, true);
-        if (!pulls_by_record(d)) return;
-        const bool turned = __ballot(fc != fpp) != 0ull;
-        if (turned || __ballot(is_surface_class(fc)) != 0ull) {
-            if (threadIdx.x == 0) {
-                r.chg_dst[seg] = r.edge_dst[seg] = kPullFull;
-                if (turned) r.list[atomicAdd(r.count, 1)] = make_uint2((uint32_t)seg, kPullDirs);
-            }
-        }
     });
 }
 
@@ -2222,22 +2277,69 @@ __device__ __forceinline__ int dir_of(int axis, int q)
     return (int)(((axis == 0 ? tx : (axis == 1 ? ty : tz)) >> (2 * q)) & 3ull) - 1;
 }
 
+/* 6 — advect_tracers (reference kernels.py:3206-3255) */
+__device__ __forceinline__ void advect_tracer(int p, float *__restrict__ pos, int32_t *__restrict__ active,
+                                      const float *__restrict__ ux, const float *__restrict__ uy,
+                                      const float *__restrict__ uz, const float *__restrict__ f_l,
+                                      const uint8_t *__restrict__ flags, float dx, int max_tracers,
+                                      Dims d)
+{
+    if (p >= max_tracers || active[p] != 1) return;
+    float px = pos[3 * p] / dx, py = pos[3 * p + 1] / dx, pz = pos[3 * p + 2] / dx;
+    int i = (int)px, j = (int)py, k = (int)pz;
+    if (i < 0 || i >= d.nx || j < 0 || j >= d.ny || k < 0 || k >= d.nz) {
+        active[p] = 0;
+        return;
+    }
+    size_t c = d.idx(i, j, k);
+    uint8_t fg = flags[c];
+    if (fg == GAS) {
+        active[p] = 0;
+        return;
+    }
+    if (f_l[c] < 0.05f || fg == SOLID) {
+        active[p] = 2;
+        return;
+    }
+    pos[3 * p] += ux[c] * dx;
+    pos[3 * p + 1] += uy[c] * dx;
+    pos[3 * p + 2] += uz[c] * dx;
+}
+
+__global__ void k_advect_tracers_step(float *__restrict__ pos, int32_t *__restrict__ active,
+                                      const float *__restrict__ ux, const float *__restrict__ uy,
+                                      const float *__restrict__ uz, const float *__restrict__ f_l,
+                                      const uint8_t *__restrict__ flags, float dx, int max_tracers,
+                                      Dims d)
+{
+    advect_tracer((int)(blockIdx.x * blockDim.x + threadIdx.x), pos, active, ux, uy, uz, f_l,
+                  flags, dx, max_tracers, d);
+}
+
 /* 7b — the pull of a steady step: the listed directions of the listed segments, a wavefront per
  * segment, kPullGroup directions' loads in flight (a whole gas segment far above the pool moves
  * its five upward directions, so one round of loads); only words that change are stored, and
  * what changed goes into the destination buffer's change words. 768x384x192 (fp16, 885 k
  * segments, about 75 k listed): 43 us, and 13 us more of kernel 1b, where the full pull took 700;
  * 512x256x128 fp32: 20 + 6 against 378. Bound by the latency of its two rounds of loads (entry
- * and flags, then the rows) per segment. Runs after kernel 7, which leaves the step's flags
- * before the freeze rules in sflags_next. Values are those of the full pulls (the words they
+ * and flags, then the rows) per segment. Kernel 4 left the step's flags before the
+ * freeze rules in sflags_next. The first `tracers` blocks advect the tracers (kernel 6: after the
+ * collision, before the freeze rules, as the pull; a launch of their own cost them 4.5 us). Values are those of the full pulls (the words they
  * would rewrite unchanged are left alone). A segment may be on the list twice: both wavefronts
  * form the same words, and the one that finds a word different records it. */
 constexpr int kPullGroup = 5;
 
 template <class E>
-__global__ void __launch_bounds__(256) k_step_pull_seg(waam_step_fields f, StepConsts s)
+__global__ void __launch_bounds__(256) k_step_pull_seg(waam_step_fields f, StepConsts s,
+                                                       int tracers)
 {
     const Dims &d = s.d;
+    if ((int)blockIdx.x < tracers) {
+        advect_tracer((int)(blockIdx.x * kBlock + threadIdx.y * blockDim.x + threadIdx.x),
+                      f.tracer_pos, f.tracer_active, f.ux, f.uy, f.uz, f.fl_out, f.flags_out,
+                      s.p.dx, f.max_tracers, d);
+        return;
+    }
     const QuietRec q = quiet_rec(f, d);
     const PullRec r = pull_rec(f, d);
     const E *src = static_cast<const E *>(f.f_src);
@@ -2245,8 +2347,8 @@ __global__ void __launch_bounds__(256) k_step_pull_seg(waam_step_fields f, StepC
     const size_t N = d.n();
     const int nx = d.nx;
     const int n = *r.count;
-    const int nw = (int)(gridDim.x * blockDim.y);
-    const int w0 = (int)(blockIdx.x * blockDim.y + threadIdx.y);
+    const int nw = ((int)gridDim.x - tracers) * (int)blockDim.y;
+    const int w0 = ((int)blockIdx.x - tracers) * (int)blockDim.y + (int)threadIdx.y;
     const int lane = (int)threadIdx.x;
     for (long long t0 = w0; t0 < n; t0 += 64LL * nw) {
         const long long tl = t0 + (long long)lane * nw;
@@ -2343,36 +2445,6 @@ __global__ void k_stream_pending(const E *__restrict__ src, E *__restrict__ dst,
     uint8_t fp = sfl[d.idx(i, j, k)];
     bool need = fp != SOLID;
     if (__ballot(need) != 0ull) pull_rows(src, dst, sfl, i, j, k, need, fp, d);
-}
-
-/* 6 — advect_tracers (reference kernels.py:3206-3255) */
-__global__ void k_advect_tracers_step(float *__restrict__ pos, int32_t *__restrict__ active,
-                                      const float *__restrict__ ux, const float *__restrict__ uy,
-                                      const float *__restrict__ uz, const float *__restrict__ f_l,
-                                      const uint8_t *__restrict__ flags, float dx, int max_tracers,
-                                      Dims d)
-{
-    int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= max_tracers || active[p] != 1) return;
-    float px = pos[3 * p] / dx, py = pos[3 * p + 1] / dx, pz = pos[3 * p + 2] / dx;
-    int i = (int)px, j = (int)py, k = (int)pz;
-    if (i < 0 || i >= d.nx || j < 0 || j >= d.ny || k < 0 || k >= d.nz) {
-        active[p] = 0;
-        return;
-    }
-    size_t c = d.idx(i, j, k);
-    uint8_t fg = flags[c];
-    if (fg == GAS) {
-        active[p] = 0;
-        return;
-    }
-    if (f_l[c] < 0.05f || fg == SOLID) {
-        active[p] = 2;
-        return;
-    }
-    pos[3 * p] += ux[c] * dx;
-    pos[3 * p + 1] += uy[c] * dx;
-    pos[3 * p + 2] += uz[c] * dx;
 }
 
 /* half-widths (cells) of the (i, j) box outside which the arc heat is exactly zero: exp(x) is
@@ -2564,6 +2636,23 @@ static void launch_k(bool capture, void (*k)(KArgs...), dim3 grid, dim3 block, h
     }
 }
 
+/* blocks of the surface cells and of the segment walk in k_step_thermal_steady (as many as the
+ * device holds at once, or a quarter of them, were slower on 301x157x83: 34 us against 31) */
+constexpr int kSteadySurfaceBlocks = 512;
+constexpr int kSteadyWalkBlocks = 512;
+/* Steady steps on grids whose plate march has up to this many blocks (by the grid's x and y
+ * extents, in either layout) run kernels 2, 2p and 3 in one launch.
+ * Beside the surface cells' registers (five wavefronts a SIMD instead of seven) a larger plate
+ * loses more than the overlap gives: the 3456 blocks of 768x384x192 take 147 us together and
+ * 73 + 18 + 41 apart; the 1536 of 512x256x128 52 and 31 + 12 + 15, the 600 of 301x157x83 31 and
+ * 19 + 9 + 18, the 30 of 64x40x32 16 and 8 + 7 + 15. */
+constexpr int kTogetherBlocks = 2048;
+static bool thermal_together(const Dims &d)
+{
+    return (d.nx + kTileFast - 1) / kTileFast * plate_row_blocks(d) * kPlateChunks <=
+           kTogetherBlocks;
+}
+
 /* the step's launches in order (kernels 1-7). A steady step (s.p.quiet_skip) lists its active
  * row segments after kernel 1 and runs kernels 2, 4 and 7 over that list only, with the surface
  * cells of kernel 3 and the pull in launches of their own. */
@@ -2578,12 +2667,15 @@ static void launch_step(const StepConsts &s, const waam_step_fields &f, hipStrea
     timed_launch(WAAM_K_BEGIN, [&](hipEvent_t a, hipEvent_t b) {
         launch_k(capture, k_step_begin, dim3(do_sums ? kReduceBlocks : 1), dim3(kBlock), st, a,
                  (do_sums || seg) ? nullptr : b, f, s, do_sums);
-        if (do_sums)
-            launch_k(capture, k_step_arc_total, dim3(1), dim3(kBlock), st, nullptr,
-                     seg ? nullptr : b, f, s);
-        if (seg)
-            launch_k(capture, k_step_quiet_list, dim3(grid_for(quiet_segments(d))), dim3(kBlock),
-                     st, nullptr, b, f, s);
+        const unsigned lists = grid_for(quiet_segments(d));
+        if (seg && do_sums)
+            launch_k(capture, k_step_quiet_list<true>, dim3(lists + 1), dim3(kBlock), st, nullptr,
+                     b, f, s);
+        else if (seg)
+            launch_k(capture, k_step_quiet_list<false>, dim3(lists), dim3(kBlock), st, nullptr, b,
+                     f, s);
+        else if (do_sums)
+            launch_k(capture, k_step_arc_total, dim3(1), dim3(kBlock), st, nullptr, b, f, s);
     });
     /* kernel 3 (the listed surface cells), with or without the temperature-dependent material */
     const bool tab = p.use_tables != 0;
@@ -2598,23 +2690,28 @@ static void launch_step(const StepConsts &s, const waam_step_fields &f, hipStrea
                      st, a, b, f, s);
     };
     if (seg) {
+        const unsigned plate = plate_slices(p, d) > 0 ? (unsigned)plate_blocks(d) : 0u;
+        const bool together = !tab && thermal_together(d);
         timed_launch(WAAM_K_THERMAL, [&](hipEvent_t a, hipEvent_t b) {
-            const bool plate = plate_slices(p, d) > 0;
-            if (plate)
-                launch_k(capture, k_step_thermal_plate,
-                         dim3((unsigned)quiet_nbx(d), (unsigned)((d.ny + kPlateRows - 1) / kPlateRows),
-                              (unsigned)kPlateChunks),
-                         dim3(kTileFast, kPlateRows), st, a, nullptr, f, s);
+            if (together) {
+                launch_k(capture, k_step_thermal_steady,
+                         dim3(kSteadySurfaceBlocks + kSteadyWalkBlocks + plate), block3(), st, a,
+                         b, f, s, kSteadySurfaceBlocks, kSteadyWalkBlocks);
+                return;
+            }
+            if (plate > 0)
+                launch_k(capture, k_step_thermal_plate, dim3(plate), block3(), st, a, nullptr, f, s);
+            hipEvent_t aw = plate > 0 ? nullptr : a;
             if (tab)
                 launch_k(capture, k_step_thermal_seg<true>,
-                         dim3(resident_blocks(k_step_thermal_seg<true>, kBlock)), block3(), st,
-                         plate ? nullptr : a, b, f, s);
+                         dim3(resident_blocks(k_step_thermal_seg<true>, kBlock)), block3(), st, aw,
+                         b, f, s);
             else
                 launch_k(capture, k_step_thermal_seg<false>,
                          dim3(resident_blocks(k_step_thermal_seg<false>, kBlock)), block3(), st,
-                         plate ? nullptr : a, b, f, s);
+                         aw, b, f, s);
         });
-        timed_launch(WAAM_K_THERMAL_SURFACE, launch_surface);
+        if (!together) timed_launch(WAAM_K_THERMAL_SURFACE, launch_surface);
     } else if (p.thermal_list_ready == 1) {
         /* enough list slices for about kListBlocksWithSweep workers */
         int per = (int)(g3.x * g3.y);
@@ -2656,7 +2753,8 @@ static void launch_step(const StepConsts &s, const waam_step_fields &f, hipStrea
                      dim3(resident_blocks(k_step_collide<WAAM_POP_F32>, kBlock)), dim3(kBlock), st,
                      a, b, f, s);
     });
-    if (f.max_tracers > 0)
+    const bool by_record = seg && pulls_by_record(d);
+    if (f.max_tracers > 0 && !by_record)
         timed_launch(WAAM_K_TRACERS, [&](hipEvent_t a, hipEvent_t b) {
             launch_k(capture, k_advect_tracers_step, dim3(grid_for((size_t)f.max_tracers)),
                      dim3(kBlock), st, a, b, f.tracer_pos, f.tracer_active, f.ux, f.uy, f.uz,
@@ -2670,7 +2768,6 @@ static void launch_step(const StepConsts &s, const waam_step_fields &f, hipStrea
      * faster: 727 against 718 us for the 16-bit pull of 768x384x192) */
     const bool wide = kWidePull && (f32 ? d.fast() % 2 == 0 : d.fast() % 4 == 0);
     const bool separate = seg || pair16 || (f32 ? kSeparatePull32 : kSeparatePull16);
-    const bool by_record = seg && pulls_by_record(d);
     if (!by_record && separate && p.pending_stream)
         timed_launch(WAAM_K_PULL, [&](hipEvent_t a, hipEvent_t b) {
             if (wide) {
@@ -2692,6 +2789,19 @@ static void launch_step(const StepConsts &s, const waam_step_fields &f, hipStrea
                 launch_k(capture, k_step_pull<uint16_t>, g3, block3(), st, a, b, f, s);
             }
         });
+    /* a steady step pulls what does not stand still, and advects the tracers beside it */
+    if (by_record)
+        timed_launch(WAAM_K_PULL, [&](hipEvent_t a, hipEvent_t b) {
+            const int tr = f.max_tracers > 0 ? (int)grid_for((size_t)f.max_tracers) : 0;
+            if (f32)
+                launch_k(capture, k_step_pull_seg<uint32_t>,
+                         dim3(tr + resident_blocks(k_step_pull_seg<uint32_t>, kBlock)), block3(),
+                         st, a, b, f, s, tr);
+            else
+                launch_k(capture, k_step_pull_seg<uint16_t>,
+                         dim3(tr + resident_blocks(k_step_pull_seg<uint16_t>, kBlock)), block3(),
+                         st, a, b, f, s, tr);
+        });
     timed_launch(WAAM_K_STREAM, [&](hipEvent_t a, hipEvent_t b) {
         dim3 gs(g3.x, g3.y, (unsigned)((d.slow() + kStreamSlices - 1) / kStreamSlices));
         if (seg)
@@ -2704,18 +2814,6 @@ static void launch_step(const StepConsts &s, const waam_step_fields &f, hipStrea
         else
             launch_k(capture, k_step_stream<uint16_t, true>, g3, block3(), st, a, b, f, s);
     });
-    /* a steady step pulls what does not stand still, after kernel 7 */
-    if (by_record)
-        timed_launch(WAAM_K_PULL, [&](hipEvent_t a, hipEvent_t b) {
-            if (f32)
-                launch_k(capture, k_step_pull_seg<uint32_t>,
-                         dim3(resident_blocks(k_step_pull_seg<uint32_t>, kBlock)), block3(), st, a,
-                         b, f, s);
-            else
-                launch_k(capture, k_step_pull_seg<uint16_t>,
-                         dim3(resident_blocks(k_step_pull_seg<uint16_t>, kBlock)), block3(), st, a,
-                         b, f, s);
-        });
 }
 
 }  // namespace waam
