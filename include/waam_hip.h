@@ -484,6 +484,52 @@ int waam_cadj_thermal_step(const double *lam_next, double *lam_out, double *lam_
                            const waam_adj_consts *ac, double *grads, double *lamC, double *lamB,
                            int nx, int ny, int nz, int layout, void *scratch, void *stream);
 
+/* ---- runs of rollout steps (the differentiation form; no counterpart in the reference) ------
+ * n steps of the rollouts above with frozen flags and phi in one call: the values of the
+ * per-kernel entries, in fewer launches. The state lives in slots of N = nx*ny*nz cells (u: 3 N,
+ * f: 19 N): step t reads slot t and writes slot t + 1 (stack 1), or the two slots in turn from
+ * slot0 on (stack 0). arc_i, arc_j (host, n doubles): the arc centre of each step, in cells;
+ * c.arc_i and c.arc_j are not read. */
+typedef struct waam_rollout {
+    waam_adj_consts c;
+    float h_conv, eps_rad;      /* the loss coefficients of the forward steps */
+    float gamma_lu, cos_t, sin_t, dgamma, p_sigma, p_pa, rho_phys, g_lu, beta, F_cap, u_cap,
+        omega_s, omega_b, C_darcy;
+    int32_t flow;               /* 0: no advection; 1: by u (3 N, held); 2: with the flow */
+    int32_t enable_csf, wetting, enable_hydro;
+    int32_t nx, ny, nz, layout, stack, slot0, n_active;
+    float *H, *T, *fl;          /* slots */
+    float *u, *f;               /* slots with the flow; u 3 N where it is held */
+    const uint8_t *flags;
+    const float *phi;
+    const int32_t *active;      /* the FLUID/IFACE cells (flow 1, 2) */
+    /* saved per step for the backward (stack 1), or NULL: enthalpy after the arc, after the first
+     * ceiling (with the flow), after the losses and after the floor (N each); the force before
+     * and after its clamp (3 N each, written on the listed cells) */
+    float *A, *B, *E, *F, *Fr, *Fc;
+    double *sums;               /* 2 per step when saving, else 2: the step's arc sums */
+    float *depth;               /* nz floats of workspace */
+    void *scratch;
+} waam_rollout;
+int waam_rollout_forward(const waam_rollout *r, const double *arc_i, const double *arc_j, int n,
+                         void *stream);
+/* The n steps saved in r back: lam (2 slots of N floats; slot `slot` holds dL/dH_n, the result is
+ * in slot (slot + n) & 1) and grads (3 doubles) += dL/d(eta, loss_scale, sigma scale). parts: n times
+ * 6 * 1024 doubles of workspace, step_totals: 3 n. */
+int waam_adj_rollback(const waam_rollout *r, const double *arc_i, const double *arc_j, int n,
+                      float *lam, int slot, double *parts, double *step_totals, double *grads,
+                      void *stream);
+/* The same for the coupled rollout, in binary64: lam_H, lam_u (3 N a slot), lam_f (19 N a slot;
+ * NULL without the flow) as above. lam_u, lam_f, lam_T1, lam_fl1 (N) and G (3 N) are read and
+ * written on the listed cells only and are 0 elsewhere; lamC, lamB: N doubles of workspace. */
+typedef struct waam_rollback {
+    double *lam_H, *lam_u, *lam_f, *lam_T1, *lam_fl1, *G, *lamC, *lamB, *parts, *step_totals,
+        *grads;
+    int32_t slot;
+} waam_rollback;
+int waam_cadj_rollback(const waam_rollout *r, const waam_rollback *b, const double *arc_i,
+                       const double *arc_j, int n, void *stream);
+
 /* ---- export-side fields and reductions -------------------------------------------------- */
 /* compute_vorticity_magnitude kernels.py:3380-3419: |curl u| / dt on non-GAS cells, 0 on GAS */
 int waam_compute_vorticity_magnitude(const float *ux, const float *uy, const float *uz,

@@ -89,6 +89,9 @@ SIGNATURES: dict[str, str] = {
     "waam_cadj_marangoni": "ppppdppiiiip",
     "waam_cadj_phase": "pppppplp",
     "waam_cadj_thermal_step": "ppppppppppppppppppiiiipp",
+    "waam_rollout_forward": "pppip",
+    "waam_adj_rollback": "pppipipppp",
+    "waam_cadj_rollback": "ppppip",
     "waam_graph_capture": "pppip",
     "waam_graph_capture_plan": "pppippp",
     "waam_graph_launch": "pppppp",

@@ -46,6 +46,28 @@ class AdjConsts(ctypes.Structure):
             "surface_weight")]
 
 
+class RolloutC(ctypes.Structure):
+    """include/waam_hip.h waam_rollout."""
+
+    _fields_ = ([("c", AdjConsts)] + [(n, _f) for n in (
+        "h_conv", "eps_rad", "gamma_lu", "cos_t", "sin_t", "dgamma", "p_sigma", "p_pa",
+        "rho_phys", "g_lu", "beta", "F_cap", "u_cap", "omega_s", "omega_b", "C_darcy")] +
+        [(n, ctypes.c_int32) for n in (
+            "flow", "enable_csf", "wetting", "enable_hydro", "nx", "ny", "nz", "layout", "stack",
+            "slot0", "n_active")] +
+        [(n, ctypes.c_void_p) for n in (
+            "H", "T", "fl", "u", "f", "flags", "phi", "active", "A", "B", "E", "F", "Fr", "Fc",
+            "sums", "depth", "scratch")])
+
+
+class RollbackC(ctypes.Structure):
+    """include/waam_hip.h waam_rollback."""
+
+    _fields_ = [(n, ctypes.c_void_p) for n in (
+        "lam_H", "lam_u", "lam_f", "lam_T1", "lam_fl1", "G", "lamC", "lamB", "parts",
+        "step_totals", "grads")] + [("slot", ctypes.c_int32)]
+
+
 class ThermalRollout:
     """n_steps of the thermal sub-step from the twin's current state along ``path``
     (step -> torch (x_m, y_m)), differentiable in theta."""
@@ -59,16 +81,12 @@ class ThermalRollout:
         self.n_steps, self.K = int(n_steps), max(1, int(checkpoint_every))
         self.path, self.is_welding = path, bool(is_welding)
         f = lambda: g.field(torch.float32)  # noqa: E731
-        self.H, self.T, self.fl, self.Htmp = f(), f(), f(), f()
         # the starting state is the twin's enthalpy with T and f_l from the phase map, as at
         # every later step boundary (and as the checkpoints restore it)
         self.H0, self.T0, self.fl0 = f(), f(), f()
         tensor_of(self.H0).copy_(tensor_of(g.H))
-        tensor_of(self.H).copy_(tensor_of(g.H))
-        self._phase()
-        tensor_of(self.T0).copy_(tensor_of(self.T))
-        tensor_of(self.fl0).copy_(tensor_of(self.fl))
-        self.zero_u = f()
+        kernels.update_phase(self.H0, self.T0, self.fl0, twin.cp_rho, twin.L_rho,
+                             twin.mat.T_solidus, twin.mat.T_liquidus)
         # the rollout's own copies of the frozen flags and phi: the twin may step (and the fused
         # step updates phi in place and swaps its flag buffers) between forward and backward
         self.flags = g.field(torch.uint8, np_dtype=np.int32)
@@ -79,74 +97,64 @@ class ThermalRollout:
         self.sigma0 = float(twin.sigma_cells)
         x0, y0 = path(0)
         self.arc_k = resolve_arc_k(twin, g, x0 / g.dx, y0 / g.dx)
-        self.norm_buf = torch.zeros((), dtype=torch.float32, device=g.device)
-        self.ckpt: list[tuple[torch.Tensor, torch.Tensor, torch.Tensor]] = []
+        self.shape = tuple(tensor_of(self.H0).shape)
+        self._slots = {k: self._new(2) for k in ("H", "T", "fl")}
+        self._sums = torch.empty(2, dtype=torch.float64, device=g.device)
+        self._depth = torch.empty(g.nz, dtype=torch.float32, device=g.device)
+        self.ckpt: list[torch.Tensor] = []
         self.theta = None
 
+    def _new(self, *lead) -> torch.Tensor:
+        """Uninitialised fp32 storage of `lead` fields."""
+        return torch.empty(tuple(lead) + self.shape, dtype=torch.float32,
+                           device=self.tw.grid.device)
+
+    def _arcs(self, s0: int, n: int):
+        """The arc centres (cells) of steps s0 .. s0 + n - 1, as two double arrays."""
+        dx = self.tw.grid.dx
+        pos = [self.path(s) for s in range(s0, s0 + n)]
+        return ((ctypes.c_double * n)(*[p[0] / dx for p in pos]),
+                (ctypes.c_double * n)(*[p[1] / dx for p in pos]))
+
+    def _rollout(self, bufs: dict, stack: bool, slot0: int) -> RolloutC:
+        """The call's parameters; bufs holds the state's slots and, for the backward, the saved
+        fields (the caller keeps it until the call returns)."""
+        tw, g = self.tw, self.tw.grid
+        r = RolloutC(c=self._consts(0), h_conv=self.h_conv0 * self.theta[1],
+                     eps_rad=self.eps0 * self.theta[1], nx=g.nx, ny=g.ny, nz=g.nz,
+                     layout=g.layout, stack=int(stack), slot0=slot0, flags=P(self.flags),
+                     phi=P(self.phi), sums=P(self._sums), depth=P(self._depth),
+                     scratch=P(g.scratch))
+        for name, t in bufs.items():
+            setattr(r, name, P(t))
+        return r
+
+    def _run(self, s0: int, n: int, bufs: dict, stack: bool = False, slot0: int = 0) -> None:
+        # locals, as the arcs: addressof keeps no reference
+        r = self._rollout(bufs, stack, slot0)
+        ai, aj = self._arcs(s0, n)
+        lib().call("waam_rollout_forward", ctypes.addressof(r),
+                   ctypes.addressof(ai), ctypes.addressof(aj), n,
+                   torch.cuda.current_stream().cuda_stream)
+
+    def _segments(self):
+        return [(s0, min(self.K, self.n_steps - s0)) for s0 in range(0, self.n_steps, self.K)]
+
     # ------------------------------------------------------------------ forward
-    def _step(self, n: int, theta, save=None) -> None:
-        tw, g = self.tw, self.tw.grid
-        eta, s_h, s_sig = (float(v) for v in theta)
-        H, T, fl = self.H, self.T, self.fl
-        x, y = self.path(n)
-        if self.is_welding:
-            kernels.inject_arc_heat(H, self.flags, self.phi, fl, self.norm_buf, x / g.dx, y / g.dx,
-                                    self.arc_k, tw.Q_w, self.sigma0 * s_sig, g.dt, g.dx ** 3, eta,
-                                    tw.arc_penetration_m / g.dx,
-                                    1 if tw.arc_surface_weighting else 0, g.FLAG_SOLID,
-                                    g.FLAG_GAS, scratch=g.scratch)
-        if save is not None:
-            save["A"].copy_(tensor_of(H))
-        self._ceiling(H)
-        kernels.advect_diffuse_temperature_into(H, self.Htmp, T, self.zero_u, self.zero_u,
-                                                self.zero_u, self.flags, tw.alpha_lu, 1.0,
-                                                tw.cp_rho, g.nx, g.ny, g.nz)
-        self.H, self.Htmp = self.Htmp, self.H
-        H = self.H
-        if tw.enable_heat_loss:
-            kernels.apply_thermal_boundary_losses(
-                H, T, self.flags, tw.T_amb, self.h_conv0 * s_h, self.eps0 * s_h,
-                1 if tw.enable_convection else 0, 1 if tw.enable_radiation else 0, tw.cp_rho,
-                g.dt, g.dx, tw.sigma_sb, g.FLAG_SOLID, g.FLAG_GAS, g.nx, g.ny, g.nz)
-        if save is not None:
-            save["E"].copy_(tensor_of(H))
-        if tw.enable_heat_loss:
-            kernels.clamp_enthalpy_floor_scalar(H, tw.cp_rho, self.flags, tw.T_amb, g.FLAG_GAS)
-        if save is not None:
-            save["F"].copy_(tensor_of(H))
-        self._phase()
-        self._ceiling(H)
-        self._phase()
-
-    def _ceiling(self, H) -> None:
-        tw, g = self.tw, self.tw.grid
-        if tw.enable_enthalpy_cap:
-            kernels.clamp_enthalpy_ceiling_scalar(H, self.flags, tw.cp_rho, tw.mat.T_solidus,
-                                                  tw.mat.T_liquidus, tw.T_vapor_cap_K, tw.L_rho,
-                                                  g.FLAG_GAS)
-
-    def _phase(self) -> None:
-        tw = self.tw
-        kernels.update_phase(self.H, self.T, self.fl, tw.cp_rho, tw.L_rho, tw.mat.T_solidus,
-                             tw.mat.T_liquidus)
-
-    def _load(self, H) -> None:
-        tensor_of(self.H).copy_(H)
-        self._phase()
-
     def forward(self, theta) -> tuple[torch.Tensor, torch.Tensor]:
         """Final (T, f_l) (storage order) after n_steps with parameters theta."""
         self.theta = tuple(float(v) for v in theta)
         self.ckpt = []
-        tensor_of(self.H).copy_(tensor_of(self.H0))
-        tensor_of(self.T).copy_(tensor_of(self.T0))
-        tensor_of(self.fl).copy_(tensor_of(self.fl0))
-        for n in range(self.n_steps):
-            if n % self.K == 0:
-                self.ckpt.append(tensor_of(self.H).clone())
-            self._step(n, self.theta)
-        self.H_final = tensor_of(self.H).clone()
-        return tensor_of(self.T).clone(), tensor_of(self.fl).clone()
+        sl = self._slots
+        for name, src in (("H", self.H0), ("T", self.T0), ("fl", self.fl0)):
+            sl[name][0].copy_(tensor_of(src))
+        slot = 0
+        for s0, n in self._segments():
+            self.ckpt.append(sl["H"][slot].clone())
+            self._run(s0, n, sl, slot0=slot)
+            slot = (slot + n) & 1
+        self.H_final = sl["H"][slot].clone()
+        return sl["T"][slot].clone(), sl["fl"][slot].clone()
 
     # ------------------------------------------------------------------ backward
     def _consts(self, n: int) -> AdjConsts:
@@ -175,14 +183,12 @@ class ThermalRollout:
             raise RuntimeError("backward before forward")
         tw, g = self.tw, self.tw.grid
         st = torch.cuda.current_stream().cuda_stream
-        dev = tensor_of(self.H).device
-        n_cells = g.n_cells
-        shp = tensor_of(self.H).shape
-        lam = torch.empty(shp, dtype=torch.float32, device=dev)
-        lam2 = torch.empty_like(lam)
-        lamC = torch.empty_like(lam)
+        dev = g.device
+        L = min(self.K, self.n_steps)
+        lam = self._new(2)
         grads = torch.zeros(3, dtype=torch.float64, device=dev)
-        sums = torch.zeros(2, dtype=torch.float64, device=dev)
+        parts = torch.empty(L * 6 * 1024, dtype=torch.float64, device=dev)
+        totals = torch.empty(L * 3, dtype=torch.float64, device=dev)
         c_last = self._consts(self.n_steps - 1)
         # P() hands over a bare address: the converted seeds are held in locals until the
         # kernels that read them are queued (a temporary would be freed, and its memory reused,
@@ -190,32 +196,24 @@ class ThermalRollout:
         gT = grad_T.float().contiguous()
         gfl = grad_fl.float().contiguous()
         lib().call("waam_adj_terminal", P(self.H_final), P(gT), P(gfl), P(self.flags),
-                   ctypes.addressof(c_last), P(lam), n_cells, st)
-        seg_len = self.K
-        for s_idx in reversed(range(len(self.ckpt))):
-            s0 = s_idx * seg_len
-            s1 = min(self.n_steps, s0 + seg_len)
-            L = s1 - s0
-            Hs = torch.empty((L,) + tuple(shp), dtype=torch.float32, device=dev)
-            fls = torch.empty_like(Hs)
-            As, Es, Fs = torch.empty_like(Hs), torch.empty_like(Hs), torch.empty_like(Hs)
-            self._load(self.ckpt[s_idx])
-            for t in range(L):
-                Hs[t].copy_(tensor_of(self.H))
-                fls[t].copy_(tensor_of(self.fl))
-                self._step(s0 + t, self.theta, save={"A": As[t], "E": Es[t], "F": Fs[t]})
-            for t in reversed(range(L)):
-                n = s0 + t
-                c = self._consts(n)
-                if self.is_welding:
-                    lib().call("waam_adj_arc_sums", P(self.flags), P(fls[t]), ctypes.addressof(c),
-                               P(sums), g.nx, g.ny, g.nz, g.layout, P(g.scratch), st)
-                lib().call("waam_adj_thermal_step", P(lam), P(lam2), P(Hs[t]), P(As[t]),
-                           P(Es[t]), P(Fs[t]), P(fls[t]), P(self.flags), P(sums),
-                           ctypes.addressof(c), P(grads), P(lamC), g.nx, g.ny, g.nz, g.layout,
-                           P(g.scratch), st)
-                lam, lam2 = lam2, lam
-        self.lam0 = lam
+                   ctypes.addressof(c_last), P(lam), g.n_cells, st)
+        # a segment's state and saved fields, one slot a step, reused from segment to segment
+        sv = {k: self._new(L + 1) for k in ("H", "T", "fl")}
+        sv.update({k: self._new(L) for k in ("A", "E", "F")})
+        sv["sums"] = torch.empty(2 * L, dtype=torch.float64, device=dev)
+        slot = 0
+        for (s0, n), H in zip(reversed(self._segments()), reversed(self.ckpt)):
+            sv["H"][0].copy_(H)
+            lib().call("waam_update_phase", P(sv["H"]), P(sv["T"]), P(sv["fl"]), tw.cp_rho,
+                       tw.L_rho, tw.mat.T_solidus, tw.mat.T_liquidus, g.n_cells, st)
+            self._run(s0, n, sv, stack=True)
+            ai, aj = self._arcs(s0, n)
+            r = self._rollout(sv, True, 0)
+            lib().call("waam_adj_rollback", ctypes.addressof(r),
+                       ctypes.addressof(ai), ctypes.addressof(aj), n, P(lam), slot, P(parts),
+                       P(totals), P(grads), st)
+            slot = (slot + n) & 1
+        self.lam0 = lam[slot]
         return grads.cpu().numpy()
 
 
@@ -368,14 +366,8 @@ class CoupledRollout:
         self.tw, g = twin, twin.grid
         self.n_steps, self.K = int(n_steps), max(1, int(checkpoint_every))
         self.path, self.is_welding = path, bool(is_welding)
-        f = lambda: g.field(torch.float32)  # noqa: E731
-        fp = lambda: g.field(torch.float32, leading=(19,))  # noqa: E731
-        self.H, self.T, self.fl, self.Htmp = f(), f(), f(), f()
-        self.rho, self.ux, self.uy, self.uz = f(), f(), f(), f()
-        self.Fx, self.Fy, self.Fz = f(), f(), f()
-        self.fa, self.fb = fp(), fp()
         self.flags = g.field(torch.uint8, np_dtype=np.int32)
-        self.phi = f()
+        self.phi = g.field(torch.float32)
         tensor_of(self.flags).copy_(tensor_of(g.flags))
         tensor_of(self.phi).copy_(tensor_of(g.phi))
         # the starting state: the twin's enthalpy (T, f_l from the phase map), populations and
@@ -383,236 +375,128 @@ class CoupledRollout:
         self.H0 = tensor_of(g.H).clone()
         self.f0 = tensor_of(g.f_src).clone()
         self.u0 = [tensor_of(x).clone() for x in (g.ux, g.uy, g.uz)]
-        self.zero_u = f()
-        # the velocity the enthalpy is advected by when it does not evolve
-        self.u_adv = None
-        if advection == "frozen":
-            self.u_adv = [f() for _ in range(3)]
-            for d_, s_ in zip(self.u_adv, self.u0):
-                tensor_of(d_).copy_(s_)
-        elif advection == "none":
-            self.u_adv = [self.zero_u] * 3
+        self.shape = tuple(self.H0.shape)
+        # the FLUID/IFACE cells (the flags are held): the flow runs over them, and populations
+        # and velocity are only read and written there
+        fl = tensor_of(self.flags).reshape(-1)
+        self._cells = torch.nonzero((fl == g.FLAG_FLUID) | (fl == g.FLAG_IFACE)).reshape(-1)
+        self._active = self._cells.to(torch.int32)
+        self._slots = {k: self._new(2) for k in ("H", "T", "fl")}
+        if advection == "flow":
+            self._slots["u"], self._slots["f"] = self._new(2, 3), self._new(2, 19)
+        elif advection == "frozen":
+            # the velocity the enthalpy is advected by when it does not evolve
+            self._slots["u"] = torch.stack(self.u0)
+        self._sums = torch.empty(2, dtype=torch.float64, device=g.device)
+        self._depth = torch.empty(g.nz, dtype=torch.float32, device=g.device)
         self.h_conv0, self.eps0 = float(twin.h_conv), float(twin.eps_rad)
         self.sigma0 = float(twin.sigma_cells)
         x0, y0 = path(0)
         self.arc_k = resolve_arc_k(twin, g, x0 / g.dx, y0 / g.dx)
-        self.norm_buf = torch.zeros((), dtype=torch.float32, device=g.device)
         self.u_cap = float(getattr(twin, "u_mach_limit_lu", 0.08))
         self.F_cap = float(getattr(twin, "force_limit_lu", 0.05))
         self.ckpt: list = []
         self.theta = None
 
-    # ------------------------------------------------------------------ forward
-    def _state_in(self, H, fpop, u) -> None:
-        tensor_of(self.H).copy_(H)
-        tensor_of(self.fa).copy_(fpop)
-        for d, s in zip((self.ux, self.uy, self.uz), u):
-            tensor_of(d).copy_(s)
-        self._phase()
-
-    def _state_out(self):
-        return (tensor_of(self.H).clone(), tensor_of(self.fa).clone(),
-                [tensor_of(x).clone() for x in (self.ux, self.uy, self.uz)])
-
-    def _phase(self) -> None:
+    def _rollout(self, bufs: dict, stack: bool, slot0: int) -> RolloutC:
+        r = ThermalRollout._rollout(self, bufs, stack, slot0)
         tw = self.tw
-        kernels.update_phase(self.H, self.T, self.fl, tw.cp_rho, tw.L_rho, tw.mat.T_solidus,
-                             tw.mat.T_liquidus)
+        r.flow = {"none": 0, "frozen": 1, "flow": 2}[self.advection]
+        r.active, r.n_active = P(self._active), self._active.numel()
+        r.enable_csf, r.wetting = int(bool(tw.enable_csf_tension)), int(bool(tw.enable_wetting))
+        r.enable_hydro = int(bool(tw.enable_hydrostatic_gravity))
+        r.gamma_lu, r.dgamma = tw.gamma_lu, tw.dgamma_dT_lu
+        r.cos_t, r.sin_t = kernels.contact_angle_cos_sin(tw.theta_rad)
+        r.p_sigma = weld_forces.arc_pressure_sigma_cells(tw)
+        r.p_pa = weld_forces.arc_pressure_peak_pa(tw)
+        r.rho_phys, r.g_lu, r.beta = tw.mat.rho, tw.g_lu, tw.beta_T
+        r.F_cap, r.u_cap = self.F_cap, self.u_cap
+        r.omega_s, r.omega_b, r.C_darcy = tw.omega, tw.omega_bulk, tw.C_darcy
+        return r
 
-    def _ceiling(self) -> None:
+    def _cells_of(self, t: torch.Tensor) -> torch.Tensor:
+        """The listed cells' values of a stack of fields, (fields, cells)."""
+        return t.reshape(-1, self.tw.grid.n_cells)[:, self._cells]
+
+    def _put(self, bufs: dict, H, fc, uc) -> None:
+        """A state (H, and with the flow the listed cells' populations and velocity) into slot 0:
+        T and f_l from the phase map."""
         tw, g = self.tw, self.tw.grid
-        if tw.enable_enthalpy_cap:
-            kernels.clamp_enthalpy_ceiling_scalar(self.H, self.flags, tw.cp_rho,
-                                                  tw.mat.T_solidus, tw.mat.T_liquidus,
-                                                  tw.T_vapor_cap_K, tw.L_rho, g.FLAG_GAS)
+        bufs["H"][0].copy_(H)
+        lib().call("waam_update_phase", P(bufs["H"]), P(bufs["T"]), P(bufs["fl"]), tw.cp_rho,
+                   tw.L_rho, tw.mat.T_solidus, tw.mat.T_liquidus, g.n_cells,
+                   torch.cuda.current_stream().cuda_stream)
+        if self.advection == "flow":
+            for name, v in (("f", fc), ("u", uc)):
+                bufs[name][0].reshape(-1, g.n_cells)[:, self._cells] = v
 
-    def _step(self, n: int, theta, save=None) -> None:
-        tw, g = self.tw, self.tw.grid
-        eta, s_h, s_sig = (float(v) for v in theta)
-        x, y = self.path(n)
-        arc_i, arc_j = x / g.dx, y / g.dx
-        sv = ((lambda k, t: save[k].copy_(tensor_of(t)) if k in save else None)
-              if save is not None else None)
-        if sv:
-            sv("H", self.H)
-            sv("fl", self.fl)
-            for a, u in zip(("ux", "uy", "uz"), (self.ux, self.uy, self.uz)):
-                sv(a, u)
-        if self.is_welding:
-            kernels.inject_arc_heat(self.H, self.flags, self.phi, self.fl, self.norm_buf, arc_i,
-                                    arc_j, self.arc_k, tw.Q_w, self.sigma0 * s_sig, g.dt,
-                                    g.dx ** 3, eta, tw.arc_penetration_m / g.dx,
-                                    1 if tw.arc_surface_weighting else 0, g.FLAG_SOLID,
-                                    g.FLAG_GAS, scratch=g.scratch)
-        if sv:
-            sv("A", self.H)
-        self._ceiling()
-        if sv:
-            sv("B", self.H)
-        ua = self.u_adv or (self.ux, self.uy, self.uz)
-        kernels.advect_diffuse_temperature_into(self.H, self.Htmp, self.T, ua[0], ua[1], ua[2],
-                                                self.flags, tw.alpha_lu, 1.0, tw.cp_rho, g.nx,
-                                                g.ny, g.nz)
-        self.H, self.Htmp = self.Htmp, self.H
-        if tw.enable_heat_loss:
-            kernels.apply_thermal_boundary_losses(
-                self.H, self.T, self.flags, tw.T_amb, self.h_conv0 * s_h, self.eps0 * s_h,
-                1 if tw.enable_convection else 0, 1 if tw.enable_radiation else 0, tw.cp_rho,
-                g.dt, g.dx, tw.sigma_sb, g.FLAG_SOLID, g.FLAG_GAS, g.nx, g.ny, g.nz)
-        if sv:
-            sv("E", self.H)
-        if tw.enable_heat_loss:
-            kernels.clamp_enthalpy_floor_scalar(self.H, tw.cp_rho, self.flags, tw.T_amb,
-                                                g.FLAG_GAS)
-        if sv:
-            sv("F", self.H)
-        self._phase()
-        self._ceiling()
-        self._phase()
-        if self.advection != "flow":
-            return
-        # forces on the new temperature and liquid fraction
-        kernels.clear_forces(self.Fx, self.Fy, self.Fz)
-        if tw.enable_csf_tension:
-            kernels.compute_csf_tension(self.phi, self.flags, self.Fx, self.Fy, self.Fz,
-                                        tw.gamma_lu, g.FLAG_SOLID, g.FLAG_GAS, g.nx, g.ny, g.nz,
-                                        int(tw.enable_wetting), tw.theta_rad)
-        kernels.compute_marangoni_force(self.T, self.phi, self.fl, self.Fx, self.Fy, self.Fz,
-                                        self.flags, tw.dgamma_dT_lu, g.dx, g.FLAG_SOLID,
-                                        g.FLAG_GAS, g.nx, g.ny, g.nz)
-        if self.is_welding:
-            kernels.apply_arc_pressure(self.Fz, self.flags, self.phi, arc_i, arc_j, self.arc_k,
-                                       weld_forces.arc_pressure_sigma_cells(tw),
-                                       weld_forces.arc_pressure_peak_pa(tw), g.dt, g.dx,
-                                       tw.mat.rho, g.FLAG_SOLID, g.FLAG_GAS)
-        if tw.enable_hydrostatic_gravity:
-            kernels.add_hydrostatic_gravity(self.Fz, self.fl, self.flags, 1.0, tw.g_lu,
-                                            g.FLAG_SOLID, g.FLAG_GAS)
-        kernels.add_buoyancy(self.T, self.Fz, self.fl, self.flags, tw.g_lu, tw.beta_T,
-                             tw.mat.T_liquidus, 1.0, g.FLAG_SOLID, g.FLAG_GAS)
-        if sv:
-            for a, fld in zip(("Frx", "Fry", "Frz"), (self.Fx, self.Fy, self.Fz)):
-                sv(a, fld)
-        if self.F_cap > 0.0:
-            kernels.clamp_body_force_magnitude(self.Fx, self.Fy, self.Fz, self.flags, self.F_cap,
-                                               g.FLAG_SOLID, g.FLAG_GAS)
-        if sv:
-            for a, fld in zip(("Fx", "Fy", "Fz"), (self.Fx, self.Fy, self.Fz)):
-                sv(a, fld)
-            sv("f", self.fa)
-            sv("H1", self.H)
-            sv("T1", self.T)
-            sv("fl1", self.fl)
-        kernels.collide_mrt(self.fa, self.fb, self.rho, self.ux, self.uy, self.uz, self.Fx,
-                            self.Fy, self.Fz, self.fl, self.flags, None, None, None, None, None,
-                            tw.omega, tw.omega_bulk, tw.C_darcy, g.FLAG_SOLID, g.FLAG_GAS, g.nx,
-                            g.ny, g.nz)
-        if self.u_cap > 0.0:
-            kernels.clamp_velocity_mach(self.ux, self.uy, self.uz, self.flags, self.u_cap,
-                                        g.FLAG_SOLID, g.FLAG_GAS)
-        self.fa, self.fb = self.fb, self.fa
-
+    # ------------------------------------------------------------------ forward
     def forward(self, theta) -> tuple[torch.Tensor, torch.Tensor]:
         """Final (T, f_l) (storage order) after n_steps with parameters theta."""
         self.theta = tuple(float(v) for v in theta)
         self.ckpt = []
-        self._state_in(self.H0, self.f0, self.u0)
-        for n in range(self.n_steps):
-            if n % self.K == 0:
-                self.ckpt.append(self._state_out())
-            self._step(n, self.theta)
-        self.H_final = tensor_of(self.H).clone()
-        return tensor_of(self.T).clone(), tensor_of(self.fl).clone()
+        sl, flow = self._slots, self.advection == "flow"
+        self._put(sl, self.H0, self._cells_of(self.f0), self._cells_of(torch.stack(self.u0)))
+        slot = 0
+        for s0, n in self._segments():
+            self.ckpt.append((sl["H"][slot].clone(),) + (
+                (self._cells_of(sl["f"][slot]), self._cells_of(sl["u"][slot])) if flow
+                else (None, None)))
+            self._run(s0, n, sl, slot0=slot)
+            slot = (slot + n) & 1
+        self.H_final = sl["H"][slot].clone()
+        return sl["T"][slot].clone(), sl["fl"][slot].clone()
 
     # ------------------------------------------------------------------ backward
-    _SAVE = ("H", "fl", "ux", "uy", "uz", "A", "B", "E", "F", "Frx", "Fry", "Frz", "Fx", "Fy",
-             "Fz", "H1", "T1", "fl1")
-
     def backward(self, grad_T: torch.Tensor, grad_fl: torch.Tensor) -> np.ndarray:
         """dL/dtheta (float64) given dL/dT and dL/df_l at the final step."""
         if self.theta is None:
             raise RuntimeError("backward before forward")
-        tw, g = self.tw, self.tw.grid
+        g = self.tw.grid
         st = torch.cuda.current_stream().cuda_stream
-        dev = tensor_of(self.H).device
-        N = g.n_cells
-        shp = tuple(tensor_of(self.H).shape)
-        d64 = dict(dtype=torch.float64, device=dev)
-        flow = self.advection == "flow"
-        lam_H = torch.zeros(shp, **d64)
-        lam_Ho = torch.empty(shp, **d64)
-        lam_u = torch.zeros((3,) + shp, **d64)
-        lam_uo = torch.empty((3,) + shp, **d64)
-        lamC = torch.empty(shp, **d64)
-        lamB = torch.empty(shp, **d64)
-        grads = torch.zeros(3, **d64)
-        sums = torch.zeros(2, **d64)
+        shp = self.shape
+        d64 = dict(dtype=torch.float64, device=g.device)
+        flow, adv = self.advection == "flow", self.advection != "none"
+        L = min(self.K, self.n_steps)
+        z = lambda *lead: torch.zeros(lead + shp, **d64)  # noqa: E731
+        lam = {"lam_H": z(2), "lamC": torch.empty(shp, **d64), "lamB": torch.empty(shp, **d64),
+               "parts": torch.empty(L * 6 * 1024, **d64), "step_totals": torch.empty(3 * L, **d64),
+               "grads": torch.zeros(3, **d64)}
+        if adv:
+            lam["lam_u"] = z(2, 3)
         if flow:
-            lam_f = torch.zeros((19,) + shp, **d64)
-            lam_fin = torch.empty((19,) + shp, **d64)
-            lam_F = torch.empty((3,) + shp, **d64)
-            lam_Fr = torch.empty((3,) + shp, **d64)
-            lam_T1 = torch.empty(shp, **d64)
-            lam_fl1 = torch.empty(shp, **d64)
-            G = torch.empty((3,) + shp, **d64)
+            # zero outside the listed cells, and never written there
+            lam.update(lam_f=z(2, 19), lam_T1=z(), lam_fl1=z(), G=z(3))
         c_last = self._consts(self.n_steps - 1)
         # the binary64 seeds live in locals while their kernel is queued (P() keeps no reference)
         gT = grad_T.double().contiguous()
         gfl = grad_fl.double().contiguous()
         lib().call("waam_cadj_phase", P(self.H_final), P(self.flags), ctypes.addressof(c_last),
-                   P(gT), P(gfl), P(lam_H), N, st)
-        keys = self._SAVE if flow else ("H", "fl", "A", "B", "E", "F")
-        for s_idx in reversed(range(len(self.ckpt))):
-            s0 = s_idx * self.K
-            s1 = min(self.n_steps, s0 + self.K)
-            L = s1 - s0
-            sv = {k: torch.empty((L,) + shp, dtype=torch.float32, device=dev) for k in keys}
-            if flow:
-                sv["f"] = torch.empty((L, 19) + shp, dtype=torch.float32, device=dev)
-            self._state_in(*self.ckpt[s_idx])
-            for t in range(L):
-                self._step(s0 + t, self.theta, save={k: v[t] for k, v in sv.items()})
-            for t in reversed(range(L)):
-                c = self._consts(s0 + t)
-                if flow:
-                    # collision (with the Mach clamp) -> lam_f of the step's populations,
-                    # lam_F and f_l
-                    lam_fl1.zero_()
-                    lam_T1.zero_()
-                    lib().call("waam_cadj_collide_mrt", P(sv["f"][t]), P(sv["Fx"][t]),
-                               P(sv["Fy"][t]), P(sv["Fz"][t]), P(sv["fl1"][t]), P(self.flags),
-                               P(lam_f), P(lam_u), tw.omega, tw.omega_bulk, tw.C_darcy,
-                               self.u_cap, P(lam_fin), P(lam_F), P(lam_fl1), N, st)
-                    lib().call("waam_cadj_forces", P(sv["Frx"][t]), P(sv["Fry"][t]),
-                               P(sv["Frz"][t]), P(sv["T1"][t]), P(sv["fl1"][t]), P(self.flags),
-                               P(lam_F), self.F_cap, tw.g_lu, tw.beta_T, tw.mat.T_liquidus,
-                               1 if tw.enable_hydrostatic_gravity else 0, P(lam_Fr), P(lam_T1),
-                               P(lam_fl1), N, st)
-                    lib().call("waam_cadj_marangoni", P(self.phi), P(sv["fl1"][t]),
-                               P(self.flags), P(lam_Fr), tw.dgamma_dT_lu, P(G), P(lam_T1), g.nx,
-                               g.ny, g.nz, g.layout, st)
-                    lib().call("waam_cadj_phase", P(sv["H1"][t]), P(self.flags),
-                               ctypes.addressof(c), P(lam_T1), P(lam_fl1), P(lam_H), N, st)
-                    ua = (sv["ux"][t], sv["uy"][t], sv["uz"][t])
-                else:
-                    ua = tuple(tensor_of(x) for x in self.u_adv)
-                # the thermal chain with advection -> lam_H and lam_u of the step's start
-                if self.is_welding:
-                    lib().call("waam_adj_arc_sums", P(self.flags), P(sv["fl"][t]),
-                               ctypes.addressof(c), P(sums), g.nx, g.ny, g.nz, g.layout,
-                               P(g.scratch), st)
-                lib().call("waam_cadj_thermal_step", P(lam_H), P(lam_Ho), P(lam_uo),
-                           P(sv["H"][t]), P(sv["A"][t]), P(sv["B"][t]), P(sv["E"][t]),
-                           P(sv["F"][t]), P(sv["fl"][t]), P(ua[0]), P(ua[1]), P(ua[2]),
-                           P(self.flags), P(sums), ctypes.addressof(c), P(grads), P(lamC),
-                           P(lamB), g.nx, g.ny, g.nz, g.layout, P(g.scratch), st)
-                lam_H, lam_Ho = lam_Ho, lam_H
-                if flow:
-                    lam_u, lam_uo = lam_uo, lam_u
-                    lam_f, lam_fin = lam_fin, lam_f
-            del sv
-        self.lam0 = lam_H
-        return grads.cpu().numpy()
+                   P(gT), P(gfl), P(lam["lam_H"]), g.n_cells, st)
+        # a segment's state and saved fields, one slot a step, reused from segment to segment
+        sv = {k: self._new(L + 1) for k in ("H", "T", "fl")}
+        sv.update({k: self._new(L) for k in (("A", "B", "E", "F") if adv else ("A", "E", "F"))})
+        if flow:
+            sv.update(u=self._new(L + 1, 3), f=self._new(L + 1, 19), Fr=self._new(L, 3),
+                      Fc=self._new(L, 3))
+        elif adv:
+            sv["u"] = self._slots["u"]
+        sv["sums"] = torch.empty(2 * L, **d64)
+        slot = 0
+        for (s0, n), state in zip(reversed(self._segments()), reversed(self.ckpt)):
+            self._put(sv, *state)
+            self._run(s0, n, sv, stack=True)
+            ai, aj = self._arcs(s0, n)
+            b = RollbackC(slot=slot, **{k: P(v) for k, v in lam.items()})
+            r = self._rollout(sv, True, 0)
+            lib().call("waam_cadj_rollback", ctypes.addressof(r),
+                       ctypes.addressof(b), ctypes.addressof(ai), ctypes.addressof(aj), n, st)
+            slot = (slot + n) & 1
+        self.lam0 = lam["lam_H"][slot]
+        return lam["grads"].cpu().numpy()
+
+    _new, _arcs = ThermalRollout._new, ThermalRollout._arcs
+    _run, _segments = ThermalRollout._run, ThermalRollout._segments
 
     def _consts(self, n: int) -> AdjConsts:
         return ThermalRollout._consts(self, n)

@@ -17,6 +17,7 @@
 // (a clamped value has derivative 0; the phase map's slope is that of the side the enthalpy
 // is on). The surface weight's dependence on f_l (a step at f_l = 0.55) has derivative 0.
 #include "arc_cell.h"
+#include "rollout.h"
 #include "thermal_cell.h"
 
 namespace waam {
@@ -24,6 +25,7 @@ namespace waam {
 /* blocks of the adjoint's reductions: 6 doubles each fit the workspace's telemetry part */
 constexpr int kAdjBlocks = 1024;
 static_assert(6 * kAdjBlocks <= 8 * kReduceBlocks, "adjoint partials exceed the workspace");
+static_assert(kAdjBlocks == kReduceBlocks, "a rollback's partials are kReduceBlocks a step");
 
 struct AdjC {
     PhaseConsts pc;
@@ -170,6 +172,14 @@ __global__ void k_adj_terminal(const float *__restrict__ H, const float *__restr
     lam[c] = gT[c] * dT + gfl[c] * dfl;
 }
 
+/* adjoint through the second ceiling and the floor of a non-GAS cell: dL/dC */
+__device__ __forceinline__ float lam_c(float l, float E, float F, const AdjC &a)
+{
+    if (a.enable_cap && ceiling_clamps(F, a)) l = 0.0f;
+    if (a.enable_loss && E < a.h_floor) l = 0.0f;
+    return l;
+}
+
 /* adjoint step, part 1: through the second ceiling and the floor; lamC = dL/dC (0 on GAS) */
 __global__ void k_adj_step1(const float *__restrict__ lam_next, const float *__restrict__ E,
                             const float *__restrict__ F, const uint8_t *__restrict__ flags, AdjC a,
@@ -177,24 +187,20 @@ __global__ void k_adj_step1(const float *__restrict__ lam_next, const float *__r
 {
     size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= N) return;
-    if (flags[c] == GAS) {
-        lamC[c] = 0.0f;
-        return;
-    }
-    float l = lam_next[c];
-    if (a.enable_cap && ceiling_clamps(F[c], a)) l = 0.0f;
-    if (a.enable_loss && E[c] < a.h_floor) l = 0.0f;
-    lamC[c] = l;
+    lamC[c] = flags[c] == GAS ? 0.0f : lam_c(lam_next[c], E[c], F[c], a);
 }
 
 /* adjoint step, part 2: losses, conduction (the symmetric 6-neighbour operator over in-range
  * non-GAS neighbours), first ceiling, arc; lam_out = dL/dH_n; per-block partial sums of
- * (d/d eta, d/d s_h, d/d s_sigma) */
-__global__ void __launch_bounds__(kBlock) k_adj_step2(
-    const float *__restrict__ lamC, const float *__restrict__ H_n, const float *__restrict__ A,
-    const float *__restrict__ fl_n, const uint8_t *__restrict__ flags,
-    const double *__restrict__ arc_sums, AdjC a, Dims d, float *__restrict__ lam_out,
-    double *__restrict__ parts)
+ * (d/d eta, d/d s_h, d/d s_sigma). lamC(c): dL/dC of non-GAS cell c */
+template <class LamC>
+__device__ __forceinline__ void adj_step2(LamC &&lamC, const float *__restrict__ H_n,
+                                          const float *__restrict__ A,
+                                          const float *__restrict__ fl_n,
+                                          const uint8_t *__restrict__ flags,
+                                          const double *__restrict__ arc_sums, const AdjC &a,
+                                          const Dims &d, float *__restrict__ lam_out,
+                                          double *__restrict__ parts)
 {
     __shared__ double sh_s[kBlock], sh_c[kBlock];
     double g[3] = {0.0, 0.0, 0.0}, gc[3] = {0.0, 0.0, 0.0};
@@ -211,7 +217,7 @@ __global__ void __launch_bounds__(kBlock) k_adj_step2(
         }
         int i, j, k;
         d.ijk(c, i, j, k);
-        float lc = lamC[c];
+        float lc = lamC(c);
         float h = H_n[c];
         float Tn, fln;
         phase_of(h, a.pc, Tn, fln);
@@ -225,7 +231,7 @@ __global__ void __launch_bounds__(kBlock) k_adj_step2(
             if (ii < 0 || ii >= d.nx || jj < 0 || jj >= d.ny || kk < 0 || kk >= d.nz) continue;
             size_t n = d.idx(ii, jj, kk);
             if (flags[n] == GAS) continue;
-            acc += lamC[n] - lc;
+            acc += lamC(n) - lc;
         }
         float lT = a.kcond * acc;
         if (a.enable_loss) {
@@ -274,6 +280,67 @@ __global__ void __launch_bounds__(kBlock) k_adj_step2(
         }
         __syncthreads();
     }
+}
+
+__global__ void __launch_bounds__(kBlock) k_adj_step2(
+    const float *__restrict__ lamC, const float *__restrict__ H_n, const float *__restrict__ A,
+    const float *__restrict__ fl_n, const uint8_t *__restrict__ flags,
+    const double *__restrict__ arc_sums, AdjC a, Dims d, float *__restrict__ lam_out,
+    double *__restrict__ parts)
+{
+    adj_step2([&](size_t c) { return lamC[c]; }, H_n, A, fl_n, flags, arc_sums, a, d, lam_out,
+              parts);
+}
+
+/* both parts in one launch: dL/dC of the cell and its neighbours formed where it is read */
+__global__ void __launch_bounds__(kBlock) k_adj_step(
+    const float *__restrict__ lam_next, const float *__restrict__ E, const float *__restrict__ F,
+    const float *__restrict__ H_n, const float *__restrict__ A, const float *__restrict__ fl_n,
+    const uint8_t *__restrict__ flags, const double *__restrict__ arc_sums, AdjC a, Dims d,
+    float *__restrict__ lam_out, double *__restrict__ parts)
+{
+    adj_step2([&](size_t c) { return lam_c(lam_next[c], E[c], F[c], a); }, H_n, A, fl_n, flags,
+              arc_sums, a, d, lam_out, parts);
+}
+
+/* one block per step: the fixed-order totals of its partial sums */
+__global__ void __launch_bounds__(kBlock) k_rollback_totals(const double *__restrict__ parts,
+                                                            double *__restrict__ totals)
+{
+    __shared__ double sh_s[kBlock], sh_c[kBlock];
+    const double *p = parts + (size_t)blockIdx.x * 6 * kReduceBlocks;
+    for (int g = 0; g < 3; ++g) {
+        double s = 0.0, cmp = 0.0;
+        for (int b = threadIdx.x; b < kReduceBlocks; b += blockDim.x) {
+            double ss, e;
+            two_sum(s, p[(size_t)b * 6 + 2 * g], ss, e);
+            s = ss;
+            cmp += p[(size_t)b * 6 + 2 * g + 1] + e;
+        }
+        block_reduce_pair(s, cmp, sh_s, sh_c);
+        if (threadIdx.x == 0) totals[(size_t)blockIdx.x * 3 + g] = s + cmp;
+        __syncthreads();
+    }
+}
+
+/* the steps' totals into grads, the last step first */
+__global__ void k_rollback_add(const double *__restrict__ totals, int n,
+                               double *__restrict__ grads)
+{
+    const int g = (int)threadIdx.x;
+    if (g >= 3) return;
+    double acc = grads[g];
+    for (int t = n - 1; t >= 0; --t) acc += totals[(size_t)t * 3 + g];
+    grads[g] = acc;
+}
+
+void launch_rollback_totals(const double *parts, int n, double *step_totals, double *grads,
+                            hipStream_t st)
+{
+    hipLaunchKernelGGL(k_rollback_totals, dim3((unsigned)n), dim3(kBlock), 0, st, parts,
+                       step_totals);
+    hipLaunchKernelGGL(k_rollback_add, dim3(1), dim3(64), 0, st, (const double *)step_totals, n,
+                       grads);
 }
 
 }  // namespace waam
@@ -533,6 +600,33 @@ int waam_adj_thermal_step(const float *lam_next, float *lam_out, const float *H_
                        flags, arc_sums, a, d, lam_out, parts);
     hipLaunchKernelGGL(k_adj_total, dim3(1), dim3(kBlock), 0, s, parts, kAdjBlocks, 3, grads, 1);
     return check_launch("waam_adj_thermal_step");
+}
+
+int waam_adj_rollback(const waam_rollout *r, const double *arc_i, const double *arc_j, int n,
+                      float *lam, int slot, double *parts, double *step_totals, double *grads,
+                      void *stream)
+{
+    WAAM_RETURN_IF(check_rollout("waam_adj_rollback", r, arc_i, arc_j, n, true));
+    WAAM_RETURN_IF(check_ptrs("waam_adj_rollback", {lam, parts, step_totals, grads}));
+    if (slot < 0 || slot > 1)
+        return set_error(WAAM_ERR_INVALID, "waam_adj_rollback: slot %d", slot);
+    const Dims d{r->nx, r->ny, r->nz, r->layout};
+    const size_t N = d.n();
+    hipStream_t st = as_stream(stream);
+    waam_adj_consts c = r->c;
+    for (int t = n - 1, s = slot; t >= 0; --t, s ^= 1) {
+        c.arc_i = (float)arc_i[t];
+        c.arc_j = (float)arc_j[t];
+        const size_t at = (size_t)t * N;
+        hipLaunchKernelGGL(k_adj_step, dim3(kAdjBlocks), dim3(kBlock), 0, st,
+                           (const float *)lam + s * N, (const float *)r->E + at,
+                           (const float *)r->F + at, (const float *)r->H + at,
+                           (const float *)r->A + at, (const float *)r->fl + at, r->flags,
+                           (const double *)r->sums + 2 * t, make_adj(c), d, lam + (s ^ 1) * N,
+                           parts + (size_t)t * 6 * kReduceBlocks);
+    }
+    launch_rollback_totals(parts, n, step_totals, grads, st);
+    return check_launch("waam_adj_rollback");
 }
 
 int waam_adj_marangoni(const float *T, const float *phi, const float *f_l, const uint8_t *flags,

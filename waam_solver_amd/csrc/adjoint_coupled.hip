@@ -16,6 +16,7 @@
 // the difference it selected, the phase map the slope of its side; at u = 0 the upwind side
 // the forward used).
 #include "arc_cell.h"
+#include "rollout.h"
 #include "thermal_cell.h"
 
 namespace waam {
@@ -228,7 +229,32 @@ __global__ void k_cadj_forces(const float *__restrict__ Frx, const float *__rest
     lam_Fraw[2 * N + c] = lz;
 }
 
-/* Marangoni adjoint, projection pass with binary64 lambda (see adjoint.hip) */
+/* Marangoni adjoint, projection of one cell with binary64 lambda = (ax, ay, az) (see
+ * adjoint.hip) */
+__device__ __forceinline__ void marangoni_project(const float *__restrict__ phi, float fl,
+                                                  uint8_t fg, double ax, double ay, double az,
+                                                  double dgamma, int i, int j, int k,
+                                                  const Dims &d, double &gx, double &gy,
+                                                  double &gz)
+{
+    gx = gy = gz = 0.0;
+    if (fg == SOLID || fg == GAS || fl < 0.05f) return;
+    const int ip = imin(i + 1, d.nx - 1), im = imax(i - 1, 0);
+    const int jp = imin(j + 1, d.ny - 1), jm = imax(j - 1, 0);
+    const int kp = imin(k + 1, d.nz - 1), km = imax(k - 1, 0);
+    float dpx = 0.5f * (phi[d.idx(ip, j, k)] - phi[d.idx(im, j, k)]);
+    float dpy = 0.5f * (phi[d.idx(i, jp, k)] - phi[d.idx(i, jm, k)]);
+    float dpz = 0.5f * (phi[d.idx(i, j, kp)] - phi[d.idx(i, j, km)]);
+    float gm = sqrtf(dpx * dpx + dpy * dpy + dpz * dpz);
+    if (gm < 1e-6f) return;
+    const double nx = dpx / gm, ny = dpy / gm, nz = dpz / gm;
+    const double nl = nx * ax + ny * ay + nz * az;
+    const double w = dgamma * (double)gm;
+    gx = w * (ax - nl * nx);
+    gy = w * (ay - nl * ny);
+    gz = w * (az - nl * nz);
+}
+
 __global__ void k_cadj_marangoni_project(const float *__restrict__ phi,
                                          const float *__restrict__ f_l,
                                          const uint8_t *__restrict__ flags,
@@ -239,26 +265,9 @@ __global__ void k_cadj_marangoni_project(const float *__restrict__ phi,
     if (!d.cell(i, j, k)) return;
     const size_t N = d.n();
     const size_t c = d.idx(i, j, k);
-    double gx = 0.0, gy = 0.0, gz = 0.0;
-    const uint8_t fg = flags[c];
-    if (fg != SOLID && fg != GAS && !(f_l[c] < 0.05f)) {
-        const int ip = imin(i + 1, d.nx - 1), im = imax(i - 1, 0);
-        const int jp = imin(j + 1, d.ny - 1), jm = imax(j - 1, 0);
-        const int kp = imin(k + 1, d.nz - 1), km = imax(k - 1, 0);
-        float dpx = 0.5f * (phi[d.idx(ip, j, k)] - phi[d.idx(im, j, k)]);
-        float dpy = 0.5f * (phi[d.idx(i, jp, k)] - phi[d.idx(i, jm, k)]);
-        float dpz = 0.5f * (phi[d.idx(i, j, kp)] - phi[d.idx(i, j, km)]);
-        float gm = sqrtf(dpx * dpx + dpy * dpy + dpz * dpz);
-        if (!(gm < 1e-6f)) {
-            const double nx = dpx / gm, ny = dpy / gm, nz = dpz / gm;
-            const double ax = lam[c], ay = lam[N + c], az = lam[2 * N + c];
-            const double nl = nx * ax + ny * ay + nz * az;
-            const double w = dgamma * (double)gm;
-            gx = w * (ax - nl * nx);
-            gy = w * (ay - nl * ny);
-            gz = w * (az - nl * nz);
-        }
-    }
+    double gx, gy, gz;
+    marangoni_project(phi, f_l[c], flags[c], lam[c], lam[N + c], lam[2 * N + c], dgamma, i, j, k,
+                      d, gx, gy, gz);
     G[c] = gx;
     G[N + c] = gy;
     G[2 * N + c] = gz;
@@ -266,13 +275,10 @@ __global__ void k_cadj_marangoni_project(const float *__restrict__ phi,
 
 /* gather of the projected Marangoni adjoint over the clamped central differences (as in
  * adjoint.hip): T_adj += */
-__global__ void k_cadj_marangoni_gather(const double *__restrict__ G, double *__restrict__ T_adj,
-                                        Dims d)
+__device__ __forceinline__ double marangoni_gather(const double *__restrict__ G, int i, int j,
+                                                   int k, size_t c, const Dims &d)
 {
-    int i, j, k;
-    if (!d.cell(i, j, k)) return;
     const size_t N = d.n();
-    const size_t c = d.idx(i, j, k);
     const int n[3] = {d.nx, d.ny, d.nz};
     const int at[3] = {i, j, k};
     double acc = 0.0;
@@ -288,7 +294,29 @@ __global__ void k_cadj_marangoni_gather(const double *__restrict__ G, double *__
         if (v <= n[a] - 2) acc -= Ga[d.idx(hi[0], hi[1], hi[2])];
         if (v == 0) acc -= Ga[c];
     }
-    T_adj[c] += 0.5 * acc;
+    return 0.5 * acc;
+}
+
+__global__ void k_cadj_marangoni_gather(const double *__restrict__ G, double *__restrict__ T_adj,
+                                        Dims d)
+{
+    int i, j, k;
+    if (!d.cell(i, j, k)) return;
+    const size_t c = d.idx(i, j, k);
+    T_adj[c] += marangoni_gather(G, i, j, k, c, d);
+}
+
+/* phase slopes of the side H is on */
+__device__ __forceinline__ void phase_slopes64(float h, const PhaseConsts &pc, double &dT,
+                                               double &dfl)
+{
+    if (h <= pc.H_sol || h >= pc.H_liq) {
+        dT = 1.0 / (double)pc.cp_rho;
+        dfl = 0.0;
+    } else {
+        dfl = 1.0 / (double)pc.L_rho;
+        dT = ((double)pc.T_l - (double)pc.T_s) / (double)pc.L_rho;
+    }
 }
 
 /* lam_H += lam_T dT/dH + lam_fl df_l/dH at H (phase slopes of the side H is on); 0 on GAS */
@@ -303,15 +331,8 @@ __global__ void k_cadj_phase(const float *__restrict__ H, const uint8_t *__restr
         lam_H[c] = 0.0;
         return;
     }
-    const float h = H[c];
     double dT, dfl;
-    if (h <= pc.H_sol || h >= pc.H_liq) {
-        dT = 1.0 / (double)pc.cp_rho;
-        dfl = 0.0;
-    } else {
-        dfl = 1.0 / (double)pc.L_rho;
-        dT = ((double)pc.T_l - (double)pc.T_s) / (double)pc.L_rho;
-    }
+    phase_slopes64(H[c], pc, dT, dfl);
     lam_H[c] += lam_T[c] * dT + lam_fl[c] * dfl;
 }
 
@@ -445,13 +466,15 @@ __device__ __forceinline__ void upwind_grad_slopes(float u, float qmm, float qm,
 
 /* thermal adjoint, part 2: the advection term of the non-SOLID cells (C -= u . g(B)): lam_u =
  * -g lamC, and lamB of every operand's source cell += -u dg/dB lamC (scattered) */
-__global__ void k_cadj_advect(const double *__restrict__ lamC, const float *__restrict__ B,
-                              const float *__restrict__ ux, const float *__restrict__ uy,
-                              const float *__restrict__ uz, const uint8_t *__restrict__ flags,
-                              double *__restrict__ lamB, double *__restrict__ lam_u, Dims d)
+__device__ __forceinline__ void advect_adj(const double *__restrict__ lamC,
+                                           const float *__restrict__ B,
+                                           const float *__restrict__ ux,
+                                           const float *__restrict__ uy,
+                                           const float *__restrict__ uz,
+                                           const uint8_t *__restrict__ flags,
+                                           double *__restrict__ lamB, double *__restrict__ lam_u,
+                                           int i, int j, int k, const Dims &d)
 {
-    int i, j, k;
-    if (!d.cell(i, j, k)) return;
     const size_t N = d.n();
     const size_t c = d.idx(i, j, k);
     const uint8_t fg = flags[c];
@@ -483,6 +506,147 @@ __global__ void k_cadj_advect(const double *__restrict__ lamC, const float *__re
     lam_u[c] = lu[0];
     lam_u[N + c] = lu[1];
     lam_u[2 * N + c] = lu[2];
+}
+
+__global__ void k_cadj_advect(const double *__restrict__ lamC, const float *__restrict__ B,
+                              const float *__restrict__ ux, const float *__restrict__ uy,
+                              const float *__restrict__ uz, const uint8_t *__restrict__ flags,
+                              double *__restrict__ lamB, double *__restrict__ lam_u, Dims d)
+{
+    int i, j, k;
+    if (!d.cell(i, j, k)) return;
+    advect_adj(lamC, B, ux, uy, uz, flags, lamB, lam_u, i, j, k, d);
+}
+
+/* (i, j, k) of listed cell t */
+__device__ __forceinline__ void listed_cell(const int32_t *__restrict__ active, int t,
+                                            const Dims &d, int &i, int &j, int &k)
+{
+    d.ijk((size_t)active[t], i, j, k);
+}
+
+/* the listed FLUID/IFACE cells of a rollback step (lam_u is 0 elsewhere and stays so) */
+__global__ void __launch_bounds__(64) k_cadj_advect_list(
+    const int32_t *__restrict__ active, int n_active, const double *__restrict__ lamC,
+    const float *__restrict__ B, const float *__restrict__ ux, const float *__restrict__ uy,
+    const float *__restrict__ uz, const uint8_t *__restrict__ flags, double *__restrict__ lamB,
+    double *__restrict__ lam_u, Dims d)
+{
+    const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (t >= n_active) return;
+    int i, j, k;
+    listed_cell(active, t, d, i, j, k);
+    advect_adj(lamC, B, ux, uy, uz, flags, lamB, lam_u, i, j, k, d);
+}
+
+/* Collision, Mach clamp, force clamp, hydrostatic and buoyancy terms and the Marangoni projection
+ * of the listed cells, sixteen lanes a cell: lane t < 14 carries the tangent of input t of the
+ * collision map, so a cell's fourteen forward-mode passes run side by side instead of one after
+ * the other in one lane (a pool of some hundred cells leaves the chip to that chain: 131 us a
+ * step on 128x64x48, 8 so, and 20 with the three launches that followed). Each value is formed as
+ * in k_cadj_collide_mrt, k_cadj_forces and k_cadj_marangoni_project. */
+constexpr int kCellLanes = 16;
+
+__device__ __forceinline__ double shfl64(double v, int lane)
+{
+    return __hiloint2double(__shfl(__double2hiint(v), lane), __shfl(__double2loint(v), lane));
+}
+
+struct FlowAdj {
+    double omega_s, omega_b, C_darcy, u_cap, F_cap, g_lu, beta, T_l, dgamma;
+    int enable_hydro;
+};
+
+__global__ void __launch_bounds__(64) k_cadj_flow_list(
+    const int32_t *__restrict__ active, int n_active, const float *__restrict__ f,
+    const float *__restrict__ Fr, const float *__restrict__ Fc, const float *__restrict__ T,
+    const float *__restrict__ f_l, const float *__restrict__ phi,
+    const uint8_t *__restrict__ flags, const double *__restrict__ lam_f,
+    const double *__restrict__ lam_u, FlowAdj a, double *__restrict__ lam_fin,
+    double *__restrict__ lam_T, double *__restrict__ lam_fl, double *__restrict__ G, Dims d)
+{
+    const int lane = (int)threadIdx.x, t = lane & (kCellLanes - 1), lane0 = lane - t;
+    const int at = (int)blockIdx.x * (64 / kCellLanes) + lane / kCellLanes;
+    const bool on = at < n_active;
+    const size_t N = d.n(), c = (size_t)active[on ? at : n_active - 1];
+    double mv[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0}, lf[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const double x = f[(size_t)q * N + c];
+        lf[q] = lam_f[(size_t)q * N + c];
+#pragma unroll
+        for (int m = 0; m < 10; ++m) mv[m] += moment_row(m, q) * x;
+    }
+    D1 m[10], out[Q], u3[3];
+#pragma unroll
+    for (int s = 0; s < 10; ++s) m[s] = D1{mv[s], s == t ? 1.0 : 0.0};
+    const double fl = f_l[c];
+    mrt_map(m, D1{Fc[c], t == 10 ? 1.0 : 0.0}, D1{Fc[N + c], t == 11 ? 1.0 : 0.0},
+            D1{Fc[2 * N + c], t == 12 ? 1.0 : 0.0}, D1{fl, t == 13 ? 1.0 : 0.0}, a.omega_s,
+            a.omega_b, a.C_darcy, out, u3);
+    double lu[3] = {lam_u[c], lam_u[N + c], lam_u[2 * N + c]};
+    clamp_adj(u3[0].v, u3[1].v, u3[2].v, a.u_cap, lu[0], lu[1], lu[2]);
+    double acc = lu[0] * u3[0].d + lu[1] * u3[1].d + lu[2] * u3[2].d;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) acc += lf[q] * out[q].d;
+    double g[14];
+#pragma unroll
+    for (int s = 0; s < 14; ++s) g[s] = shfl64(acc, lane0 + s);
+    if (!on) return;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        if (q % kCellLanes != t) continue;
+        double x = 0.0;
+#pragma unroll
+        for (int s = 0; s < 10; ++s) x += g[s] * moment_row(s, q);
+        lam_fin[(size_t)q * N + c] = x;
+    }
+    if (t != 0) return;
+    double lx = g[10], ly = g[11], lz = g[12], lT = 0.0, lfl = g[13];
+    clamp_adj(Fr[c], Fr[N + c], Fr[2 * N + c], a.F_cap, lx, ly, lz);
+    if (fl > 0.0) {
+        double dfl = a.g_lu * a.beta * ((double)T[c] - a.T_l);
+        if (a.enable_hydro) dfl -= a.g_lu;
+        lfl += lz * dfl;
+        lT += lz * a.g_lu * a.beta * fl;
+    }
+    lam_T[c] = lT;
+    lam_fl[c] = lfl;
+    int i, j, k;
+    listed_cell(active, at, d, i, j, k);
+    double gx, gy, gz;
+    marangoni_project(phi, f_l[c], flags[c], lx, ly, lz, a.dgamma, i, j, k, d, gx, gy, gz);
+    G[c] = gx;
+    G[N + c] = gy;
+    G[2 * N + c] = gz;
+}
+
+/* The Marangoni gather, the phase map and part 1 of the thermal adjoint of every cell: lamC and
+ * lamB from lam_H = dL/dH_{n+1} (FLOW: plus what the flow adds through T and f_l at H1) */
+template <bool FLOW>
+__global__ void k_cadj_lamC(const double *__restrict__ lam_H, const double *__restrict__ lam_T,
+                            const double *__restrict__ lam_fl, const double *__restrict__ G,
+                            const float *__restrict__ H1, const float *__restrict__ E,
+                            const float *__restrict__ F, const uint8_t *__restrict__ flags, CAdj a,
+                            double *__restrict__ lamC, double *__restrict__ lamB, Dims d)
+{
+    int i, j, k;
+    if (!d.cell(i, j, k)) return;
+    const size_t c = d.idx(i, j, k);
+    double l = 0.0;
+    if (flags[c] != GAS) {
+        l = lam_H[c];
+        if (FLOW) {
+            const double lT = lam_T[c] + marangoni_gather(G, i, j, k, c, d);
+            double dT, dfl;
+            phase_slopes64(H1[c], a.pc, dT, dfl);
+            l += lT * dT + lam_fl[c] * dfl;
+        }
+        if (a.enable_cap && cceil(F[c], a)) l = 0.0;
+        if (a.enable_loss && E[c] < (float)a.h_floor) l = 0.0;
+    }
+    lamC[c] = l;
+    lamB[c] = l;
 }
 
 /* thermal adjoint, part 3: conduction (symmetric operator on lamC), losses (on lamC), the first
@@ -592,7 +756,7 @@ __global__ void __launch_bounds__(kBlock) k_cadj_total(const double *__restrict_
     }
 }
 
-constexpr int kCAdjBlocks = 1024;
+constexpr int kCAdjBlocks = kReduceBlocks;  // a rollback's partials are kReduceBlocks a step
 
 }  // namespace waam
 
@@ -688,6 +852,66 @@ int waam_cadj_thermal_step(const double *lam_next, double *lam_out, double *lam_
     hipLaunchKernelGGL(k_cadj_total, dim3(1), dim3(kBlock), 0, s, (const double *)parts,
                        kCAdjBlocks, grads);
     return check_launch("waam_cadj_thermal_step");
+}
+
+int waam_cadj_rollback(const waam_rollout *r, const waam_rollback *b, const double *arc_i,
+                       const double *arc_j, int n, void *stream)
+{
+    WAAM_RETURN_IF(check_rollout("waam_cadj_rollback", r, arc_i, arc_j, n, true));
+    if (!b) return set_error(WAAM_ERR_INVALID, "waam_cadj_rollback: NULL argument");
+    WAAM_RETURN_IF(check_ptrs("waam_cadj_rollback", {b->lam_H, b->lamC, b->lamB, b->parts,
+                                                     b->step_totals, b->grads}));
+    if (b->slot < 0 || b->slot > 1)
+        return set_error(WAAM_ERR_INVALID, "waam_cadj_rollback: slot %d", b->slot);
+    const bool flow = r->flow == 2;
+    if (r->flow)
+        WAAM_RETURN_IF(check_ptrs("waam_cadj_rollback", {b->lam_u, r->B}));
+    if (flow)
+        WAAM_RETURN_IF(check_ptrs("waam_cadj_rollback", {b->lam_f, b->lam_T1, b->lam_fl1, b->G}));
+    const Dims d{r->nx, r->ny, r->nz, r->layout};
+    const size_t N = d.n();
+    hipStream_t st = as_stream(stream);
+    waam_adj_consts c = r->c;
+    const FlowAdj fa{r->omega_s, r->omega_b, r->C_darcy, r->u_cap, r->F_cap, r->g_lu, r->beta,
+                     c.T_l, r->dgamma, r->enable_hydro};
+    for (int t = n - 1, s = b->slot; t >= 0; --t, s ^= 1) {
+        c.arc_i = (float)arc_i[t];
+        c.arc_j = (float)arc_j[t];
+        const CAdj a = make_cadj(c);
+        const size_t at = (size_t)t * N, nx = at + N;
+        if (flow && r->n_active > 0)
+            hipLaunchKernelGGL(k_cadj_flow_list, dim3(grid_for((size_t)r->n_active, 64 / kCellLanes)),
+                               dim3(64), 0, st, r->active, r->n_active,
+                               (const float *)r->f + Q * at, (const float *)r->Fr + 3 * at,
+                               (const float *)r->Fc + 3 * at, (const float *)r->T + nx,
+                               (const float *)r->fl + nx, r->phi, r->flags,
+                               (const double *)b->lam_f + (size_t)s * Q * N,
+                               (const double *)b->lam_u + (size_t)s * 3 * N, fa,
+                               b->lam_f + (size_t)(s ^ 1) * Q * N, b->lam_T1, b->lam_fl1, b->G, d);
+        auto lam_c = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid3(d), block3(), 0, st,
+                               (const double *)b->lam_H + s * N, (const double *)b->lam_T1,
+                               (const double *)b->lam_fl1, (const double *)b->G,
+                               (const float *)r->H + nx, (const float *)r->E + at,
+                               (const float *)r->F + at, r->flags, a, b->lamC, b->lamB, d);
+        };
+        if (flow) lam_c(k_cadj_lamC<true>);
+        else lam_c(k_cadj_lamC<false>);
+        if (r->flow && r->n_active > 0) {
+            const float *u = flow ? r->u + 3 * at : r->u;
+            hipLaunchKernelGGL(k_cadj_advect_list, dim3(grid_for((size_t)r->n_active, 64)),
+                               dim3(64), 0, st, r->active, r->n_active, (const double *)b->lamC,
+                               (const float *)r->B + at, u, u + N, u + 2 * N, r->flags, b->lamB,
+                               b->lam_u + (size_t)(s ^ 1) * 3 * N, d);
+        }
+        hipLaunchKernelGGL(k_cadj_step2, dim3(kCAdjBlocks), dim3(kBlock), 0, st,
+                           (const double *)b->lamC, (const double *)b->lamB,
+                           (const float *)r->H + at, (const float *)r->A + at,
+                           (const float *)r->fl + at, r->flags, (const double *)r->sums + 2 * t, a,
+                           d, b->lam_H + (s ^ 1) * N, b->parts + (size_t)t * 6 * kReduceBlocks);
+    }
+    launch_rollback_totals(b->parts, n, b->step_totals, b->grads, st);
+    return check_launch("waam_cadj_rollback");
 }
 
 }  // extern "C"
