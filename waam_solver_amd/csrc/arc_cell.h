@@ -46,24 +46,42 @@ __device__ __forceinline__ bool arc_cell_weights(const ArcParams &p, int i, int 
     return true;
 }
 
+__device__ __forceinline__ double shfl_down64(double v, int off)
+{
+    return __hiloint2double(__shfl_down(__double2hiint(v), off),
+                            __shfl_down(__double2loint(v), off));
+}
+
+/* The block's total of its threads' compensated pairs, in thread 0 (blocks of a power of two of at
+ * least 64 threads; every thread calls it): halves added pairwise, between wavefronts through
+ * LDS, then within the first by shuffles. The same additions as a tree in LDS all the way, whose
+ * eight barriers cost a 256-thread block 2 us. */
 __device__ __forceinline__ void block_reduce_pair(double &s, double &c, double *sh_s, double *sh_c)
 {
-    int t = threadIdx.x;
+    const int t = threadIdx.x;
     sh_s[t] = s;
     sh_c[t] = c;
     __syncthreads();
-    for (int off = blockDim.x / 2; off > 0; off >>= 1) {
+    for (int off = blockDim.x / 2; off >= 64; off >>= 1) {
         if (t < off) {
-            double a = sh_s[t], b = sh_s[t + off], ss, e;
-            two_sum(a, b, ss, e);
-            sh_s[t] = ss;
-            sh_c[t] = sh_c[t] + sh_c[t + off] + e;
+            double ss, e;
+            two_sum(s, sh_s[t + off], ss, e);
+            c = c + sh_c[t + off] + e;
+            s = ss;
+            sh_s[t] = s;
+            sh_c[t] = c;
         }
         __syncthreads();
     }
-    s = sh_s[0];
-    c = sh_c[0];
+    if (t < 64) {
+        for (int off = 32; off > 0; off >>= 1) {
+            const double os = shfl_down64(s, off), oc = shfl_down64(c, off);
+            double ss, e;
+            two_sum(s, os, ss, e);
+            c = c + oc + e;
+            s = ss;
+        }
+    }
 }
-
 
 }  // namespace waam

@@ -489,6 +489,131 @@ __device__ __forceinline__ uint32_t pull_dirs(const PullRec &r, const QuietRec &
  * block at a time (one atomic per block; the block's segments in index order, blocks in
  * arrival order: each segment's results depend only on the sweeps' inputs, so the order is
  * free). One atomic per wavefront, on the one counter, took 36 against 20 us at 768x384x192. */
+/* the block's appends to both lists, V segments a thread: one atomic per block and list */
+template <int V>
+__device__ __forceinline__ void append_segments(const QuietRec &q, const PullRec &r,
+                                                const uint32_t (&sg)[V], const bool (&act)[V],
+                                                const uint32_t (&dirs)[V])
+{
+    __shared__ int s_cnt[2][kBlock / 64];
+    __shared__ int s_base[2];
+    const int lane = (int)__lane_id();
+    const int wave = (int)threadIdx.x >> 6;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    unsigned long long m[V], mp[V];
+    int n = 0, np = 0;
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        m[v] = __ballot(act[v]);
+        mp[v] = __ballot(dirs[v] != 0u);
+        n += __popcll(m[v]);
+        np += __popcll(mp[v]);
+    }
+    if (lane == 0) {
+        s_cnt[0][wave] = n;
+        s_cnt[1][wave] = np;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        int tot = 0;
+        for (int w = 0; w < kBlock / 64; ++w) tot += s_cnt[threadIdx.x][w];
+        s_base[threadIdx.x] = tot ? atomicAdd(threadIdx.x == 0 ? q.count : r.count, tot) : 0;
+    }
+    __syncthreads();
+    int base = s_base[0], pbase = s_base[1];
+    for (int w = 0; w < wave; ++w) {
+        base += s_cnt[0][w];
+        pbase += s_cnt[1][w];
+    }
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+        if (act[v]) q.list[base + __popcll(m[v] & below)] = (int32_t)sg[v];
+        if (dirs[v] != 0u) r.list[pbase + __popcll(mp[v] & below)] = make_uint2(sg[v], dirs[v]);
+        base += __popcll(m[v]);
+        pbase += __popcll(mp[v]);
+    }
+}
+
+/* Four segments of a row a thread, on grids whose rows hold a multiple of four (ZYX): the record
+ * bytes of a row come as one dword and the change words as 16 bytes, 60 loads for four segments
+ * where one at a time takes 55 each. The tests are segment_active's and pull_dirs's, byte by byte
+ * of a dword. 768x384x192 (885 k segments): 28 -> 15 us. */
+__host__ __device__ inline bool quad_segments(const Dims &d)
+{
+    return d.layout == kLayoutZYX && quiet_nbx(d) % 4 == 0;
+}
+
+__device__ __forceinline__ void quiet_list_quad(const waam_step_fields &f, const StepConsts &s)
+{
+    const Dims &d = s.d;
+    const QuietRec q = quiet_rec(f, d);
+    const PullRec r = pull_rec(f, d);
+    const size_t nseg = quiet_segments(d);
+    const size_t s0 = 4 * ((size_t)blockIdx.x * blockDim.x + threadIdx.x);
+    constexpr uint32_t kOnes = 0x01010101u;
+    uint32_t sg[4], dirs[4] = {0u, 0u, 0u, 0u};
+    bool act[4] = {false, false, false, false};
+    if (s0 < nseg) {
+        const int bx = (int)(s0 % (size_t)q.nbx);
+        const size_t rowi = s0 / (size_t)q.nbx;
+        const int j = (int)(rowi % (size_t)d.ny), k = (int)(rowi / (size_t)d.ny);
+        const int xl = bx > 0 ? bx - 1 : q.nbx - 1, xr = bx + 4 < q.nbx ? bx + 4 : 0;
+        uint32_t all = kOnes, own = 0u;
+#pragma unroll
+        for (int dk = -2; dk <= 1; ++dk) {
+#pragma unroll
+            for (int dj = -1; dj <= 1; ++dj) {
+                const size_t row = seg_index(q, 0, imax(0, imin(j + dj, d.ny - 1)),
+                                             imax(0, imin(k + dk, d.nz - 1)), d);
+                const uint32_t w = *reinterpret_cast<const uint32_t *>(q.bits + row + bx);
+                const uint32_t l = q.bits[row + xl], h = q.bits[row + xr];
+                if (dk == 0 && dj == 0) own = w;
+                all &= w & ((w << 8) | l) & ((w >> 8) | (h << 24));
+            }
+        }
+        /* not swept: quiet for two steps with every neighbour quiet, or cold plate */
+        uint32_t idle = all & own & (own >> 1) & kOnes;
+        if (k < plate_slices(s.p, d)) idle |= (own >> 2) & (own >> 3) & kOnes;
+        uint32_t ownc[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int dk = -1; dk <= 1; ++dk) {
+#pragma unroll
+            for (int dj = -1; dj <= 1; ++dj) {
+                const uint32_t any = row_dirs(dj, dk, 2);
+                const uint32_t up = row_dirs(dj, dk, 1), dn = row_dirs(dj, dk, -1);
+                if (any == 0u) continue;
+                const size_t row = seg_index(q, 0, imax(0, imin(j - dj, d.ny - 1)),
+                                             imax(0, imin(k - dk, d.nz - 1)), d);
+                const uint4 c4 = *reinterpret_cast<const uint4 *>(r.chg_src + row + bx);
+                const uint32_t c[4] = {c4.x, c4.y, c4.z, c4.w};
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    dirs[v] |= c[v] & any;
+                    if (dj == 0 && dk == 0) ownc[v] = c[v];
+                }
+                if (up == 0u && dn == 0u) continue;
+                const uint4 e4 = *reinterpret_cast<const uint4 *>(r.edge_src + row + bx);
+                const uint32_t e[6] = {r.edge_src[row + xl], e4.x, e4.y, e4.z, e4.w,
+                                       r.edge_src[row + xr]};
+#pragma unroll
+                for (int v = 0; v < 4; ++v) dirs[v] |= (e[v] & up) | (e[v + 2] & dn);
+            }
+        }
+        uint32_t fresh[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            sg[v] = (uint32_t)s0 + (uint32_t)v;
+            act[v] = ((idle >> (8 * v)) & 1u) == 0u;
+            if ((ownc[v] & ~kPullDirs) != 0u) dirs[v] = kPullDirs;
+            fresh[v] = ownc[v] == kPullUnknown ? kPullFull : 0u;
+        }
+        const uint4 f4 = make_uint4(fresh[0], fresh[1], fresh[2], fresh[3]);
+        *reinterpret_cast<uint4 *>(r.chg_dst + s0) = f4;
+        *reinterpret_cast<uint4 *>(r.edge_dst + s0) = f4;
+    }
+    append_segments<4>(q, r, sg, act, dirs);
+}
+
 __device__ __forceinline__ void quiet_list(const waam_step_fields &f, const StepConsts &s)
 {
     const Dims &d = s.d;
@@ -518,31 +643,12 @@ __device__ __forceinline__ void quiet_list(const waam_step_fields &f, const Step
         r.chg_dst[sg] = fresh;
         r.edge_dst[sg] = fresh;
     }
-    __shared__ int s_cnt[2][kBlock / 64];
-    __shared__ int s_base[2];
-    const unsigned long long m = __ballot(act), mp = __ballot(dirs != 0u);
-    const int lane = (int)__lane_id();
-    const int wave = (int)threadIdx.x >> 6;
-    if (lane == 0) {
-        s_cnt[0][wave] = __popcll(m);
-        s_cnt[1][wave] = __popcll(mp);
-    }
-    __syncthreads();
-    if (threadIdx.x < 2) {
-        int tot = 0;
-        for (int w = 0; w < kBlock / 64; ++w) tot += s_cnt[threadIdx.x][w];
-        s_base[threadIdx.x] = tot ? atomicAdd(threadIdx.x == 0 ? q.count : r.count, tot) : 0;
-    }
-    __syncthreads();
-    int base = s_base[0], pbase = s_base[1];
-    for (int w = 0; w < wave; ++w) {
-        base += s_cnt[0][w];
-        pbase += s_cnt[1][w];
-    }
-    const unsigned long long below = (1ull << lane) - 1ull;
-    if (act) q.list[base + __popcll(m & below)] = (int32_t)sg;
-    if (dirs != 0u) r.list[pbase + __popcll(mp & below)] = make_uint2((uint32_t)sg, dirs);
+    const uint32_t sgs[1] = {(uint32_t)sg};
+    const bool acts[1] = {act};
+    const uint32_t dirss[1] = {dirs};
+    append_segments<1>(q, r, sgs, acts, dirss);
 }
+
 
 /* the cell of this lane in segment seg (block3() blocks: the lanes along the contiguous axis,
  * one wavefront per threadIdx.y) */
@@ -665,6 +771,9 @@ static unsigned resident_blocks(K kernel, int threads)
     return n;
 }
 
+/* slices whose depth weight a block of kernel 1 keeps in LDS (the others are formed per cell) */
+constexpr int kDepthLds = 1024;
+
 /* 1 — surface height in the torch column (reference kernels.py:625-641 and
  *     coupled_step.py:34-59) and per-block compensated arc weight sums (kernels.py:443-496);
  *     empties the collision list, and the thermal list unless it was built ahead. */
@@ -673,7 +782,7 @@ __global__ void __launch_bounds__(kBlock) k_step_begin(waam_step_fields f, StepC
 {
     __shared__ double sh_s[kBlock], sh_c[kBlock];
     __shared__ int sh_k[kBlock];
-    __shared__ float s_arck;
+    __shared__ float s_arck, s_depth[kDepthLds];
     const Dims &d = s.d;
     const waam_step_params &p = s.p;
     const ArcStep at = arc_step(s);
@@ -713,13 +822,30 @@ __global__ void __launch_bounds__(kBlock) k_step_begin(waam_step_fields f, StepC
     ap.arc_i = at.arc_i;
     ap.arc_j = at.arc_j;
     ap.arc_k = p.use_arc_k_override ? p.arc_k_override : s_arck;
-    if (do_sums && blockIdx.x == 0) {
-        /* the surface weight of a cell that is not liquid, by slice (HView) */
-        float *depth = reinterpret_cast<float *>(f.quiet + quiet_depth_offset(d));
-        for (int k = threadIdx.x; k < d.nz; k += blockDim.x)
-            depth[k] = arc_deposition_weight(k, ap.arc_k, 0.0f, ap.pen, ap.enable);
-    }
     double sum = 0.0, comp = 0.0;
+    if (do_sums) {
+        /* the surface weight of a cell that is not liquid, by slice: for this block's sums and,
+         * from the first block, for the rest of the step (HView) */
+        float *depth = reinterpret_cast<float *>(f.quiet + quiet_depth_offset(d));
+        for (int k = threadIdx.x; k < (blockIdx.x == 0 ? d.nz : imin(d.nz, kDepthLds));
+             k += blockDim.x) {
+            const float w = arc_deposition_weight(k, ap.arc_k, 0.0f, ap.pen, ap.enable);
+            if (k < kDepthLds) s_depth[k] = w;
+            if (blockIdx.x == 0) depth[k] = w;
+        }
+        __syncthreads();
+    }
+    auto term = [&](int i, int j, int k, float fl) {
+        const float wk = k < kDepthLds
+                             ? s_depth[k]
+                             : arc_deposition_weight(k, ap.arc_k, 0.0f, ap.pen, ap.enable);
+        const float wdep = fl > 0.55f ? 1.0f : wk;
+        if (wdep < 1e-6f) return;
+        double ss, e;
+        two_sum(sum, (double)(arc_shape(ap, i, j, k) * wdep), ss, e);
+        sum = ss;
+        comp += e;
+    };
     size_t N = d.n();
     /* the arc's weights are exactly zero outside its (i, j) box (exp underflows to 0 there), so
      * on a grid wider than the box the sums run over the box's columns only. The TwoSum pairs
@@ -752,12 +878,7 @@ __global__ void __launch_bounds__(kBlock) k_step_begin(waam_step_fields f, StepC
                 if (flg[u] == GAS) continue;
                 int i, j, k;
                 cell_ijk(base + u * stride, d, i, j, k);
-                float wg, wdep;
-                if (!arc_cell_weights(ap, i, j, k, flv[u], wg, wdep)) continue;
-                double ss, e;
-                two_sum(sum, (double)(wg * wdep), ss, e);
-                sum = ss;
-                comp += e;
+                term(i, j, k, flv[u]);
             }
         }
     } else if (d.fast() % 4 == 0) {
@@ -800,12 +921,7 @@ __global__ void __launch_bounds__(kBlock) k_step_begin(waam_step_fields f, StepC
                 for (int e = 0; e < 4; ++e) {
                     if (((fw[u] >> (8 * e)) & 0xffu) == GAS) continue;
                     const int i = zyx ? i0 + e : i0, k = zyx ? k0 : k0 + e;
-                    float wg, wdep;
-                    if (!arc_cell_weights(ap, i, j0, k, flv[e], wg, wdep)) continue;
-                    double ss, er;
-                    two_sum(sum, (double)(wg * wdep), ss, er);
-                    sum = ss;
-                    comp += er;
+                    term(i, j0, k, flv[e]);
                 }
             }
         }
@@ -839,12 +955,7 @@ __global__ void __launch_bounds__(kBlock) k_step_begin(waam_step_fields f, StepC
                 if (flg[u] == GAS) continue;
                 int i, j, k;
                 cell_ijk((size_t)cells[u], d, i, j, k);
-                float wg, wdep;
-                if (!arc_cell_weights(ap, i, j, k, flv[u], wg, wdep)) continue;
-                double ss, e;
-                two_sum(sum, (double)(wg * wdep), ss, e);
-                sum = ss;
-                comp += e;
+                term(i, j, k, flv[u]);
             }
         }
     }
@@ -889,10 +1000,11 @@ __global__ void __launch_bounds__(kBlock) k_step_arc_total(waam_step_fields f, S
 
 /* the segment list of a steady step and, in the last block, the arc total (TOTAL: the step has
  * sums): neither needs the other, and a launch of its own cost the total 4.5 us */
-template <bool TOTAL>
+template <bool TOTAL, bool QUAD>
 __global__ void __launch_bounds__(kBlock) k_step_quiet_list(waam_step_fields f, StepConsts s)
 {
     if (TOTAL && blockIdx.x == gridDim.x - 1) arc_total(f, s);
+    else if (QUAD) quiet_list_quad(f, s);
     else quiet_list(f, s);
 }
 
@@ -1228,7 +1340,7 @@ __device__ __forceinline__ void plate_march(const waam_step_fields &f, const Ste
         return ((unsigned)__shfl((int)mybits, k) & 12u) == 12u;
     };
     /* slice state: own T and flag at k-1, k, k+1 (and k+2 in flight), the halo column's and
-     * halo row's T and flag at k (and k+1 in flight), the cell's H, f_l, T_max and T_prev at k
+     * halo row's T and flag at k (and k+1 in flight), the cell's H, f_l and T_max at k
      * (and k+1 in flight) */
     auto idx = [&](int ii, int jj, int kk) { return d.idx(ii, jj, imax(0, imin(kk, d.nz - 1))); };
     /* the block's slices: one of kPlateChunks ranges */
@@ -1242,10 +1354,10 @@ __device__ __forceinline__ void plate_march(const waam_step_fields &f, const Ste
     Fc = f.flags_in[idx(ic, jc, k0)];
     Tp = f.T_in[idx(ic, jc, k0 + 1)];
     Fp = f.flags_in[idx(ic, jc, k0 + 1)];
-    float Th = 0.0f, Tr = 0.0f, H = 0.0f, FL = 0.0f, TX = 0.0f, TP = 0.0f;
+    float Th = 0.0f, Tr = 0.0f, H = 0.0f, FL = 0.0f, TX = 0.0f;
     uint8_t Fh = GAS, Fr = GAS;
     auto load_k = [&](int k, bool hist, float &th, uint8_t &fh, float &tr, uint8_t &fr,
-                      float &h, float &fl, float &tx, float &tp) {
+                      float &h, float &fl, float &tx) {
         if (first || last) {
             th = f.T_in[idx(i_h, jc, k)];
             fh = f.flags_in[idx(i_h, jc, k)];
@@ -1259,20 +1371,19 @@ __device__ __forceinline__ void plate_march(const waam_step_fields &f, const Ste
             h = f.H_in[c];
             fl = hv.heated(i, j) ? f.fl_in[c] : 0.0f;
             tx = f.T_max[c];
-            tp = f.T_prev[c];
         }
     };
     float WK = hv.arc_on && k0 < k1 ? hv.depth[k0] : 0.0f;
-    if (k0 < k1) load_k(k0, hist_at(k0), Th, Fh, Tr, Fr, H, FL, TX, TP);
+    if (k0 < k1) load_k(k0, hist_at(k0), Th, Fh, Tr, Fr, H, FL, TX);
     for (int k = k0; k < k1; ++k) {
         const bool hist = hist_at(k);
         /* in flight during slice k's arithmetic: T and flags of k+2, the rest of k+1 */
         Tn = f.T_in[idx(ic, jc, k + 2)];
         Fn = f.flags_in[idx(ic, jc, k + 2)];
-        float Th1 = 0.0f, Tr1 = 0.0f, H1 = 0.0f, FL1 = 0.0f, TX1 = 0.0f, TP1 = 0.0f;
+        float Th1 = 0.0f, Tr1 = 0.0f, H1 = 0.0f, FL1 = 0.0f, TX1 = 0.0f;
         uint8_t Fh1 = GAS, Fr1 = GAS;
         const float WK1 = hv.arc_on && k + 1 < k1 ? hv.depth[k + 1] : 0.0f;
-        if (k + 1 < k1) load_k(k + 1, hist_at(k + 1), Th1, Fh1, Tr1, Fr1, H1, FL1, TX1, TP1);
+        if (k + 1 < k1) load_k(k + 1, hist_at(k + 1), Th1, Fh1, Tr1, Fr1, H1, FL1, TX1);
         sT[r][lane] = Tc;
         sF[r][lane] = Fc;
         __syncthreads();
@@ -1324,7 +1435,8 @@ __device__ __forceinline__ void plate_march(const waam_step_fields &f, const Ste
                 const size_t c = d.idx(i, j, k);
                 const float H_c = hv.value(H, FL, 0.0f, WK, i, j, k);
                 const float dH = conduction_dH(pr, Tc, m_im, m_ip, m_jm, m_jp, m_km, m_kp);
-                const float2 tf = thermal_finish<false>(f, s, c, Tc, H_c, dH, n_exp, pr, TX, TP,
+                /* T_prev holds the cell's own T: the step that left it cold stored both */
+                const float2 tf = thermal_finish<false>(f, s, c, Tc, H_c, dH, n_exp, pr, TX, Tc,
                                                         true);
                 cold = tf.x < T_cold && tf.y == 0.0f;
             }
@@ -1351,7 +1463,6 @@ __device__ __forceinline__ void plate_march(const waam_step_fields &f, const Ste
         FL = FL1;
         WK = WK1;
         TX = TX1;
-        TP = TP1;
     }
 }
 
@@ -2667,13 +2778,22 @@ static void launch_step(const StepConsts &s, const waam_step_fields &f, hipStrea
     timed_launch(WAAM_K_BEGIN, [&](hipEvent_t a, hipEvent_t b) {
         launch_k(capture, k_step_begin, dim3(do_sums ? kReduceBlocks : 1), dim3(kBlock), st, a,
                  (do_sums || seg) ? nullptr : b, f, s, do_sums);
-        const unsigned lists = grid_for(quiet_segments(d));
-        if (seg && do_sums)
-            launch_k(capture, k_step_quiet_list<true>, dim3(lists + 1), dim3(kBlock), st, nullptr,
-                     b, f, s);
-        else if (seg)
-            launch_k(capture, k_step_quiet_list<false>, dim3(lists), dim3(kBlock), st, nullptr, b,
-                     f, s);
+        const bool quad = quad_segments(d);
+        const dim3 lists(grid_for(quiet_segments(d) / (quad ? 4 : 1)) + (do_sums ? 1u : 0u));
+        if (seg) {
+            if (quad && do_sums)
+                launch_k(capture, k_step_quiet_list<true, true>, lists, dim3(kBlock), st, nullptr, b,
+                         f, s);
+            else if (quad)
+                launch_k(capture, k_step_quiet_list<false, true>, lists, dim3(kBlock), st, nullptr,
+                         b, f, s);
+            else if (do_sums)
+                launch_k(capture, k_step_quiet_list<true, false>, lists, dim3(kBlock), st, nullptr,
+                         b, f, s);
+            else
+                launch_k(capture, k_step_quiet_list<false, false>, lists, dim3(kBlock), st, nullptr,
+                         b, f, s);
+        }
         else if (do_sums)
             launch_k(capture, k_step_arc_total, dim3(1), dim3(kBlock), st, nullptr, b, f, s);
     });
