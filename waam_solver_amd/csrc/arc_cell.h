@@ -58,11 +58,11 @@ __device__ __forceinline__ double shfl_down64(double v, int off)
  * eight barriers cost a 256-thread block 2 us. */
 __device__ __forceinline__ void block_reduce_pair(double &s, double &c, double *sh_s, double *sh_c)
 {
-    const int t = threadIdx.x;
+    const int t = (int)(threadIdx.y * blockDim.x + threadIdx.x);
     sh_s[t] = s;
     sh_c[t] = c;
     __syncthreads();
-    for (int off = blockDim.x / 2; off >= 64; off >>= 1) {
+    for (int off = (int)(blockDim.x * blockDim.y) / 2; off >= 64; off >>= 1) {
         if (t < off) {
             double ss, e;
             two_sum(s, sh_s[t + off], ss, e);

@@ -291,8 +291,11 @@ __device__ __forceinline__ void cell_ijk(size_t c, const Dims &d, int &i, int &j
  * again and leaves it out of kernels 4 and 7 (need[pos] = 0 at its list position). */
 struct QuietRec {
     uint8_t *bits;
+    /* the step's counters; kernel 7 empties the next step's (its own are read until it ends, and
+     * the next step's first launch appends), and leaves the count for a reader in `last` */
     int *count;
     int *warm;      // segments kernel 2p lists, from the list's end backwards
+    int *last, *next;
     int32_t *list;
     uint8_t *need;  // per list position: kernels 4 and 7 visit the segment
     int nbx;        // segments per row
@@ -345,13 +348,24 @@ __host__ __device__ inline int plate_slices(const waam_step_params &p, const Dim
     return d.layout == kLayoutZYX && !p.use_tables && n > 0 ? n : 0;
 }
 
+/* which of the record's two sets of counters and change words belongs to the step: the two
+ * population buffers take turns as its source */
+__device__ __forceinline__ int record_parity(const waam_step_fields &f)
+{
+    return f.f_src < f.f_dst ? 0 : 1;
+}
+
 __device__ __forceinline__ QuietRec quiet_rec(const waam_step_fields &f, const Dims &d)
 {
     QuietRec q;
     q.nbx = quiet_nbx(d);
     q.bits = f.quiet;
-    q.count = reinterpret_cast<int *>(f.quiet + quiet_count_offset(d));
-    q.warm = q.count + 1;
+    int *line = reinterpret_cast<int *>(f.quiet + quiet_count_offset(d));
+    const int p = record_parity(f);
+    q.count = line + 4 + p;
+    q.warm = line + 6 + p;
+    q.last = line;
+    q.next = line + 4 + (p ^ 1);
     q.list = reinterpret_cast<int32_t *>(f.quiet + quiet_count_offset(d) + 256);
     q.need = f.quiet + quiet_need_offset(d);
     return q;
@@ -423,8 +437,8 @@ constexpr uint32_t kPullUnknown = 0xffffffffu;
 
 struct PullRec {
     uint32_t *chg_src, *edge_src, *chg_dst, *edge_dst;
-    int *count;
-    uint2 *list;  // (segment, directions)
+    int *count, *last, *next;  // as the segment list's
+    uint2 *list;               // (segment, directions)
 };
 
 __device__ __forceinline__ PullRec pull_rec(const waam_step_fields &f, const Dims &d)
@@ -432,12 +446,14 @@ __device__ __forceinline__ PullRec pull_rec(const waam_step_fields &f, const Dim
     const size_t nseg = quiet_segments(d);
     uint8_t *base = f.quiet + quiet_still_offset(d);
     uint32_t *w = reinterpret_cast<uint32_t *>(base + 256);
-    const bool lower = f.f_src < f.f_dst;
+    const int p = record_parity(f);
     PullRec r;
-    r.count = reinterpret_cast<int *>(base);
-    r.chg_src = w + (lower ? 0 : 2) * nseg;
+    r.last = reinterpret_cast<int *>(base);
+    r.count = r.last + 4 + p;
+    r.next = r.last + 4 + (p ^ 1);
+    r.chg_src = w + (p ? 2 : 0) * nseg;
     r.edge_src = r.chg_src + nseg;
-    r.chg_dst = w + (lower ? 2 : 0) * nseg;
+    r.chg_dst = w + (p ? 0 : 2) * nseg;
     r.edge_dst = r.chg_dst + nseg;
     r.list = reinterpret_cast<uint2 *>(w + 4 * nseg);
     return r;
@@ -543,13 +559,14 @@ __host__ __device__ inline bool quad_segments(const Dims &d)
     return d.layout == kLayoutZYX && quiet_nbx(d) % 4 == 0;
 }
 
-__device__ __forceinline__ void quiet_list_quad(const waam_step_fields &f, const StepConsts &s)
+__device__ __forceinline__ void quiet_list_quad(const waam_step_fields &f, const StepConsts &s,
+                                                unsigned block)
 {
     const Dims &d = s.d;
     const QuietRec q = quiet_rec(f, d);
     const PullRec r = pull_rec(f, d);
     const size_t nseg = quiet_segments(d);
-    const size_t s0 = 4 * ((size_t)blockIdx.x * blockDim.x + threadIdx.x);
+    const size_t s0 = 4 * ((size_t)block * blockDim.x + threadIdx.x);
     constexpr uint32_t kOnes = 0x01010101u;
     uint32_t sg[4], dirs[4] = {0u, 0u, 0u, 0u};
     bool act[4] = {false, false, false, false};
@@ -614,12 +631,13 @@ __device__ __forceinline__ void quiet_list_quad(const waam_step_fields &f, const
     append_segments<4>(q, r, sg, act, dirs);
 }
 
-__device__ __forceinline__ void quiet_list(const waam_step_fields &f, const StepConsts &s)
+__device__ __forceinline__ void quiet_list(const waam_step_fields &f, const StepConsts &s,
+                                           unsigned block)
 {
     const Dims &d = s.d;
     const QuietRec q = quiet_rec(f, d);
     const size_t nseg = quiet_segments(d);
-    const size_t sg = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const size_t sg = (size_t)block * blockDim.x + threadIdx.x;
     const int KP = plate_slices(s.p, d);
     bool act = false;
     if (sg < nseg) {
@@ -728,6 +746,13 @@ __device__ __forceinline__ void record_quiet(const QuietRec &q, size_t seg, bool
     }
 }
 
+/* kernel 7, one thread: the next step's counters start empty */
+__device__ __forceinline__ void empty_next_lists(const QuietRec &q, const PullRec &r)
+{
+    q.next[0] = q.next[2] = 0;
+    r.next[0] = 0;
+}
+
 /* a step that is not steady leaves the pull's record unknown for both buffers */
 __device__ __forceinline__ void forget_pull(const PullRec &r, size_t seg)
 {
@@ -777,8 +802,8 @@ constexpr int kDepthLds = 1024;
 /* 1 — surface height in the torch column (reference kernels.py:625-641 and
  *     coupled_step.py:34-59) and per-block compensated arc weight sums (kernels.py:443-496);
  *     empties the collision list, and the thermal list unless it was built ahead. */
-__global__ void __launch_bounds__(kBlock) k_step_begin(waam_step_fields f, StepConsts s,
-                                                       int do_sums)
+__device__ __forceinline__ void step_begin(const waam_step_fields &f, const StepConsts &s,
+                                           int do_sums, unsigned nblocks)
 {
     __shared__ double sh_s[kBlock], sh_c[kBlock];
     __shared__ int sh_k[kBlock];
@@ -789,11 +814,6 @@ __global__ void __launch_bounds__(kBlock) k_step_begin(waam_step_fields f, StepC
     if (blockIdx.x == 0) {
         if (!p.thermal_list_ready) cell_list(f, s.d.n(), 0).count(threadIdx.x) = 0;
         cell_list(f, s.d.n(), 1).count(threadIdx.x) = 0;
-        if (p.quiet_skip && threadIdx.x == 0) {
-            *quiet_rec(f, d).count = 0;
-            *quiet_rec(f, d).warm = 0;
-            *pull_rec(f, d).count = 0;
-        }
     }
     int best = -1;
     for (int k = threadIdx.x; k < d.nz; k += blockDim.x) {
@@ -859,7 +879,7 @@ __global__ void __launch_bounds__(kBlock) k_step_begin(waam_step_fields f, StepC
     const unsigned bj = bj1 >= bj0 ? (unsigned)(bj1 - bj0 + 1) : 0u;
     const size_t nbox = (size_t)bi * bj * (size_t)d.nz;
     const bool whole = bi == (unsigned)d.nx && bj == (unsigned)d.ny;
-    size_t stride = (size_t)gridDim.x * blockDim.x;
+    size_t stride = (size_t)nblocks * blockDim.x;
     constexpr int kUnroll = 8;
     if (whole) {
         for (size_t base = (size_t)blockIdx.x * blockDim.x + threadIdx.x; do_sums && base < N;
@@ -968,44 +988,67 @@ __global__ void __launch_bounds__(kBlock) k_step_begin(waam_step_fields f, StepC
     }
 }
 
-/* 1b — fixed-order total of the block sums and the energy per unit weight (reference
- *      kernels.py:493-496); one block */
-__device__ __forceinline__ void arc_total(const waam_step_fields &f, const StepConsts &s)
+/* the first `sums` blocks: kernel 1; the rest, on a steady step: its segment list (1b). Neither
+ * needs the other: apart they took 14 + 8 us on 301x157x83, 20 + 15 on 768x384x192 */
+template <bool QUAD>
+__global__ void __launch_bounds__(kBlock, 4) k_step_begin(waam_step_fields f, StepConsts s,
+                                                       int do_sums, int sums)
+{
+    if ((int)blockIdx.x < sums) step_begin(f, s, do_sums, (unsigned)sums);
+    else if (QUAD) quiet_list_quad(f, s, blockIdx.x - (unsigned)sums);
+    else quiet_list(f, s, blockIdx.x - (unsigned)sums);
+}
+
+/* blocks of kernel 1's sums: every block of a merged thermal launch adds their pairs up, so a small
+ * grid takes few, and a large one leaves half the chip to the list beside them (1024 blocks on
+ * 768x384x192: 31.8 us for the two, 512: 28.9) */
+static int sum_blocks(const Dims &d) { return d.n() <= ((size_t)1 << 19) ? 256 : 512; }
+
+/* fixed-order total of kernel 1's block sums and the energy per unit weight (reference
+ * kernels.py:493-496), formed by a whole block (of kBlock threads); the value is every thread's.
+ * store: write both for the rest of the step */
+__device__ __forceinline__ float arc_total(const waam_step_fields &f, const StepConsts &s, int nparts,
+                                           bool store)
 {
     __shared__ double sh_s[kBlock], sh_c[kBlock];
-    const double *parts = reinterpret_cast<const double *>((char *)f.scratch + kScratchPartials);
+    __shared__ float s_epw;
+    const double2 *parts = reinterpret_cast<const double2 *>((char *)f.scratch + kScratchPartials);
+    const int t = (int)(threadIdx.y * blockDim.x + threadIdx.x);
     double sum = 0.0, comp = 0.0;
-    for (int b = threadIdx.x; b < kReduceBlocks; b += blockDim.x) {
+    for (int b = t; b < nparts; b += kBlock) {
+        const double2 pr = parts[b];
         double ss, e;
-        two_sum(sum, parts[2 * b], ss, e);
+        two_sum(sum, pr.x, ss, e);
         sum = ss;
-        comp += parts[2 * b + 1] + e;
+        comp += pr.y + e;
     }
     block_reduce_pair(sum, comp, sh_s, sh_c);
-    if (threadIdx.x == 0) {
+    if (t == 0) {
         const waam_step_params &p = s.p;
         float *tot = reinterpret_cast<float *>((char *)f.scratch + kScratchTelemetry);
         float w_total = (float)(sum + comp);
         float epw = 0.0f;
         if (w_total > 1e-9f) epw = p.Q_w * p.eta * p.dt / (w_total * p.dx3);
-        tot[0] = w_total;
-        tot[1] = epw;
+        s_epw = epw;
+        if (store) {
+            tot[0] = w_total;
+            tot[1] = epw;
+        }
     }
+    __syncthreads();
+    return s_epw;
 }
 
-__global__ void __launch_bounds__(kBlock) k_step_arc_total(waam_step_fields f, StepConsts s)
+__global__ void __launch_bounds__(kBlock) k_step_arc_total(waam_step_fields f, StepConsts s,
+                                                           int nparts)
 {
-    arc_total(f, s);
+    (void)arc_total(f, s, nparts, true);
 }
 
-/* the segment list of a steady step and, in the last block, the arc total (TOTAL: the step has
- * sums): neither needs the other, and a launch of its own cost the total 4.5 us */
-template <bool TOTAL, bool QUAD>
-__global__ void __launch_bounds__(kBlock) k_step_quiet_list(waam_step_fields f, StepConsts s)
+/* the energy per unit weight a launch of its own has left */
+__device__ __forceinline__ float stored_epw(const waam_step_fields &f)
 {
-    if (TOTAL && blockIdx.x == gridDim.x - 1) arc_total(f, s);
-    else if (QUAD) quiet_list_quad(f, s);
-    else quiet_list(f, s);
+    return reinterpret_cast<const float *>((char *)f.scratch + kScratchTelemetry)[1];
 }
 
 /* Enthalpy of a non-GAS cell as the thermal kernel reads it: after this step's arc injection
@@ -1066,7 +1109,7 @@ struct HView {
     }
 };
 
-__device__ __forceinline__ HView make_hview(const waam_step_fields &f, const StepConsts &s)
+__device__ __forceinline__ HView make_hview(const waam_step_fields &f, const StepConsts &s, float epw)
 {
     const float *tot = reinterpret_cast<const float *>((char *)f.scratch + kScratchTelemetry);
     HView hv;
@@ -1080,7 +1123,7 @@ __device__ __forceinline__ HView make_hview(const waam_step_fields &f, const Ste
     hv.ap.arc_i = at.arc_i;
     hv.ap.arc_j = at.arc_j;
     hv.ap.arc_k = step_arc_k(s.p, tot);
-    hv.epw = tot[1];
+    hv.epw = epw;
     hv.H_liq = s.pc.H_liq;
     hv.cap_l = s.cap_l;
     hv.cap_s = s.cap_s;
@@ -1170,7 +1213,7 @@ __device__ __forceinline__ float2 thermal_finish(const waam_step_fields &f, cons
  * ended the last two steps cold), so a new f_l of 0 is not stored again */
 template <bool TAB, bool ADV = true>
 __device__ __forceinline__ float2 thermal_cell(const waam_step_fields &f, const StepConsts &s,
-                                             int i, int j, int k, size_t c, uint8_t flag,
+                                             float epw, int i, int j, int k, size_t c, uint8_t flag,
                                              float h_gas, bool fl_zero_held = false)
 {
     const Dims &d = s.d;
@@ -1188,7 +1231,7 @@ __device__ __forceinline__ float2 thermal_cell(const waam_step_fields &f, const 
         if (TAB) store_props(f, c, cell_props(p.tables, p.refs, 1, GAS, 0.0f));
         return make_float2(T, fl);
     }
-    HView hv = make_hview(f, s);
+    HView hv = make_hview(f, s, epw);
     /* advect_diffuse_temperature (Jacobi: every neighbour value is pre-kernel) */
     float T_c = f.T_in[c];
     float T_im = masked_at(f.T_in, f.flags_in, i - 1, j, k, T_c, d);
@@ -1256,10 +1299,10 @@ __device__ __forceinline__ float vof_advect_cell(const waam_step_fields &f, cons
 /* thermal chain and VOF advection of one cell */
 template <bool TAB>
 __device__ __forceinline__ void thermal_vof_cell(const waam_step_fields &f, const StepConsts &s,
-                                                 int i, int j, int k, size_t c, uint8_t flag)
+                                                 float epw, int i, int j, int k, size_t c, uint8_t flag)
 {
     float phi_new = s.p.enable_vof ? vof_advect_cell(f, s.d, i, j, k, flag) : 0.0f;
-    thermal_cell<TAB>(f, s, i, j, k, c, flag, f.H_in[c]);
+    thermal_cell<TAB>(f, s, epw, i, j, k, c, flag, f.H_in[c]);
     if (s.p.enable_vof) f.phi_tmp[c] = phi_new;
 }
 
@@ -1280,7 +1323,7 @@ __global__ void __launch_bounds__(256) k_step_thermal(waam_step_fields f, StepCo
     float phi_new = (in && s.p.enable_vof) ? vof_advect_cell(f, d, i, j, k, flag) : 0.0f;
     if (LIST) list_append(in && is_surface_class(flag), c, cell_list(f, s.d.n(), 0));
     if (!in || is_surface_class(flag)) return;
-    thermal_cell<TAB, false>(f, s, i, j, k, c, flag, h_in);
+    thermal_cell<TAB, false>(f, s, stored_epw(f), i, j, k, c, flag, h_in);
     if (s.p.enable_vof) f.phi_tmp[c] = phi_new;
 }
 
@@ -1308,14 +1351,14 @@ __host__ __device__ inline int plate_blocks(const Dims &d)
 }
 
 __device__ __forceinline__ void plate_march(const waam_step_fields &f, const StepConsts &s,
-                                            int block)
+                                            float epw, int block)
 {
     __shared__ float sT[kPlateRows][kTileFast];
     __shared__ uint8_t sF[kPlateRows][kTileFast];
     const Dims &d = s.d;
     const waam_step_params &p = s.p;
     const QuietRec q = quiet_rec(f, d);
-    const HView hv = make_hview(f, s);
+    const HView hv = make_hview(f, s, epw);
     const float T_cold = cold_limit(p);
     const int KP = plate_slices(p, d);
     const int lane = (int)threadIdx.x, r = (int)threadIdx.y;
@@ -1470,7 +1513,7 @@ __device__ __forceinline__ void plate_march(const waam_step_fields &f, const Ste
  * of them kernels 4 and 7 visit: all but the segments that stay cold plate */
 template <bool TAB>
 __device__ __forceinline__ void thermal_walk(const waam_step_fields &f, const StepConsts &s,
-                                             int block, int nblocks)
+                                             float epw, int block, int nblocks)
 {
     const Dims &d = s.d;
     const QuietRec q = quiet_rec(f, d);
@@ -1486,7 +1529,7 @@ __device__ __forceinline__ void thermal_walk(const waam_step_fields &f, const St
         bool cold = !in;
         if (hist) {
             if (in) {
-                const float2 tf = thermal_cell<TAB, false>(f, s, i, j, k, c, SOLID, 0.0f, true);
+                const float2 tf = thermal_cell<TAB, false>(f, s, epw, i, j, k, c, SOLID, 0.0f, true);
                 cold = tf.x < T_cold && tf.y == 0.0f;
             }
         } else {
@@ -1500,7 +1543,7 @@ __device__ __forceinline__ void thermal_walk(const waam_step_fields &f, const St
                 phi_new = vof_advect_cell(f, d, i, j, k, flag);
             if (in && !is_surface_class(flag)) {
                 /* flag is SOLID or GAS: no enthalpy advection */
-                const float2 tf = thermal_cell<TAB, false>(f, s, i, j, k, c, flag, h_in);
+                const float2 tf = thermal_cell<TAB, false>(f, s, epw, i, j, k, c, flag, h_in);
                 if (s.p.enable_vof) f.phi_tmp[c] = phi_new;
                 cold = flag == SOLID && tf.x < T_cold && tf.y == 0.0f;
             }
@@ -1517,21 +1560,22 @@ __device__ __forceinline__ void thermal_walk(const waam_step_fields &f, const St
 /* the march in a launch of its own (a plate past kTogetherBlocks) */
 __global__ void __launch_bounds__(256) k_step_thermal_plate(waam_step_fields f, StepConsts s)
 {
-    plate_march(f, s, (int)blockIdx.x);
+    plate_march(f, s, stored_epw(f), (int)blockIdx.x);
 }
 
 /* the walk in a launch of its own (temperature-dependent material, or a plate of that size) */
 template <bool TAB>
 __global__ void __launch_bounds__(256) k_step_thermal_seg(waam_step_fields f, StepConsts s)
 {
-    thermal_walk<TAB>(f, s, (int)blockIdx.x, (int)gridDim.x);
+    thermal_walk<TAB>(f, s, stored_epw(f), (int)blockIdx.x, (int)gridDim.x);
 }
 
 /* thermal chain (with enthalpy advection) and VOF advection of the listed FLUID/IFACE cells;
  * worker b of nb, 256 threads each */
 template <bool TAB>
 __device__ __forceinline__ void thermal_surface_list(const waam_step_fields &f,
-                                                     const StepConsts &s, int b, int nb)
+                                                     const StepConsts &s, float epw, int b,
+                                                     int nb)
 {
     __shared__ int s_pref[kListSegments + 1];
     const Dims &d = s.d;
@@ -1542,7 +1586,7 @@ __device__ __forceinline__ void thermal_surface_list(const waam_step_fields &f,
         size_t c = list_at(l, s_pref, t);
         int i, j, k;
         cell_ijk(c, d, i, j, k);
-        thermal_vof_cell<TAB>(f, s, i, j, k, c, f.flags_in[c]);
+        thermal_vof_cell<TAB>(f, s, epw, i, j, k, c, f.flags_in[c]);
     }
 }
 
@@ -1550,20 +1594,22 @@ __device__ __forceinline__ void thermal_surface_list(const waam_step_fields &f,
 template <bool TAB>
 __global__ void __launch_bounds__(256) k_step_thermal_surface(waam_step_fields f, StepConsts s)
 {
-    thermal_surface_list<TAB>(f, s, blockIdx.x, gridDim.x);
+    thermal_surface_list<TAB>(f, s, stored_epw(f), blockIdx.x, gridDim.x);
 }
 
 /* 2, 2p and 3 of a steady step in one launch: the first `surface` blocks take the listed
  * FLUID/IFACE cells (the longest chain, so first), the next `walk` the active segments, the rest
- * the plate's cold segments. Constant material: with the tables the two inlined copies of the
+ * the plate's cold segments. Every block forms the arc total itself (nparts > 0), for a
+ * microsecond where a launch between kernel 1 and this one costs four and a half. Constant material: with the tables the two inlined copies of the
  * cell routine make the compiler copy the argument structs to private memory */
 __global__ void __launch_bounds__(256) k_step_thermal_steady(waam_step_fields f, StepConsts s,
-                                                             int surface, int walk)
+                                                             int surface, int walk, int nparts)
 {
     const int b = (int)blockIdx.x;
-    if (b < surface) thermal_surface_list<false>(f, s, b, surface);
-    else if (b < surface + walk) thermal_walk<false>(f, s, b - surface, walk);
-    else plate_march(f, s, b - surface - walk);
+    const float epw = nparts > 0 ? arc_total(f, s, nparts, b == 0) : 0.0f;
+    if (b < surface) thermal_surface_list<false>(f, s, epw, b, surface);
+    else if (b < surface + walk) thermal_walk<false>(f, s, epw, b - surface, walk);
+    else plate_march(f, s, epw, b - surface - walk);
 }
 
 /* 2+3 in one launch, when the previous step's kernel 7 has listed this step's FLUID/IFACE
@@ -1605,7 +1651,7 @@ __global__ void __launch_bounds__(256) k_step_thermal_all(waam_step_fields f, St
         float h_in = f.H_in[c];
         float phi_new = s.p.enable_vof ? vof_advect_cell(f, d, i, j, k, flag) : 0.0f;
         if (!list && is_surface_class(flag)) return;
-        thermal_cell<TAB>(f, s, i, j, k, c, flag, h_in);
+        thermal_cell<TAB>(f, s, stored_epw(f), i, j, k, c, flag, h_in);
         if (s.p.enable_vof) f.phi_tmp[c] = phi_new;
     }
 }
@@ -2044,6 +2090,9 @@ __global__ void __launch_bounds__(256) k_step_stream(waam_step_fields f, StepCon
 {
     const Dims &d = s.d;
     const QuietRec q = quiet_rec(f, d);
+    if (blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x == 0 &&
+        threadIdx.y == 0)
+        empty_next_lists(q, pull_rec(f, d));
     int i, j, k;
     if (PULL) {
         const bool in = d.cell(i, j, k);
@@ -2100,6 +2149,12 @@ __global__ void __launch_bounds__(256) k_step_stream_seg(waam_step_fields f, Ste
     const Dims &d = s.d;
     const QuietRec q = quiet_rec(f, d);
     const float T_cold = cold_limit(s.p);
+    if (blockIdx.x == 0 && threadIdx.x == 0 && threadIdx.y == 0) {
+        const PullRec r = pull_rec(f, d);
+        *q.last = *q.count;
+        *r.last = *r.count;
+        empty_next_lists(q, r);
+    }
     for_needed_segments(q, d, [&](size_t seg) {
         int i, j, k;
         const bool in = seg_cell(q, seg, d, i, j, k);
@@ -2439,6 +2494,7 @@ __global__ void k_advect_tracers_step(float *__restrict__ pos, int32_t *__restri
  * would rewrite unchanged are left alone). A segment may be on the list twice: both wavefronts
  * form the same words, and the one that finds a word different records it. */
 constexpr int kPullGroup = 5;
+constexpr int kPullItems = (Q + kPullGroup - 1) / kPullGroup;
 
 template <class E>
 __global__ void __launch_bounds__(256) k_step_pull_seg(waam_step_fields f, StepConsts s,
@@ -2457,15 +2513,30 @@ __global__ void __launch_bounds__(256) k_step_pull_seg(waam_step_fields f, StepC
     E *dst = static_cast<E *>(f.f_dst);
     const size_t N = d.n();
     const int nx = d.nx;
-    const int n = *r.count;
     const int nw = ((int)gridDim.x - tracers) * (int)blockDim.y;
     const int w0 = ((int)blockIdx.x - tracers) * (int)blockDim.y + (int)threadIdx.y;
     const int lane = (int)threadIdx.x;
+    /* a list that leaves wavefronts idle is dealt out a round of loads at a time, kPullGroup of an
+     * entry's directions (64x40x32, 600 entries: 8.0 -> 5.9 us); a longer one by whole entries
+     * (75 k entries: 42 us, 70 by rounds, whose wavefronts read the flags of each again) */
+    const int count = *r.count;
+    const int items = count <= nw / kPullItems ? kPullItems : 1;
+    const long long n = (long long)count * items;
     for (long long t0 = w0; t0 < n; t0 += 64LL * nw) {
         const long long tl = t0 + (long long)lane * nw;
-        const uint2 mine = tl < n ? r.list[tl] : make_uint2(0u, 0u);
-        const int cnt = (int)std::min<long long>(64, (n - t0 + nw - 1) / nw);
-        for (int it = 0; it < cnt; ++it) {
+        uint2 mine = make_uint2(0u, 0u);
+        if (tl < n) mine = r.list[tl / items];
+        if (items > 1) {
+            uint32_t rest = mine.y;
+            for (int g = kPullGroup * (int)(tl % items); g > 0; --g) rest &= rest - 1u;
+            uint32_t after = rest;
+            for (int g = 0; g < kPullGroup; ++g) after &= after - 1u;
+            mine.y = rest ^ after;
+        }
+        unsigned long long m = __ballot(mine.y != 0u);
+        while (m != 0ull) {
+            const int it = __builtin_ctzll(m);
+            m &= m - 1ull;
             const uint32_t seg = (uint32_t)__builtin_amdgcn_readlane((int)mine.x, it);
             uint32_t dirs = (uint32_t)__builtin_amdgcn_readlane((int)mine.y, it);
             const uint32_t rowi = seg / (uint32_t)q.nbx;
@@ -2517,12 +2588,12 @@ __global__ void __launch_bounds__(256) k_step_pull_seg(waam_step_fields f, StepC
                 for (int u = 0; u < kPullGroup; ++u) {
                     if (qs[u] < 0) continue;
                     const bool ch = need && v[u] != old[u];
-                    const unsigned long long m = __ballot(ch);
-                    if (m == 0ull) continue;
+                    const unsigned long long mc = __ballot(ch);
+                    if (mc == 0ull) continue;
                     if (ch) dst[(size_t)qs[u] * N + c] = v[u];
                     const int sh = dir_of(0, qs[u]);
                     chg |= 1u << qs[u];
-                    if (sh > 0 ? (m >> last) & 1ull : (sh < 0 && (m & 1ull))) edge |= 1u << qs[u];
+                    if (sh > 0 ? (mc >> last) & 1ull : (sh < 0 && (mc & 1ull))) edge |= 1u << qs[u];
                 }
             }
             if (chg != 0u && lane == 0) {
@@ -2775,30 +2846,23 @@ static void launch_step(const StepConsts &s, const waam_step_fields &f, hipStrea
     dim3 g3 = grid3(d);
     const bool seg = p.quiet_skip != 0;
     int do_sums = p.is_welding && !p.arc_applied ? 1 : 0;
+    const bool tab = p.use_tables != 0;
+    const bool together = seg && !tab && thermal_together(d);
+    const int nsum = do_sums ? sum_blocks(d) : 1;
     timed_launch(WAAM_K_BEGIN, [&](hipEvent_t a, hipEvent_t b) {
-        launch_k(capture, k_step_begin, dim3(do_sums ? kReduceBlocks : 1), dim3(kBlock), st, a,
-                 (do_sums || seg) ? nullptr : b, f, s, do_sums);
-        const bool quad = quad_segments(d);
-        const dim3 lists(grid_for(quiet_segments(d) / (quad ? 4 : 1)) + (do_sums ? 1u : 0u));
-        if (seg) {
-            if (quad && do_sums)
-                launch_k(capture, k_step_quiet_list<true, true>, lists, dim3(kBlock), st, nullptr, b,
-                         f, s);
-            else if (quad)
-                launch_k(capture, k_step_quiet_list<false, true>, lists, dim3(kBlock), st, nullptr,
-                         b, f, s);
-            else if (do_sums)
-                launch_k(capture, k_step_quiet_list<true, false>, lists, dim3(kBlock), st, nullptr,
-                         b, f, s);
-            else
-                launch_k(capture, k_step_quiet_list<false, false>, lists, dim3(kBlock), st, nullptr,
-                         b, f, s);
-        }
-        else if (do_sums)
-            launch_k(capture, k_step_arc_total, dim3(1), dim3(kBlock), st, nullptr, b, f, s);
+        const bool total = do_sums && !together;
+        const bool quad = seg && quad_segments(d);
+        const unsigned lists = seg ? grid_for(quiet_segments(d) / (quad ? 4 : 1)) : 0u;
+        if (quad)
+            launch_k(capture, k_step_begin<true>, dim3((unsigned)nsum + lists), dim3(kBlock), st, a,
+                     total ? nullptr : b, f, s, do_sums, nsum);
+        else
+            launch_k(capture, k_step_begin<false>, dim3((unsigned)nsum + lists), dim3(kBlock), st,
+                     a, total ? nullptr : b, f, s, do_sums, nsum);
+        if (total)
+            launch_k(capture, k_step_arc_total, dim3(1), dim3(kBlock), st, nullptr, b, f, s, nsum);
     });
     /* kernel 3 (the listed surface cells), with or without the temperature-dependent material */
-    const bool tab = p.use_tables != 0;
     auto launch_surface = [&](hipEvent_t a, hipEvent_t b) {
         if (tab)
             launch_k(capture, k_step_thermal_surface<true>,
@@ -2811,12 +2875,11 @@ static void launch_step(const StepConsts &s, const waam_step_fields &f, hipStrea
     };
     if (seg) {
         const unsigned plate = plate_slices(p, d) > 0 ? (unsigned)plate_blocks(d) : 0u;
-        const bool together = !tab && thermal_together(d);
         timed_launch(WAAM_K_THERMAL, [&](hipEvent_t a, hipEvent_t b) {
             if (together) {
                 launch_k(capture, k_step_thermal_steady,
                          dim3(kSteadySurfaceBlocks + kSteadyWalkBlocks + plate), block3(), st, a,
-                         b, f, s, kSteadySurfaceBlocks, kSteadyWalkBlocks);
+                         b, f, s, kSteadySurfaceBlocks, kSteadyWalkBlocks, do_sums ? nsum : 0);
                 return;
             }
             if (plate > 0)
@@ -3298,7 +3361,7 @@ __global__ void __launch_bounds__(256) k_droplet_arc(waam_step_fields f, StepCon
     }
     int i, j, k;
     if (!d.cell(i, j, k)) return;
-    const HView hv = make_hview(f, s);
+    const HView hv = make_hview(f, s, stored_epw(f));
     const size_t c = d.idx(i, j, k);
     if (f.flags_in[c] == GAS) return;
     f.H_in[c] = hv.at(c, i, j, k);
@@ -3401,8 +3464,10 @@ static void launch_droplet_step(const StepConsts &s0, const waam_step_fields &f,
     sa.p.use_arc_k_override = 0;
     sa.p.quiet_skip = 0;
     sa.p.thermal_list_ready = 0;
-    hipLaunchKernelGGL(k_step_begin, dim3(kReduceBlocks), dim3(kBlock), 0, st, f, sa, 1);
-    hipLaunchKernelGGL(k_step_arc_total, dim3(1), dim3(kBlock), 0, st, f, sa);
+    const int nsum = sum_blocks(d);
+    hipLaunchKernelGGL(k_step_begin<false>, dim3((unsigned)nsum), dim3(kBlock), 0, st, f, sa, 1,
+                       nsum);
+    hipLaunchKernelGGL(k_step_arc_total, dim3(1), dim3(kBlock), 0, st, f, sa, nsum);
     hipLaunchKernelGGL(k_droplet_arc, grid3(d), block3(), 0, st, f, sa);
     /* forces, cleared before the droplet's impact pressure adds to them */
     {
