@@ -359,6 +359,35 @@ int waam_apply_lorentz_JxB(float *Fx, float *Fy, float *Fz, const float *Jx, con
                            const float *f_l, const uint8_t *flags, float dt, float dx,
                            float rho_ref, int64_t n, void *stream);
 
+/* The whole solve and its force (physics/weld_forces.py:196-281), as the entries above give it in
+ * that order bit for bit: conductivity, normalised source, sweeps in chunks of ten with the
+ * convergence test sum |change| / max(sum |phi|, 1e-30) < tol after each, J, bins, B, force.
+ * max_sweeps bounds the sweeps; cold != 0 starts from phi = 0. Synchronises the stream. */
+typedef struct waam_lorentz {
+    float *phi, *phi_tmp;     /* potential in, and the Jacobi partner */
+    float *sigma, *source, *Jx, *Jy, *Jz, *Bx, *By, *Bz;
+    float *bins, *bins_raw;   /* nz x n_bins each; bins gets the enclosed current */
+    float *l1;                /* device, 2 floats: as waam_elec_l1_diff */
+    float *Fx, *Fy, *Fz;
+    float *Fx_snap, *Fy_snap, *Fz_snap;  /* waam_step_fused_lorentz: the step's forces copied */
+    const float *f_l;
+    const uint8_t *flags;
+    void *scratch;
+    const int32_t *bead_top;  /* device word to return with the result (waam_bead_top_k), or null */
+    double tol;
+    float arc_i, arc_j, arc_k, sigma_cells, current, dx, sigma_liquid, sigma_solid, omega;
+    float bin_dr, mu0, dt, rho;
+    int32_t nz_solid, n_bins, cold, max_sweeps, nx, ny, nz, layout;
+} waam_lorentz;
+typedef struct waam_lorentz_result {
+    float res, norm;          /* L1 sums of the last sweep done */
+    int32_t sweeps, converged;
+    int32_t in_tmp;           /* the potential is left in phi_tmp, not in phi */
+    float arc_k;              /* the arc's height that the source took */
+    int32_t bead_top;         /* what bead_top held, -1 without it */
+} waam_lorentz_result;
+int waam_lorentz_solve(const waam_lorentz *p, waam_lorentz_result *out, void *stream);
+
 /* ---- moving window: shift_simulation_window_x kernels.py:2620-2723 ------------------------ */
 /* Every listed field (both population buffers included) becomes new[i] = old[i + n_shift] for
  * i < nx - n_shift (the reference's ascending serial loop), and the last n_shift columns are
@@ -652,6 +681,13 @@ typedef struct waam_step_params {
 } waam_step_params;
 
 int waam_step_fused(const waam_step_params *p, const waam_step_fields *f, void *stream);
+/* waam_step_fused with the Lorentz solve between its flag update and its collision, whose forces
+ * then end with J x B (reference solvers/coupled_step.py:349-351). q: f_l, flags, scratch, arc_k
+ * and the force fields are the step's own, what q holds there is not read. Welding steps with
+ * arc_applied 0, use_arc_k_override 0, enable_vof 1 and fp32 populations only; synchronises the
+ * stream before the collision is launched. */
+int waam_step_fused_lorentz(const waam_step_params *p, const waam_step_fields *f,
+                            const waam_lorentz *q, waam_lorentz_result *out, void *stream);
 /* A step on which a droplet detaches (reference solvers/coupled_step.py:97-166 followed by the
  * rest of the step), with everything the host would read back kept on the device: the previous
  * step's deferred stream is materialised; the torch column's surface height (with the robot

@@ -125,6 +125,8 @@ SIGNATURES: dict[str, str] = {
     "waam_elec_prefix_bins": "piip",
     "waam_elec_B_axisymmetric": "ppppfffffiiiiip",
     "waam_apply_lorentz_JxB": "pppppppppppffflp",
+    "waam_lorentz_solve": "ppp",
+    "waam_step_fused_lorentz": "ppppp",
     "waam_compute_vorticity_magnitude": "pppppffiiiip",
     "waam_max_norm3": "pppplp",
     "waam_probe_gather": "pppilpp",

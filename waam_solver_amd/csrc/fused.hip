@@ -60,6 +60,7 @@
 #include "droplet_launch.h"
 #include "forces_cell.h"
 #include "lbm_cell.h"
+#include "lorentz.h"
 #include "pop_store.h"
 #include "tables_cell.h"
 #include "thermal_cell.h"
@@ -1828,11 +1829,18 @@ __device__ __forceinline__ void pull_rows(const E *__restrict__ src, E *__restri
     for (int q = 0; q < Q; ++q) dst[(size_t)q * N + c] = v[q];
 }
 
+/* the welding current's fields of a step with the Lorentz force */
+struct LorentzFields {
+    const float *Jx, *Jy, *Jz, *Bx, *By, *Bz;
+    float dt, dx, rho;
+};
+
 /* body forces, collision and Mach clamp of one FLUID/IFACE cell; populations in storage form
- * PD (fp32 arithmetic either way) */
-template <int PD>
+ * PD (fp32 arithmetic either way); LZ: with the Lorentz force */
+template <int PD, bool LZ>
 __device__ __forceinline__ void collide_cell(const waam_step_fields &f, const StepConsts &s,
-                                             int i, int j, int k, size_t c)
+                                             const LorentzFields &lz, int i, int j, int k,
+                                             size_t c)
 {
     using PS = PopStore<PD>;
     const typename PS::E *f_src = static_cast<const typename PS::E *>(f.f_src);
@@ -1896,6 +1904,13 @@ __device__ __forceinline__ void collide_cell(const waam_step_fields &f, const St
     }
     if (p.enable_hydro && fl > 0.0f) fz += -1.0f * p.g_lu * fl;
     if (fl > 0.0f) fz += 1.0f * p.g_lu * p.beta * (T_c - p.T_l) * fl;
+    if (LZ && !(fl < 0.05f)) {
+        lorentz_force(lz.Jx[c], lz.Jy[c], lz.Jz[c], lz.Bx[c], lz.By[c], lz.Bz[c], fl, lz.dt, lz.dx,
+                      lz.rho, tx, ty, tz);
+        fx += tx;
+        fy += ty;
+        fz += tz;
+    }
     if (p.F_cap > 0.0f) {
         float mag = sqrtf(fx * fx + fy * fy + fz * fz);
         if (mag > p.F_cap) {
@@ -1938,8 +1953,9 @@ __device__ __forceinline__ void collide_cell(const waam_step_fields &f, const St
 }
 
 /* 5 — forces + collision of the FLUID/IFACE cells listed by kernel 4 */
-template <int PD>
-__global__ void __launch_bounds__(256) k_step_collide(waam_step_fields f, StepConsts s)
+template <int PD, bool LZ>
+__global__ void __launch_bounds__(256) k_step_collide(waam_step_fields f, StepConsts s,
+                                                      LorentzFields lz)
 {
     __shared__ int s_pref[kListSegments + 1];
     const Dims &d = s.d;
@@ -1949,7 +1965,7 @@ __global__ void __launch_bounds__(256) k_step_collide(waam_step_fields f, StepCo
         size_t c = list_at(l, s_pref, t);
         int i, j, k;
         cell_ijk(c, d, i, j, k);
-        collide_cell<PD>(f, s, i, j, k, c);
+        collide_cell<PD, LZ>(f, s, lz, i, j, k, c);
     }
 }
 
@@ -2838,7 +2854,8 @@ static bool thermal_together(const Dims &d)
 /* the step's launches in order (kernels 1-7). A steady step (s.p.quiet_skip) lists its active
  * row segments after kernel 1 and runs kernels 2, 4 and 7 over that list only, with the surface
  * cells of kernel 3 and the pull in launches of their own. */
-static void launch_step(const StepConsts &s, const waam_step_fields &f, hipStream_t st,
+/* kernels 1 to 4 */
+static void launch_heat(const StepConsts &s, const waam_step_fields &f, hipStream_t st,
                         bool capture)
 {
     const waam_step_params &p = s.p;
@@ -2922,19 +2939,45 @@ static void launch_step(const StepConsts &s, const waam_step_fields &f, hipStrea
                      dim3(resident_blocks(k_step_vof_flags_seg, kBlock)), block3(), st, a, b, f, s);
         else launch_k(capture, k_step_vof_flags, g3, block3(), st, a, b, f, s);
     });
+}
+
+__global__ void k_copy3(const float *__restrict__ ax, const float *__restrict__ ay,
+                        const float *__restrict__ az, float *__restrict__ bx,
+                        float *__restrict__ by, float *__restrict__ bz, size_t N)
+{
+    size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= N) return;
+    bx[c] = ax[c];
+    by[c] = ay[c];
+    bz[c] = az[c];
+}
+
+template <int PD, bool LZ>
+static void launch_collide(const StepConsts &s, const waam_step_fields &f, const LorentzFields &lz,
+                           hipStream_t st, bool capture, hipEvent_t a, hipEvent_t b)
+{
+    launch_k(capture, k_step_collide<PD, LZ>, dim3(resident_blocks(k_step_collide<PD, LZ>, kBlock)),
+             dim3(kBlock), st, a, b, f, s, lz);
+}
+
+/* kernels 5 to 7; lz: with the Lorentz force, on fp32 populations */
+static void launch_flow(const StepConsts &s, const waam_step_fields &f, hipStream_t st,
+                        bool capture, const LorentzFields *lz)
+{
+    const waam_step_params &p = s.p;
+    const Dims &d = s.d;
+    dim3 g3 = grid3(d);
+    const bool seg = p.quiet_skip != 0;
     timed_launch(WAAM_K_COLLIDE, [&](hipEvent_t a, hipEvent_t b) {
-        if (f.pop_dtype == WAAM_POP_F16)
-            launch_k(capture, k_step_collide<WAAM_POP_F16>,
-                     dim3(resident_blocks(k_step_collide<WAAM_POP_F16>, kBlock)), dim3(kBlock), st,
-                     a, b, f, s);
+        const LorentzFields none{};
+        if (lz)
+            launch_collide<WAAM_POP_F32, true>(s, f, *lz, st, capture, a, b);
+        else if (f.pop_dtype == WAAM_POP_F16)
+            launch_collide<WAAM_POP_F16, false>(s, f, none, st, capture, a, b);
         else if (f.pop_dtype == WAAM_POP_BF16)
-            launch_k(capture, k_step_collide<WAAM_POP_BF16>,
-                     dim3(resident_blocks(k_step_collide<WAAM_POP_BF16>, kBlock)), dim3(kBlock), st,
-                     a, b, f, s);
+            launch_collide<WAAM_POP_BF16, false>(s, f, none, st, capture, a, b);
         else
-            launch_k(capture, k_step_collide<WAAM_POP_F32>,
-                     dim3(resident_blocks(k_step_collide<WAAM_POP_F32>, kBlock)), dim3(kBlock), st,
-                     a, b, f, s);
+            launch_collide<WAAM_POP_F32, false>(s, f, none, st, capture, a, b);
     });
     const bool by_record = seg && pulls_by_record(d);
     if (f.max_tracers > 0 && !by_record)
@@ -2999,6 +3042,13 @@ static void launch_step(const StepConsts &s, const waam_step_fields &f, hipStrea
     });
 }
 
+static void launch_step(const StepConsts &s, const waam_step_fields &f, hipStream_t st,
+                        bool capture)
+{
+    launch_heat(s, f, st, capture);
+    launch_flow(s, f, st, capture, nullptr);
+}
+
 }  // namespace waam
 
 /* a captured run of fused steps (waam_graph_capture) */
@@ -3057,6 +3107,44 @@ int waam_step_fused(const waam_step_params *pp, const waam_step_fields *ff, void
     StepConsts s = make_step_consts(p, d);
     launch_step(s, f, as_stream(stream), false);
     return check_launch("waam_step_fused");
+}
+
+int waam_step_fused_lorentz(const waam_step_params *pp, const waam_step_fields *ff,
+                            const waam_lorentz *lp, waam_lorentz_result *out, void *stream)
+{
+    const char *who = "waam_step_fused_lorentz";
+    if (!pp || !ff || !lp || !out) return set_error(WAAM_ERR_INVALID, "%s: NULL argument", who);
+    const waam_step_params &p = *pp;
+    const waam_step_fields &f = *ff;
+    WAAM_RETURN_IF(check_fields(who, f));
+    WAAM_RETURN_IF(check_tables(who, p, f));
+    if (p.col_i < 0 || p.col_i >= f.nx || p.col_j < 0 || p.col_j >= f.ny)
+        return set_error(WAAM_ERR_INVALID, "%s: arc column outside the grid", who);
+    if (!p.is_welding || p.arc_applied || p.use_arc_k_override || !p.enable_vof ||
+        f.pop_dtype != WAAM_POP_F32)
+        return set_error(WAAM_ERR_INVALID,
+                         "%s: needs a welding step that resolves the arc itself, the VOF rules "
+                         "and fp32 populations", who);
+    waam_lorentz q = *lp;
+    if (q.nx != f.nx || q.ny != f.ny || q.nz != f.nz || q.layout != f.layout)
+        return set_error(WAAM_ERR_INVALID, "%s: the two grids differ", who);
+    WAAM_RETURN_IF(check_lorentz(who, q));
+    WAAM_RETURN_IF(check_ptrs(who, {q.Fx_snap, q.Fy_snap, q.Fz_snap, f.Fx, f.Fy, f.Fz}));
+    q.f_l = f.fl_out;
+    q.flags = f.flags_out;
+    q.scratch = f.scratch;
+    Dims d{f.nx, f.ny, f.nz, f.layout};
+    StepConsts s = make_step_consts(p, d);
+    hipStream_t st = as_stream(stream);
+    launch_heat(s, f, st, false);
+    /* where step_arc_k finds it on such a step */
+    const float *arc_k = reinterpret_cast<const float *>((char *)f.scratch + kScratchTelemetry) + 2;
+    WAAM_RETURN_IF(lorentz_run(who, q, arc_k, false, *out, st));
+    const LorentzFields lz{q.Jx, q.Jy, q.Jz, q.Bx, q.By, q.Bz, q.dt, q.dx, q.rho};
+    launch_flow(s, f, st, false, &lz);
+    hipLaunchKernelGGL(k_copy3, dim3(grid_for(d.n())), dim3(kBlock), 0, st, f.Fx, f.Fy, f.Fz,
+                       q.Fx_snap, q.Fy_snap, q.Fz_snap, d.n());
+    return check_launch(who);
 }
 
 }  // extern "C"

@@ -143,6 +143,9 @@ class WAAMGrid:
         self.n_elec_bins = 64
         self.elec_rad_bins = DeviceField.zeros((self.nz, self.n_elec_bins), torch.float32,
                                                self.device)
+        # the bins before their running sum (an array of its own, see waam_lorentz_solve)
+        self.elec_bins_raw = DeviceField.zeros((self.nz, self.n_elec_bins), torch.float32,
+                                               self.device)
         self.elec_l1_buf = DeviceField.zeros((2,), torch.float32, self.device)
         self._has_lorentz = True
         self._n_optional_volume += 10

@@ -13,6 +13,7 @@ pre-kernel field (Jacobi order), which is the one deterministic order a parallel
 
 from __future__ import annotations
 
+import ctypes
 import math
 
 import torch
@@ -734,6 +735,60 @@ def apply_lorentz_JxB(Fx, Fy, Fz, Jx, Jy, Jz, Bx, By, Bz, f_l, flags, dt, dx, rh
     _need(_n(Fx), Fy, Fz, Jx, Jy, Jz, Bx, By, Bz, f_l, flags)
     _call("waam_apply_lorentz_JxB", P(Fx), P(Fy), P(Fz), P(Jx), P(Jy), P(Jz), P(Bx), P(By), P(Bz),
           P(f_l), P(flags), dt, dx, rho_ref, _n(Fx), _stream())
+
+
+class LorentzC(ctypes.Structure):
+    """include/waam_hip.h waam_lorentz."""
+
+    _fields_ = ([(n, ctypes.c_void_p) for n in (
+        "phi", "phi_tmp", "sigma", "source", "Jx", "Jy", "Jz", "Bx", "By", "Bz", "bins",
+        "bins_raw", "l1", "Fx", "Fy", "Fz", "Fx_snap", "Fy_snap", "Fz_snap", "f_l", "flags",
+        "scratch", "bead_top")] +
+        [("tol", ctypes.c_double)] +
+        [(n, ctypes.c_float) for n in (
+            "arc_i", "arc_j", "arc_k", "sigma_cells", "current", "dx", "sigma_liquid",
+            "sigma_solid", "omega", "bin_dr", "mu0", "dt", "rho")] +
+        [(n, ctypes.c_int32) for n in (
+            "nz_solid", "n_bins", "cold", "max_sweeps", "nx", "ny", "nz", "layout")])
+
+
+class LorentzResultC(ctypes.Structure):
+    """include/waam_hip.h waam_lorentz_result."""
+
+    _fields_ = [("res", ctypes.c_float), ("norm", ctypes.c_float), ("sweeps", ctypes.c_int32),
+                ("converged", ctypes.c_int32), ("in_tmp", ctypes.c_int32),
+                ("arc_k", ctypes.c_float), ("bead_top", ctypes.c_int32)]
+
+
+def lorentz_struct(g, arc, sigma_cells, current_A, sigma_liquid, sigma_solid, omega_j, nz_solid,
+                   bin_dr_cells, mu0, rho_ref, max_sweeps, tol, cold) -> LorentzC:
+    """The waam_lorentz of a grid's fields."""
+    _need(g.nx * g.ny * g.nz, g.phi_elec, g.phi_elec_tmp, g.sigma_elec, g.elec_source, g.Jx, g.Jy,
+          g.Jz, g.Bx, g.By, g.Bz, g.Fx, g.Fy, g.Fz, g.Fx_snap, g.Fy_snap, g.Fz_snap, g.f_l, g.flags)
+    if min(_n(g.elec_rad_bins), _n(g.elec_bins_raw)) < g.nz * g.n_elec_bins:
+        raise ValueError("bins must hold nz x n_bins values")
+    return LorentzC(
+        P(g.phi_elec), P(g.phi_elec_tmp), P(g.sigma_elec), P(g.elec_source), P(g.Jx), P(g.Jy),
+        P(g.Jz), P(g.Bx), P(g.By), P(g.Bz), P(g.elec_rad_bins), P(g.elec_bins_raw),
+        P(g.elec_l1_buf), P(g.Fx), P(g.Fy), P(g.Fz), P(g.Fx_snap), P(g.Fy_snap), P(g.Fz_snap),
+        P(g.f_l), P(g.flags), P(g.scratch), None, float(tol), arc[0], arc[1], arc[2], sigma_cells, current_A, g.dx, sigma_liquid,
+        sigma_solid, omega_j, bin_dr_cells, mu0, g.dt, rho_ref, int(nz_solid),
+        int(g.n_elec_bins), int(cold), int(max_sweeps), g.nx, g.ny, g.nz, layout_of(g.phi_elec))
+
+
+def lorentz_done(g, r: LorentzResultC) -> LorentzResultC:
+    """After a solve: ``g.phi_elec`` names the buffer that holds the potential."""
+    if r.in_tmp:
+        g.phi_elec, g.phi_elec_tmp = g.phi_elec_tmp, g.phi_elec
+    return r
+
+
+def lorentz_solve(g, *args, **kw) -> LorentzResultC:
+    """The entries above in solve order (reference physics/weld_forces.py:196-281), on a grid's
+    Lorentz fields, with the force added to its Fx, Fy, Fz. Arguments: ``lorentz_struct``."""
+    q, r = lorentz_struct(g, *args, **kw), LorentzResultC()
+    _call("waam_lorentz_solve", ctypes.addressof(q), ctypes.addressof(r), _stream())
+    return lorentz_done(g, r)
 
 
 # ------------------------------------------------------------------ export-side fields

@@ -32,7 +32,10 @@ def measure_bead_height_m(twin, g) -> float:
     from .. import kernels
 
     kernels.bead_top_k(g.flags, twin.nz_solid, g.bead_top_buf)
-    top = int(g.bead_top_buf.to_numpy()[0])
+    return _bead_height_m(twin, g, int(g.bead_top_buf.to_numpy()[0]))
+
+
+def _bead_height_m(twin, g, top: int) -> float:
     if top < 0:
         return 0.0
     return float((top - twin.nz_solid + 1) * g.dx)
@@ -43,6 +46,14 @@ def update_ctwd(twin, g) -> None:
     physics/electrical_stickout.py:53-59)."""
     if not twin.enable_ctwd:
         return
-    h_meas = measure_bead_height_m(twin, g)
+    set_ctwd(twin, measure_bead_height_m(twin, g))
+
+
+def set_ctwd_from_top(twin, g, top: int) -> None:
+    """``update_ctwd`` on a bead top (``waam_bead_top_k``) that was read elsewhere."""
+    set_ctwd(twin, _bead_height_m(twin, g, top))
+
+
+def set_ctwd(twin, h_meas: float) -> None:
     twin._bead_height_m = h_meas
     twin.ctwd_m = max(twin.ctwd_nominal_m, twin.ctwd_nominal_m + (h_meas - twin.layer_height_m))

@@ -36,7 +36,7 @@ from .. import kernels
 from .._lib import lib
 from ..field import DeviceField, P, tensor_of, write_epoch
 from ..physics import weld_forces
-from ..physics.electrical_stickout import update_ctwd
+from ..physics.electrical_stickout import set_ctwd_from_top, update_ctwd
 from ..gpu_tables import MaterialTablesC, PropertyRefsC
 from .coupled_step import (_clamp_enthalpy_ceiling, _droplet, droplet_due, droplet_plan,
                            resolve_arc_k)
@@ -351,15 +351,28 @@ class FusedStepper:
         k_robot = tw.nz_solid + (z_bead - tw.substrate_z_m) / g.dx - 1.0
         return max(float(tw.nz_solid) + 0.5, min(k_robot, float(g.nz) - 2.0))
 
+    def takes_lorentz(self, is_welding: bool) -> bool:
+        """Whether a step of a twin with the Lorentz force is a fused one: fp32 populations, the
+        VOF rules (the force then acts on the colliding cells only), stored forces, and an arc
+        that the step itself places."""
+        tw = self.twin
+        if (self.pop_code or not tw.enable_vof or not tw.snapshot_forces
+                or self.entry != "waam_step_fused"):
+            return False
+        return not (is_welding and (type(tw.arc_source).__name__ == "ConicalVolume"
+                                    or droplet_due(tw, tw.grid)))
+
     def step(self, torch_x_m: float, torch_y_m: float, is_welding: bool,
              torch_z_m: float | None = None) -> None:
         tw, g = self.twin, self.twin.grid
-        if tw.enable_lorentz:
-            raise NotImplementedError("the Lorentz force solve is not built")
+        if tw.enable_lorentz and not self.takes_lorentz(is_welding):
+            raise NotImplementedError("a Lorentz step of this kind runs in the other engine")
         arc_i = torch_x_m / g.dx
         arc_j = torch_y_m / g.dx
         p = self._params(arc_i, arc_j, is_welding, torch_z_m)
-        if tw.enable_ctwd:
+        # a step with the Lorentz solve reads the bead's top back with the solve's own result
+        lorentz = tw.enable_lorentz and is_welding
+        if tw.enable_ctwd and not lorentz:
             # after arc_k's inputs, before this step changes the flags (reference order)
             update_ctwd(tw, g)
         conical = type(tw.arc_source).__name__ == "ConicalVolume"
@@ -403,9 +416,24 @@ class FusedStepper:
         if drop is not None:
             lib().call("waam_step_fused_droplet", ctypes.addressof(p), ctypes.addressof(fields),
                        ctypes.addressof(drop), torch.cuda.current_stream().cuda_stream)
+        elif lorentz:
+            args = weld_forces.lorentz_args(tw, g, arc_i, arc_j, 0.0)
+            q, r = kernels.lorentz_struct(g, **args), kernels.LorentzResultC()
+            if tw.enable_ctwd:
+                kernels.bead_top_k(g.flags, tw.nz_solid, g.bead_top_buf)
+                q.bead_top = P(g.bead_top_buf)
+            lib().call("waam_step_fused_lorentz", ctypes.addressof(p), ctypes.addressof(fields),
+                       ctypes.addressof(q), ctypes.addressof(r),
+                       torch.cuda.current_stream().cuda_stream)
+            weld_forces.note_lorentz(tw, kernels.lorentz_done(g, r), args)
+            tw._last_arc_ijk = (float(arc_i), float(arc_j), float(r.arc_k))
+            if tw.enable_ctwd:
+                set_ctwd_from_top(tw, g, r.bead_top)
         else:
             lib().call(self.entry, ctypes.addressof(p), ctypes.addressof(fields),
                        torch.cuda.current_stream().cuda_stream)
+            if tw.enable_lorentz:  # such a twin's snapshot fields follow every step
+                kernels.snapshot_forces(g.Fx, g.Fy, g.Fz, g.Fx_snap, g.Fy_snap, g.Fz_snap)
         for a, b in (("H", "H_tmp"), ("T", "T_tmp"), ("f_l", "fl_tmp"), ("flags", "flags_tmp"),
                      ("sflags", "sflags_tmp")):
             _swap(g, a, b)

@@ -392,15 +392,15 @@ class WAAMTwin:
             self._maybe_shift_window(torch_x_m)
         sim_x = torch_x_m - self._window_offset_x_m - self._sim_origin_offset_x_m
         sim_y = torch_y_m - self._sim_origin_offset_y_m
-        if self.engine == "fused" and self.enable_lorentz:
-            # the Lorentz solve (a Jacobi iteration over the whole grid that dominates such a
-            # step) runs through the reference-order kernels, which give the same fields
-            self.sync()
-            coupled_step(self, sim_x, sim_y, is_welding, torch_z_m)
-        elif self.engine == "fused":
+        if self.engine == "fused":
             if self._fused is None:
                 self._fused = FusedStepper(self)
-            self._fused.step(sim_x, sim_y, is_welding, torch_z_m)
+            if self.enable_lorentz and not self._fused.takes_lorentz(is_welding):
+                # the reference-order kernels give the same fields
+                self.sync()
+                coupled_step(self, sim_x, sim_y, is_welding, torch_z_m)
+            else:
+                self._fused.step(sim_x, sim_y, is_welding, torch_z_m)
         elif self.engine == "reference":
             self.sync()
             coupled_step(self, sim_x, sim_y, is_welding, torch_z_m)
