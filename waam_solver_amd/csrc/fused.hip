@@ -1601,16 +1601,17 @@ __global__ void __launch_bounds__(256) k_step_thermal_surface(waam_step_fields f
 /* 2, 2p and 3 of a steady step in one launch: the first `surface` blocks take the listed
  * FLUID/IFACE cells (the longest chain, so first), the next `walk` the active segments, the rest
  * the plate's cold segments. Every block forms the arc total itself (nparts > 0), for a
- * microsecond where a launch between kernel 1 and this one costs four and a half. Constant material: with the tables the two inlined copies of the
- * cell routine make the compiler copy the argument structs to private memory */
+ * microsecond where a launch between kernel 1 and this one costs four and a half. 200x100x62 with
+ * tables: 29 us, 24 + 17 in launches of their own and 4.6 for the total's. */
+template <bool TAB>
 __global__ void __launch_bounds__(256) k_step_thermal_steady(waam_step_fields f, StepConsts s,
                                                              int surface, int walk, int nparts)
 {
     const int b = (int)blockIdx.x;
     const float epw = nparts > 0 ? arc_total(f, s, nparts, b == 0) : 0.0f;
-    if (b < surface) thermal_surface_list<false>(f, s, epw, b, surface);
-    else if (b < surface + walk) thermal_walk<false>(f, s, epw, b - surface, walk);
-    else plate_march(f, s, epw, b - surface - walk);
+    if (b < surface) thermal_surface_list<TAB>(f, s, epw, b, surface);
+    else if (b < surface + walk) thermal_walk<TAB>(f, s, epw, b - surface, walk);
+    else if (!TAB) plate_march(f, s, epw, b - surface - walk);
 }
 
 /* 2+3 in one launch, when the previous step's kernel 7 has listed this step's FLUID/IFACE
@@ -2845,8 +2846,14 @@ constexpr int kSteadyWalkBlocks = 512;
  * 73 + 18 + 41 apart; the 1536 of 512x256x128 52 and 31 + 12 + 15, the 600 of 301x157x83 31 and
  * 19 + 9 + 18, the 30 of 64x40x32 16 and 8 + 7 + 15. */
 constexpr int kTogetherBlocks = 2048;
-static bool thermal_together(const Dims &d)
+/* With the tables there is no plate march, so the walk has the plate's segments too and fills the
+ * chip sooner: up to this many row segments together (a step of 200x100x62, 24800 of them, 94 us
+ * together and 105 apart; 256x128x64, 32768, 107 and 115; 320x160x72, 57600, 137 and 136;
+ * 400x200x100, 140000, 223 and 203). */
+constexpr size_t kTogetherTableSegments = 40960;
+static bool thermal_together(const Dims &d, bool tab)
 {
+    if (tab) return quiet_segments(d) <= kTogetherTableSegments;
     return (d.nx + kTileFast - 1) / kTileFast * plate_row_blocks(d) * kPlateChunks <=
            kTogetherBlocks;
 }
@@ -2864,7 +2871,7 @@ static void launch_heat(const StepConsts &s, const waam_step_fields &f, hipStrea
     const bool seg = p.quiet_skip != 0;
     int do_sums = p.is_welding && !p.arc_applied ? 1 : 0;
     const bool tab = p.use_tables != 0;
-    const bool together = seg && !tab && thermal_together(d);
+    const bool together = seg && thermal_together(d, tab);
     const int nsum = do_sums ? sum_blocks(d) : 1;
     timed_launch(WAAM_K_BEGIN, [&](hipEvent_t a, hipEvent_t b) {
         const bool total = do_sums && !together;
@@ -2894,9 +2901,14 @@ static void launch_heat(const StepConsts &s, const waam_step_fields &f, hipStrea
         const unsigned plate = plate_slices(p, d) > 0 ? (unsigned)plate_blocks(d) : 0u;
         timed_launch(WAAM_K_THERMAL, [&](hipEvent_t a, hipEvent_t b) {
             if (together) {
-                launch_k(capture, k_step_thermal_steady,
-                         dim3(kSteadySurfaceBlocks + kSteadyWalkBlocks + plate), block3(), st, a,
-                         b, f, s, kSteadySurfaceBlocks, kSteadyWalkBlocks, do_sums ? nsum : 0);
+                const dim3 gt(kSteadySurfaceBlocks + kSteadyWalkBlocks + plate);
+                const int np = do_sums ? nsum : 0;
+                if (tab)
+                    launch_k(capture, k_step_thermal_steady<true>, gt, block3(), st, a, b, f, s,
+                             kSteadySurfaceBlocks, kSteadyWalkBlocks, np);
+                else
+                    launch_k(capture, k_step_thermal_steady<false>, gt, block3(), st, a, b, f, s,
+                             kSteadySurfaceBlocks, kSteadyWalkBlocks, np);
                 return;
             }
             if (plate > 0)

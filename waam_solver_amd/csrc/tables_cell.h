@@ -13,10 +13,18 @@ __device__ __forceinline__ float lookup_table_1d(float T, const float *t_arr, co
 {
     float result = fallback;
     if (n > 0) {
+        /* the last knot by selects: an array of a kernel's arguments that is indexed by a variable
+         * is copied to private memory in a kernel that inlines this twice */
+        float t_last = t_arr[0], v_last = v_arr[0];
+#pragma unroll
+        for (int idx = 1; idx < WAAM_MAX_KNOTS; ++idx) {
+            t_last = idx < n ? t_arr[idx] : t_last;
+            v_last = idx < n ? v_arr[idx] : v_last;
+        }
         if (T <= t_arr[0]) {
             result = v_arr[0];
-        } else if (T >= t_arr[n - 1]) {
-            result = v_arr[n - 1];
+        } else if (T >= t_last) {
+            result = v_last;
         } else {
             /* the last interval that holds T (as the reference's loop leaves it), then one
              * division: a division per interval under its own branch made four lookups of a
