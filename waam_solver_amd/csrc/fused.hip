@@ -1005,24 +1005,36 @@ __global__ void __launch_bounds__(kBlock, 4) k_step_begin(waam_step_fields f, St
  * 768x384x192: 31.8 us for the two, 512: 28.9) */
 static int sum_blocks(const Dims &d) { return d.n() <= ((size_t)1 << 19) ? 256 : 512; }
 
+/* this thread's pairs of kernel 1's block sums (up to 512 blocks), requested */
+struct ArcParts {
+    double2 v[2];
+};
+__device__ __forceinline__ ArcParts arc_parts(const waam_step_fields &f, int nparts)
+{
+    const double2 *parts = reinterpret_cast<const double2 *>((char *)f.scratch + kScratchPartials);
+    const int t = (int)(threadIdx.y * blockDim.x + threadIdx.x);
+    ArcParts a;
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+        const int b = t + n * kBlock;
+        a.v[n] = b < nparts ? parts[b] : make_double2(0.0, 0.0);
+    }
+    return a;
+}
+
 /* fixed-order total of kernel 1's block sums and the energy per unit weight (reference
  * kernels.py:493-496), formed by a whole block (of kBlock threads); the value is every thread's.
  * store: write both for the rest of the step */
-__device__ __forceinline__ float arc_total(const waam_step_fields &f, const StepConsts &s, int nparts,
-                                           bool store)
+__device__ __forceinline__ float arc_total(const waam_step_fields &f, const StepConsts &s,
+                                           const ArcParts &a, bool store)
 {
     __shared__ double sh_s[kBlock], sh_c[kBlock];
     __shared__ float s_epw;
-    const double2 *parts = reinterpret_cast<const double2 *>((char *)f.scratch + kScratchPartials);
     const int t = (int)(threadIdx.y * blockDim.x + threadIdx.x);
-    double sum = 0.0, comp = 0.0;
-    for (int b = t; b < nparts; b += kBlock) {
-        const double2 pr = parts[b];
-        double ss, e;
-        two_sum(sum, pr.x, ss, e);
-        sum = ss;
-        comp += pr.y + e;
-    }
+    double sum = a.v[0].x, comp = a.v[0].y, ss, e;
+    two_sum(sum, a.v[1].x, ss, e);
+    sum = ss;
+    comp += a.v[1].y + e;
     block_reduce_pair(sum, comp, sh_s, sh_c);
     if (t == 0) {
         const waam_step_params &p = s.p;
@@ -1043,7 +1055,7 @@ __device__ __forceinline__ float arc_total(const waam_step_fields &f, const Step
 __global__ void __launch_bounds__(kBlock) k_step_arc_total(waam_step_fields f, StepConsts s,
                                                            int nparts)
 {
-    (void)arc_total(f, s, nparts, true);
+    (void)arc_total(f, s, arc_parts(f, nparts), true);
 }
 
 /* the energy per unit weight a launch of its own has left */
@@ -1572,22 +1584,41 @@ __global__ void __launch_bounds__(256) k_step_thermal_seg(waam_step_fields f, St
 }
 
 /* thermal chain (with enthalpy advection) and VOF advection of the listed FLUID/IFACE cells;
- * worker b of nb, 256 threads each */
+ * worker b of nb, 256 threads each. nparts > 0: the block forms the arc total itself, with its
+ * operands, the list's lengths and the first cell on their way before it adds them up (1.0 to 1.6 %
+ * of a step of 64x40x32 to 512x256x128; with the tables, whose registers are full, 1.4 to 3 %
+ * slower at 200x100x62: they pass the total in) */
 template <bool TAB>
 __device__ __forceinline__ void thermal_surface_list(const waam_step_fields &f,
-                                                     const StepConsts &s, float epw, int b,
-                                                     int nb)
+                                                     const StepConsts &s, int nparts, bool store,
+                                                     float epw, int b, int nb)
 {
     __shared__ int s_pref[kListSegments + 1];
     const Dims &d = s.d;
     CellList l = cell_list(f, s.d.n(), 0);
+    const ArcParts parts = arc_parts(f, nparts);
     int n = list_prefix(l, s_pref);
-    int tid = threadIdx.y * blockDim.x + threadIdx.x;
-    for (int t = b * kBlock + tid; t < n; t += nb * kBlock) {
-        size_t c = list_at(l, s_pref, t);
+    int t = b * kBlock + (int)(threadIdx.y * blockDim.x + threadIdx.x);
+    if (TAB) {
+        for (; t < n; t += nb * kBlock) {
+            const size_t c = list_at(l, s_pref, t);
+            int i, j, k;
+            cell_ijk(c, d, i, j, k);
+            thermal_vof_cell<TAB>(f, s, epw, i, j, k, c, f.flags_in[c]);
+        }
+        return;
+    }
+    size_t c = t < n ? list_at(l, s_pref, t) : 0;
+    uint8_t flag = f.flags_in[c];
+    if (nparts > 0) epw = arc_total(f, s, parts, store);
+    while (t < n) {
         int i, j, k;
         cell_ijk(c, d, i, j, k);
-        thermal_vof_cell<TAB>(f, s, epw, i, j, k, c, f.flags_in[c]);
+        thermal_vof_cell<false>(f, s, epw, i, j, k, c, flag);
+        t += nb * kBlock;
+        if (t >= n) break;
+        c = list_at(l, s_pref, t);
+        flag = f.flags_in[c];
     }
 }
 
@@ -1595,7 +1626,7 @@ __device__ __forceinline__ void thermal_surface_list(const waam_step_fields &f,
 template <bool TAB>
 __global__ void __launch_bounds__(256) k_step_thermal_surface(waam_step_fields f, StepConsts s)
 {
-    thermal_surface_list<TAB>(f, s, stored_epw(f), blockIdx.x, gridDim.x);
+    thermal_surface_list<TAB>(f, s, 0, false, stored_epw(f), blockIdx.x, gridDim.x);
 }
 
 /* 2, 2p and 3 of a steady step in one launch: the first `surface` blocks take the listed
@@ -1608,8 +1639,12 @@ __global__ void __launch_bounds__(256) k_step_thermal_steady(waam_step_fields f,
                                                              int surface, int walk, int nparts)
 {
     const int b = (int)blockIdx.x;
-    const float epw = nparts > 0 ? arc_total(f, s, nparts, b == 0) : 0.0f;
-    if (b < surface) thermal_surface_list<TAB>(f, s, epw, b, surface);
+    if (!TAB && b < surface) {
+        thermal_surface_list<false>(f, s, nparts, b == 0, 0.0f, b, surface);
+        return;
+    }
+    const float epw = nparts > 0 ? arc_total(f, s, arc_parts(f, nparts), TAB && b == 0) : 0.0f;
+    if (b < surface) thermal_surface_list<TAB>(f, s, 0, false, epw, b, surface);
     else if (b < surface + walk) thermal_walk<TAB>(f, s, epw, b - surface, walk);
     else if (!TAB) plate_march(f, s, epw, b - surface - walk);
 }
