@@ -165,40 +165,33 @@ def cpu_baseline(w: dict, seconds: float, one_thread_steps: int) -> dict:
     return out
 
 
-# The dominant kernel is k_step_pull, the deferred pull stream of the populations (a launch of
-# its own ahead of k_step_stream). Its algorithmic bytes per launch (each array element touched
-# once; neighbour re-reads not counted):
-#   every cell        flags read, previous stream flags read                         2 B
-#   pulled cell       19 populations read + 19 written: fp32 152 B, 16-bit storage  76 B
-# A pulled cell is one the collision skips this step that was not SOLID at the step whose
-# stream is being completed.
-STREAM_B_EVERY = 2
-STREAM_B_PULL = {"fp32": 152, "fp16": 76, "bf16": 76}
-# Whole-step compulsory bytes by cell class (each persistent field read and written once):
-#   every cell          H T f_l phi r/w 32 B, u r/w 24 B, flags r/w 2 B, rho w 4 B    62 B
-#   non-SOLID cell      populations read + written: 2 x 19 x 4 B (fp32), 2 x 19 x 2 B (16-bit)
-#   non-GAS cell        HAZ fields: T_max r/w, T_prev r/w, dT_dt w, three time-above r/w  44 B
-# SOLID cells neither collide nor stream; GAS cells skip every HAZ update (reference
-# kernels.py:2971-3010, 3016-3032, 2013-2027, 3261-3283).
-STEP_B_EVERY = 62
+# The dominant kernel is k_step_thermal: the enthalpy chain of the plate, marched along z, and of
+# the listed row segments (on grids that do not fill the chip the surface cells share the launch).
+# Its algorithmic bytes per launch are those of the SOLID cells, each array element touched once
+# (neighbour re-reads and the listed GAS cells not counted):
+#   SOLID cell          H, T, T_prev, T_max read; H, T, T_prev, dT/dt written       32 B
+THERMAL_B_SOLID = 32
+# What a whole step cannot do without: the SOLID cells' chain as above, and for each collided
+# (FLUID/IFACE) cell
+#   H T f_l phi r/w 32 B, u r/w 24 B, flags r/w 2 B, rho w 4 B, HAZ fields (T_max r/w, T_prev r/w,
+#   dT_dt w, three time-above r/w) 44 B                                              106 B
+#   populations read + written: 2 x 19 x 4 B (fp32), 2 x 19 x 2 B (16-bit)
+# The gas and the plate's other fields stand still from step to step and cost nothing.
+STEP_B_SURFACE = 106
 STEP_B_POP = {"fp32": 152, "fp16": 76, "bf16": 76}
-STEP_B_HAZ = 44
-DOMINANT = "k_step_pull"
+DOMINANT = "k_step_thermal"
 TIMING_EVERY = 4
 
 
 def traffic_file(w: dict, pop: str) -> str:
     return os.path.join(ROOT, "profiles",
-                        f"k_step_pull_bead_on_plate_{w['nx']}x{w['ny']}x{w['nz']}_{pop}_pmc.md")
+                        f"k_step_thermal_bead_on_plate_{w['nx']}x{w['ny']}x{w['nz']}_{pop}_pmc.md")
 
 
-def stream_classes(g) -> tuple[int, int]:
-    """(collided cells, pulled cells) of the last fused step, from its stream flags."""
+def collided_cells(g) -> int:
+    """Cells the last fused step collided, from its stream flags."""
     cur = g.sflags.to_numpy()
-    prev = g.sflags_tmp.to_numpy()
-    active = (cur == 0) | (cur == 4)
-    pull = (~active) & (prev != 1)
-    return int(active.sum()), int(pull.sum())
+    return int(((cur == 0) | (cur == 4)).sum())
 
 
 def cell_classes(g) -> tuple[int, int]:
@@ -211,19 +204,14 @@ def cell_classes(g) -> tuple[int, int]:
     return int((fl == 1).sum().item()), int((fl == 2).sum().item())
 
 
-def stream_bytes(ncell: int, pull: float, pop: str = "fp32") -> float:
-    return STREAM_B_EVERY * ncell + STREAM_B_PULL[pop] * pull
-
-
-def step_bytes(ncell: int, solid: float, gas: float, pop: str) -> float:
-    return (STEP_B_EVERY * ncell + STEP_B_POP[pop] * (ncell - solid)
-            + STEP_B_HAZ * (ncell - gas))
+def step_bytes(solid: float, collided: float, pop: str) -> float:
+    return THERMAL_B_SOLID * solid + (STEP_B_SURFACE + STEP_B_POP[pop]) * collided
 
 
 def timed_run(w: dict, args, pop: str):
     """Build the seeded twin with population storage `pop`, step the pre-roll (captured steps)
     and the warm-up, then time args.steps steps. Returns (twin, seconds, host seconds, (solid, gas) averaged over the
-    start and end of the timed steps, (collided, pulled) likewise)."""
+    start and end of the timed steps, collided cells likewise)."""
     import torch
 
     tw = build_gpu_twin(w, pop)
@@ -238,11 +226,11 @@ def timed_run(w: dict, args, pop: str):
     torch.cuda.synchronize()
     fused = args.engine == "fused"
     cls0 = cell_classes(g)
-    sc0 = stream_classes(g) if fused and hasattr(g, "sflags_tmp") else None
+    sc0 = collided_cells(g) if fused and hasattr(g, "sflags_tmp") else None
     if fused:
         from waam_solver_amd._lib import STEP_KERNELS, lib
 
-        # every fourth step's pull carries the timing events (each recorded dispatch costs a
+        # every fourth step's kernel carries the timing events (each recorded dispatch costs a
         # few microseconds of the step)
         lib().call("waam_timing_begin_every", STEP_KERNELS.index(DOMINANT),
                    (args.steps + TIMING_EVERY - 1) // TIMING_EVERY, TIMING_EVERY)
@@ -263,9 +251,8 @@ def timed_run(w: dict, args, pop: str):
     classes = ((cls0[0] + cls1[0]) / 2.0, (cls0[1] + cls1[1]) / 2.0)
     sc = None
     if fused:
-        sc1 = stream_classes(g)
-        sc0 = sc0 or sc1
-        sc = ((sc0[0] + sc1[0]) / 2.0, (sc0[1] + sc1[1]) / 2.0)
+        sc1 = collided_cells(g)
+        sc = ((sc0 if sc0 is not None else sc1) + sc1) / 2.0
     return tw, el, t_host, classes, sc, timing
 
 
@@ -292,10 +279,10 @@ def compare_form(w: dict, args, pop: str):
     (twin, MLUPS, summary). The forms' errors against a binary64 build are measured over 2000
     steps with a molten pool by tests/precision_c3.py; main() adds each 16-bit form's error
     against this fp32 run over the same steps."""
-    tw, el, _, classes, _, _ = timed_run(w, args, pop)
+    tw, el, _, classes, sc, _ = timed_run(w, args, pop)
     g = tw.grid
     mlups = g.n_cells * args.steps / el / 1e6
-    sb = step_bytes(g.n_cells, classes[0], classes[1], pop)
+    sb = step_bytes(classes[0], sc, pop)
     out = {"value": round(mlups, 2), "ms_per_step": round(el * 1e3 / args.steps, 4),
            "step_bytes_per_cell": round(sb / g.n_cells, 1),
            "step_frac": round(sb * args.steps / el / 1e9 / HBM_PEAK_GBS, 4)}
@@ -424,7 +411,7 @@ def multipass(args) -> int:
 
 
 def measured_traffic(w: dict, pop: str) -> dict | None:
-    """HBM bytes per k_step_pull launch and per step from the committed rocprofv3 counter
+    """HBM bytes per launch of the dominant kernel and per step from the committed rocprofv3 counter
     summary of this workload and population form."""
     out = {}
     try:
@@ -546,18 +533,18 @@ def main() -> int:
     roofline = None
     if fused:
         tot_ms, n_launch = timing
-        per_launch = stream_bytes(ncell, sc[1], args.pop)
+        per_launch = THERMAL_B_SOLID * classes[0]
         avg_s = tot_ms / 1e3 / max(n_launch, 1)
         achieved = per_launch / avg_s / 1e9
         meas = measured_traffic(w, args.pop)
-        sb = step_bytes(ncell, classes[0], classes[1], args.pop)
+        sb = step_bytes(classes[0], sc, args.pop)
         roofline = {"bound": "hbm", "kernel": DOMINANT, "achieved": round(achieved, 1),
                     "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                     "traffic": meas.get("traffic_bytes_per_launch") if meas else None,
                     "algorithmic_bytes_per_launch": round(per_launch),
                     "avg_launch_us": round(avg_s * 1e6, 2), "timed_launches": n_launch,
                     "timed_every": TIMING_EVERY,
-                    "cells_collided": round(sc[0]), "cells_pulled": round(sc[1]),
+                    "cells_collided": round(sc),
                     "step": {"compulsory_bytes_per_cell": round(sb / ncell, 1),
                              "cells_solid": round(classes[0]), "cells_gas": round(classes[1]),
                              "achieved": round(sb * args.steps / el / 1e9, 1),
@@ -627,7 +614,7 @@ def main() -> int:
                    "engine": args.engine, "population_storage": args.pop,
                    "pool_width_mm": tel["pool_width_mm"], "pool_depth_mm": tel["pool_depth_mm"],
                    "peak_temp_K": tel["peak_temp_K"], "n_droplets": tel["n_droplets_fired"],
-                   "surface_cells": round(sc[0]) if sc else None},
+                   "surface_cells": round(sc) if sc is not None else None},
     }
     if roofline is not None:
         result["roofline"] = roofline

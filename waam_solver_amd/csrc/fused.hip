@@ -1,4 +1,4 @@
-// fused.hip — the coupled step in seven launches (waam_step_fused).
+// fused.hip — the coupled step in six to nine launches (waam_step_fused).
 //
 // Launch sequence for one step (reference solvers/coupled_step.py:73-464):
 //   1 k_step_begin           torch-column surface height (arc_k); arc weight partial sums
@@ -18,12 +18,12 @@
 //   7 k_step_stream          every other cell: the previous step's pull stream, force reset;
 //                            every cell: remelt, trailing-pool and cooled-metal solidification
 // On steady steps (the row-segment record below) 2, 4 and 7 walk a list of the row segments
-// whose results can change (k_step_quiet_list builds it after 1, with the arc total in its last
-// block), the pull runs after 5 over the directions and segments whose populations do not stand
-// still (k_step_pull_seg, with the tracers; other steps pull everything ahead of 7 in launches of
-// its own), 2 and 3 share a launch on grids that do not fill the chip (k_step_thermal_steady: a
-// steady step is then seven launches), and in the ZYX layout the plate's cold segments are
-// marched along z by k_step_thermal_plate instead of being listed.
+// whose results can change (built beside 1 in its launch), the pull runs after 5 over the
+// directions and segments whose populations do not stand still (k_step_pull_seg, with the tracers;
+// other steps pull everything ahead of 7 in launches of its own), 2, 3 and the arc total share a
+// launch on grids that do not fill the chip (k_step_thermal_steady: a steady step is then six
+// launches), and in the ZYX layout the plate's cold segments are marched along z (plate_march)
+// instead of being listed. waam_step_fused_lorentz runs the Lorentz solve between 4 and 5.
 // Every cell value is produced by the same fp32 expression sequence as the one-kernel-per-
 // reference-kernel path, so both paths give identical bits.
 //
@@ -2538,12 +2538,12 @@ __global__ void k_advect_tracers_step(float *__restrict__ pos, int32_t *__restri
  * segment, kPullGroup directions' loads in flight (a whole gas segment far above the pool moves
  * its five upward directions, so one round of loads); only words that change are stored, and
  * what changed goes into the destination buffer's change words. 768x384x192 (fp16, 885 k
- * segments, about 75 k listed): 43 us, and 13 us more of kernel 1b, where the full pull took 700;
- * 512x256x128 fp32: 20 + 6 against 378. Bound by the latency of its two rounds of loads (entry
+ * segments, about 75 k listed): 43 us, and 7 us more of the segment list's launch, where the full pull took
+ * 700; 512x256x128 fp32: 19 against 378. Bound by the latency of its two rounds of loads (entry
  * and flags, then the rows) per segment. Kernel 4 left the step's flags before the
  * freeze rules in sflags_next. The first `tracers` blocks advect the tracers (kernel 6: after the
- * collision, before the freeze rules, as the pull; a launch of their own cost them 4.5 us). Values are those of the full pulls (the words they
- * would rewrite unchanged are left alone). A segment may be on the list twice: both wavefronts
+ * collision, before the freeze rules, as the pull; a launch of their own cost them 4.5 us). Values
+ * are those of the full pulls (the words they would rewrite unchanged are left alone). A segment may be on the list twice: both wavefronts
  * form the same words, and the one that finds a word different records it. */
 constexpr int kPullGroup = 5;
 constexpr int kPullItems = (Q + kPullGroup - 1) / kPullGroup;
@@ -2893,10 +2893,10 @@ static bool thermal_together(const Dims &d, bool tab)
            kTogetherBlocks;
 }
 
-/* the step's launches in order (kernels 1-7). A steady step (s.p.quiet_skip) lists its active
- * row segments after kernel 1 and runs kernels 2, 4 and 7 over that list only, with the surface
- * cells of kernel 3 and the pull in launches of their own. */
-/* kernels 1 to 4 */
+/* The step's launches in order: kernels 1 to 4 here, 5 to 7 in launch_flow. A steady step
+ * (s.p.quiet_skip) lists its active row segments beside kernel 1 and runs kernels 2, 4 and 7 over
+ * that list only, the surface cells of kernel 3 in their launch or one of their own, the pull after
+ * the collision. */
 static void launch_heat(const StepConsts &s, const waam_step_fields &f, hipStream_t st,
                         bool capture)
 {
