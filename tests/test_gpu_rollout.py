@@ -6,6 +6,7 @@ that holds no liquid. (The gradients against binary64 differences: test_gpu_adjo
 from __future__ import annotations
 
 import ctypes
+import math
 
 import numpy as np
 import pytest
@@ -179,3 +180,22 @@ def test_rollout_calls_reject_bad_arguments():
         lib().call("waam_rollout_forward", a(r), a(arcs), a(arcs), 0, None)
     with pytest.raises(WaamError, match="NULL"):
         lib().call("waam_rollout_forward", None, a(arcs), a(arcs), 1, None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("eta", [math.nan, math.inf])
+@pytest.mark.parametrize("mode", ["thermal", "flow"])
+def test_a_bad_efficiency_is_not_swallowed(hip_device, mode, eta, monkeypatch):
+    """An efficiency that is no number reaches every cell that the arc heats, as it does through
+    the per-kernel entries."""
+    from waam_solver_amd.adjoint import CoupledRollout, ThermalRollout
+
+    tw, path = _twin(33, 17, 19, 1)
+    ro = ThermalRollout(tw, 2, path) if mode == "thermal" else CoupledRollout(tw, 2, path)
+    theta = (eta, 1.0, 1.0)
+    monkeypatch.setitem(globals(), "THETA", theta)
+    T, fl = ro.forward(theta)
+    want = _chain(tw, ro, mode == "flow", True)
+    assert np.isnan(want[0]).any() == math.isnan(eta)  # the ceiling bounds an infinite one
+    for name, a, b in zip(("H", "T", "f_l"), (ro.H_final, T, fl), want):
+        assert bits_equal(a.cpu().numpy(), b), mismatch_report(name, a.cpu().numpy(), b)

@@ -44,11 +44,12 @@ __device__ __forceinline__ void roll_ijk(size_t c, const Dims &d, int &i, int &j
     k = d.layout == kLayoutZYX ? b : a;
 }
 
-/* enthalpy after arc injection (A) */
+/* enthalpy after arc injection (A); an energy that is no number is kept out by nothing, as in the
+ * arc's own entry, so that a run with a bad efficiency does not end in a cold plate */
 __device__ __forceinline__ float arc_heated(float h, float fl, float wk, float epw,
                                             const RollConsts &a, int i, int j, int k)
 {
-    if (!(epw > 0.0f)) return h;
+    if (epw <= 0.0f) return h;
     const float wdep = fl > 0.55f ? 1.0f : wk;
     const float hot = h + epw * arc_shape(a.ap, i, j, k) * wdep;
     return wdep < 1e-6f ? h : hot;
