@@ -35,7 +35,7 @@
 extern "C" {
 #endif
 
-#define WAAM_ABI_VERSION 5
+#define WAAM_ABI_VERSION 6
 
 enum { WAAM_FLAG_FLUID = 0, WAAM_FLAG_SOLID = 1, WAAM_FLAG_GAS = 2, WAAM_FLAG_IFACE = 4 };
 /* the moving lid of the lid-driven cavity (waam_cavity_step); not a flag of the coupled step */
@@ -550,10 +550,14 @@ int waam_adj_rollback(const waam_rollout *r, const double *arc_i, const double *
                       void *stream);
 /* The same for the coupled rollout, in binary64: lam_H, lam_u (3 N a slot), lam_f (19 N a slot;
  * NULL without the flow) as above. lam_u, lam_f, lam_T1, lam_fl1 (N) and G (3 N) are read and
- * written on the listed cells only and are 0 elsewhere; lamC, lamB: N doubles of workspace. */
+ * written on the listed cells only and are 0 elsewhere; lamC, lamB: N doubles of workspace. With
+ * the flow, the coefficients of its adjoint in binary64, as waam_cadj_collide_mrt,
+ * waam_cadj_forces and waam_cadj_marangoni take them (those of waam_rollout, which the forward
+ * reads, are fp32). */
 typedef struct waam_rollback {
     double *lam_H, *lam_u, *lam_f, *lam_T1, *lam_fl1, *G, *lamC, *lamB, *parts, *step_totals,
         *grads;
+    double omega_s, omega_b, C_darcy, u_cap, F_cap, g_lu, beta, T_l, dgamma;
     int32_t slot;
 } waam_rollback;
 int waam_cadj_rollback(const waam_rollout *r, const waam_rollback *b, const double *arc_i,

@@ -65,7 +65,9 @@ class RollbackC(ctypes.Structure):
 
     _fields_ = [(n, ctypes.c_void_p) for n in (
         "lam_H", "lam_u", "lam_f", "lam_T1", "lam_fl1", "G", "lamC", "lamB", "parts",
-        "step_totals", "grads")] + [("slot", ctypes.c_int32)]
+        "step_totals", "grads")] + [(n, ctypes.c_double) for n in (
+            "omega_s", "omega_b", "C_darcy", "u_cap", "F_cap", "g_lu", "beta", "T_l",
+            "dgamma")] + [("slot", ctypes.c_int32)]
 
 
 class ThermalRollout:
@@ -414,6 +416,16 @@ class CoupledRollout:
         r.omega_s, r.omega_b, r.C_darcy = tw.omega, tw.omega_bulk, tw.C_darcy
         return r
 
+    def _rollback(self, lam: dict, slot: int) -> RollbackC:
+        """The backward call's parameters; lam holds its buffers (kept by the caller). The flow's
+        coefficients go in binary64: the adjoint is one of the step's equations, whose forward
+        alone is fp32."""
+        tw = self.tw
+        return RollbackC(omega_s=tw.omega, omega_b=tw.omega_bulk, C_darcy=tw.C_darcy,
+                         u_cap=self.u_cap, F_cap=self.F_cap, g_lu=tw.g_lu, beta=tw.beta_T,
+                         T_l=tw.mat.T_liquidus, dgamma=tw.dgamma_dT_lu, slot=slot,
+                         **{k: P(v) for k, v in lam.items()})
+
     def _cells_of(self, t: torch.Tensor) -> torch.Tensor:
         """The listed cells' values of a stack of fields, (fields, cells)."""
         return t.reshape(-1, self.tw.grid.n_cells)[:, self._cells]
@@ -487,7 +499,7 @@ class CoupledRollout:
             self._put(sv, *state)
             self._run(s0, n, sv, stack=True)
             ai, aj = self._arcs(s0, n)
-            b = RollbackC(slot=slot, **{k: P(v) for k, v in lam.items()})
+            b = self._rollback(lam, slot)
             r = self._rollout(sv, True, 0)
             lib().call("waam_cadj_rollback", ctypes.addressof(r),
                        ctypes.addressof(b), ctypes.addressof(ai), ctypes.addressof(aj), n, st)

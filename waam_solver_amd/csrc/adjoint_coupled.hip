@@ -872,8 +872,8 @@ int waam_cadj_rollback(const waam_rollout *r, const waam_rollback *b, const doub
     const size_t N = d.n();
     hipStream_t st = as_stream(stream);
     waam_adj_consts c = r->c;
-    const FlowAdj fa{r->omega_s, r->omega_b, r->C_darcy, r->u_cap, r->F_cap, r->g_lu, r->beta,
-                     c.T_l, r->dgamma, r->enable_hydro};
+    const FlowAdj fa{b->omega_s, b->omega_b, b->C_darcy, b->u_cap, b->F_cap, b->g_lu, b->beta,
+                     b->T_l, b->dgamma, r->enable_hydro};
     for (int t = n - 1, s = b->slot; t >= 0; --t, s ^= 1) {
         c.arc_i = (float)arc_i[t];
         c.arc_j = (float)arc_j[t];
