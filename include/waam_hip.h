@@ -366,7 +366,8 @@ int waam_apply_lorentz_JxB(float *Fx, float *Fy, float *Fz, const float *Jx, con
 typedef struct waam_lorentz {
     float *phi, *phi_tmp;     /* potential in, and the Jacobi partner */
     float *sigma, *source, *Jx, *Jy, *Jz, *Bx, *By, *Bz;
-    float *bins, *bins_raw;   /* nz x n_bins each; bins gets the enclosed current */
+    float *bins, *bins_raw;   /* nz x n_bins each; bins gets the enclosed current; bins_raw, a
+                               * workspace, may be null */
     float *l1;                /* device, 2 floats: as waam_elec_l1_diff */
     float *Fx, *Fy, *Fz;
     float *Fx_snap, *Fy_snap, *Fz_snap;  /* waam_step_fused_lorentz: the step's forces copied */

@@ -127,3 +127,28 @@ def test_fused_steps_equal_the_entries(hip_device, layout, name, overrides):
         if welding:
             assert np.float32(a._last_arc_ijk[2]) == np.float32(b._last_arc_ijk[2])
     assert fused_steps > 15
+
+
+@pytest.mark.parametrize("layout", [0, 1])
+@pytest.mark.parametrize("n_bins,own_raw", [(4096, True), (100, False)])
+def test_replaced_bins(hip_device, layout, n_bins, own_raw):
+    """As many radial bins as the entries take, and a grid whose bins a program has replaced by
+    more than ensure_lorentz_fields made (its second array is then too short, and the solve takes
+    the entries' kernels): solved as by the entries."""
+    from waam_solver_amd.field import DeviceField
+
+    twins = []
+    for _ in range(2):
+        g = _grid((24, 43, 9), layout, 7)
+        g.n_elec_bins = n_bins
+        g.elec_rad_bins = DeviceField.zeros((g.nz, n_bins), torch.float32, g.device)
+        if own_raw:
+            g.elec_bins_raw = DeviceField.zeros((g.nz, n_bins), torch.float32, g.device)
+        twins.append(g)
+    one, ref = twins
+    arc, dr = (12.3, 21.3, 4.9), 0.01
+    _by_entries(ref, arc, dr, 20, 1e-30, True)
+    K.lorentz_solve(one, arc, bin_dr_cells=dr, max_sweeps=20, tol=1e-30, cold=True, **SCALARS)
+    for n in ("phi_elec", "Jx", "Jy", "Jz", "elec_rad_bins", "Bx", "By", "Bz", "Fx", "Fy", "Fz"):
+        a, b = getattr(one, n).to_numpy(), getattr(ref, n).to_numpy()
+        assert np.array_equal(a, b), (n, float(np.abs(a - b).max()))

@@ -819,24 +819,32 @@ int check_lorentz(const char *who, const waam_lorentz &q)
 {
     WAAM_RETURN_IF(check_dims(who, q.nx, q.ny, q.nz, q.layout));
     WAAM_RETURN_IF(check_ptrs(who, {q.phi, q.phi_tmp, q.sigma, q.source, q.Jx, q.Jy, q.Jz, q.Bx,
-                                    q.By, q.Bz, q.bins, q.bins_raw, q.l1}));
+                                    q.By, q.Bz, q.bins, q.l1}));
     if (q.phi == q.phi_tmp || q.bins == q.bins_raw)
         return set_error(WAAM_ERR_INVALID, "%s: buffers alias", who);
     if (q.max_sweeps <= 0)
         return set_error(WAAM_ERR_INVALID, "%s: max_sweeps %d", who, q.max_sweeps);
-    /* k_elec_J_bins lists a cell of a slab with its bin in one word */
-    if ((int64_t)q.nx * q.ny > (int64_t)(0x7fffffff / kJBinGroup))
-        return set_error(WAAM_ERR_INVALID, "%s: slab of %d x %d cells", who, q.nx, q.ny);
     if (q.n_bins <= 0 || q.n_bins > kElecMaxBins || !(q.bin_dr > 0.0f))
         return set_error(WAAM_ERR_INVALID, "%s: bins", who);
     return WAAM_OK;
+}
+
+/* whether J, the bins, B and the force run in the kernels that take a slab piece by piece. They
+ * need x rows contiguous (in the XYZ layout a slab's cells lie a row apart and such a piece would
+ * read a line for every cell), the second array of bins and, since k_elec_J_bins lists a cell with
+ * its bin in one word, a slab of less than 2^29 cells. Every other solve takes the entries'
+ * kernels. */
+static bool by_slab(const waam_lorentz &q)
+{
+    return q.layout == kLayoutZYX && q.bins_raw &&
+           (int64_t)q.nx * q.ny <= (int64_t)(0x7fffffff / kJBinGroup);
 }
 
 int lorentz_run(const char *who, const waam_lorentz &q, const float *arc_k_dev, bool force,
                 waam_lorentz_result &out, hipStream_t st)
 {
     Dims d{q.nx, q.ny, q.nz, q.layout};
-    const bool zyx = q.layout == kLayoutZYX;
+    const bool zyx = q.layout == kLayoutZYX, slabs = by_slab(q);
     const size_t N = d.n();
     double *src_parts = reinterpret_cast<double *>((char *)q.scratch + kScratchPartials);
     double *l1_parts = reinterpret_cast<double *>((char *)q.scratch + kScratchTelemetryParts);
@@ -886,7 +894,7 @@ int lorentz_run(const char *who, const waam_lorentz &q, const float *arc_k_dev, 
     auto fields = [&](const ElecStatus *gate) {
         const dim3 bins_grid((unsigned)d.nz,
                              (unsigned)((q.n_bins + kJBinGroup - 1) / kJBinGroup));
-        if (zyx) {
+        if (slabs) {
             hipLaunchKernelGGL(k_elec_J_bins, bins_grid, dim3(kJBinThreads), 0, st, q.Jx, q.Jy,
                                q.Jz, q.bins_raw, in, q.sigma, q.flags, q.arc_i, q.arc_j, q.dx,
                                q.bin_dr, q.n_bins, gate, d);
@@ -900,8 +908,6 @@ int lorentz_run(const char *who, const waam_lorentz &q, const float *arc_k_dev, 
                 dim3(kBlock), 0, st, f, d);
             return;
         }
-        /* rows along z: a slab's cells lie a row apart, so the pieces by slab would read a line
-         * for every cell; the kernels that walk rows stay */
         hipLaunchKernelGGL(k_elec_J, grid3(d), block3(), 0, st, q.Jx, q.Jy, q.Jz, in, q.sigma,
                            q.flags, q.dx, d);
         hipLaunchKernelGGL(k_elec_bins,
@@ -931,13 +937,13 @@ int lorentz_run(const char *who, const waam_lorentz &q, const float *arc_k_dev, 
             sweep_chunk(n);
             launched += n;
         }
-        if (first && zyx) fields(status);
+        if (first && slabs) fields(status);
         WAAM_RETURN_IF(check_launch(who));
         hipError_t rc = hipMemcpyAsync(&h, status, sizeof(h), hipMemcpyDeviceToHost, st);
         if (rc == hipSuccess) rc = hipStreamSynchronize(st);
         if (rc != hipSuccess)
             return set_error(WAAM_ERR_HIP, "%s: %s", who, hipGetErrorString(rc));
-        if (!(first && zyx && h.done) && (h.done || launched >= q.max_sweeps)) fields(nullptr);
+        if (!(first && slabs && h.done) && (h.done || launched >= q.max_sweeps)) fields(nullptr);
         group = first ? 3 : 4;
     }
     out.res = h.res;

@@ -765,15 +765,19 @@ def lorentz_struct(g, arc, sigma_cells, current_A, sigma_liquid, sigma_solid, om
     """The waam_lorentz of a grid's fields."""
     _need(g.nx * g.ny * g.nz, g.phi_elec, g.phi_elec_tmp, g.sigma_elec, g.elec_source, g.Jx, g.Jy,
           g.Jz, g.Bx, g.By, g.Bz, g.Fx, g.Fy, g.Fz, g.Fx_snap, g.Fy_snap, g.Fz_snap, g.f_l, g.flags)
-    if min(_n(g.elec_rad_bins), _n(g.elec_bins_raw)) < g.nz * g.n_elec_bins:
+    if _n(g.elec_rad_bins) < g.nz * g.n_elec_bins:
         raise ValueError("bins must hold nz x n_bins values")
+    # a second array that is not there, or too short for the bins, is not used
+    raw = getattr(g, "elec_bins_raw", None)
+    if raw is not None and _n(raw) < g.nz * g.n_elec_bins:
+        raw = None
     return LorentzC(
         P(g.phi_elec), P(g.phi_elec_tmp), P(g.sigma_elec), P(g.elec_source), P(g.Jx), P(g.Jy),
-        P(g.Jz), P(g.Bx), P(g.By), P(g.Bz), P(g.elec_rad_bins), P(g.elec_bins_raw),
+        P(g.Jz), P(g.Bx), P(g.By), P(g.Bz), P(g.elec_rad_bins), P(raw),
         P(g.elec_l1_buf), P(g.Fx), P(g.Fy), P(g.Fz), P(g.Fx_snap), P(g.Fy_snap), P(g.Fz_snap),
-        P(g.f_l), P(g.flags), P(g.scratch), None, float(tol), arc[0], arc[1], arc[2], sigma_cells, current_A, g.dx, sigma_liquid,
-        sigma_solid, omega_j, bin_dr_cells, mu0, g.dt, rho_ref, int(nz_solid),
-        int(g.n_elec_bins), int(cold), int(max_sweeps), g.nx, g.ny, g.nz, layout_of(g.phi_elec))
+        P(g.f_l), P(g.flags), P(g.scratch), None, float(tol), arc[0], arc[1], arc[2], sigma_cells,
+        current_A, g.dx, sigma_liquid, sigma_solid, omega_j, bin_dr_cells, mu0, g.dt, rho_ref,
+        int(nz_solid), int(g.n_elec_bins), int(cold), int(max_sweeps), g.nx, g.ny, g.nz, layout_of(g.phi_elec))
 
 
 def lorentz_done(g, r: LorentzResultC) -> LorentzResultC:
