@@ -132,10 +132,9 @@ def apply_gas_shear(twin, g, arc_i: float, arc_j: float, arc_k: float) -> None:
 
 def lorentz_args(twin, g, arc_i: float, arc_j: float, arc_k: float) -> dict:
     """Arguments of ``kernels.lorentz_struct`` for this step's solve (the first one of a run
-    starts cold and may take 2 n_max^2 sweeps)."""
+    starts cold and may take 2 n_max^2 sweeps; ``note_lorentz`` takes note that it has run)."""
     g.ensure_lorentz_fields()
     cold_start = not getattr(twin, "_lorentz_warm", False)
-    twin._lorentz_warm = True
     max_iters = max(int(twin.lorentz_jacobi_iters), 20)
     if cold_start:
         n_max = max(g.nx, g.ny, g.nz)
@@ -149,7 +148,8 @@ def lorentz_args(twin, g, arc_i: float, arc_j: float, arc_k: float) -> dict:
 
 
 def note_lorentz(twin, r, args: dict) -> None:
-    """Count a solve that did not converge."""
+    """After a solve: the next one starts from its potential; count one that did not converge."""
+    twin._lorentz_warm = True
     if r.converged:
         twin._lorentz_unconverged_streak = 0
         return
