@@ -72,7 +72,10 @@ def _by_entries(g, arc, dr, max_sweeps, tol, cold):
     ((24, 43, 9), 60, 6e-2, True),     # converges on the way
     ((80, 40, 30), 41, 1e-30, True),   # more than one read by the host
     ((131, 67, 25), 23, 1e30, True),
-    ((96, 96, 73), 22, 1e-30, False),  # more tiles than blocks
+    ((96, 96, 73), 22, 1e-30, False),  # single sweeps, a last chunk of two
+    ((64, 64, 32), 41, 1e-30, False),  # as many tiles as are swept in LDS
+    ((65, 64, 32), 41, 1e-30, False),  # a row of them more
+    ((65, 64, 32), 60, 2e-1, True),    # converges on the way, read chunk by chunk
 ])
 def test_solve_equals_its_entries(hip_device, layout, dims, max_sweeps, tol, cold):
     one, ref = _grid(dims, layout, 7), _grid(dims, layout, 7)

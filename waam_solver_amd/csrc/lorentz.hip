@@ -12,7 +12,7 @@
 // waam_lorentz_solve runs the same solve as a whole: entry by entry a warm solve took 23 to 63
 // launches, each waiting for the one before on a grid that it covers in less than its own latency,
 // with a read by the host after every tenth sweep. Its kernels cover several of these each (source
-// and its total, sweeps in LDS tiles, J with the radial bins, prefix with B and the force), and
+// and its total, on grids of up to 256 tiles the sweeps in LDS, J with the radial bins, prefix with B and the force), and
 // the convergence test is taken on the device: a solve that converges in its first chunk of ten
 // is seven launches and one read, with the same values bit for bit. In the fused step
 // (waam_step_fused_lorentz) a step of 80x40x30 takes 173 us, 615 to 660 through the entries.
@@ -454,13 +454,27 @@ struct ElecSweep {
 constexpr int kSweepTile = 8;
 constexpr int kSweepThreads = 1024;
 constexpr int kSweepMax = 5;  // sweeps a launch can take
+/* Grids of up to this many tiles take their sweeps in tiles: one for each of the 256 CUs, since a
+ * workgroup's LDS leaves no room for a second. From there on a chunk's two launches take as many
+ * rounds of 12 us as there are tiles for a CU, and single sweeps, bound by their 4 us launches up
+ * to about 300 k cells and by memory above, are the shorter: a step of 80x40x30 (200 tiles) takes
+ * 193 us in tiles and 207 sweep by sweep (XYZ layout 225, 234), 80x64x32 (320) 217 and 204 (247,
+ * 241), 128x64x40 (640) 241 and 199 (295, 280), 160x80x60 (1600) 328 and 230 (430, 372);
+ * 400x200x100 took 2390 in tiles and 1610 entry by entry. */
+constexpr int kTiledSweepTiles = 256;
+
+static int64_t sweep_tiles(const Dims &d)
+{
+    constexpr int T = kSweepTile;
+    return (int64_t)((d.nx + T - 1) / T) * ((d.ny + T - 1) / T) * ((d.nz + T - 1) / T);
+}
 
 /* Up to five Jacobi sweeps (k_elec_jacobi, the same sums in the same order) of an 8^3 tile in LDS:
  * the tile is loaded with a margin of five cells and each sweep computes what the ones after it
  * still need, the last one the tile itself. That is 3.9 updates for one, and still less than the
- * launches it replaces: 80x40x30 (200 tiles, one block a CU) 12.4 us for five sweeps, against
- * five dependent launches at 4.5 us and more each. A thread keeps its four cells of the 16^3 that
- * the first sweep computes, so that conductivities, their sum, the source and the neighbours'
+ * launches it replaces while each tile has a CU: 80x40x30 (200 tiles) 12.4 us for five sweeps,
+ * against five dependent launches at 4.5 us and more each. A thread keeps its four cells of the
+ * 16^3 that the first sweep computes, so that conductivities, their sum, the source and the neighbours'
  * places are found once and a sweep is seven LDS reads and the arithmetic (all found again in
  * each sweep: 13.8 us). The L1 sums are those of the last sweep. */
 template <bool ZYX>
@@ -473,115 +487,113 @@ __global__ void __launch_bounds__(kSweepThreads) k_elec_sweeps(ElecSweep e, Dims
     __shared__ double sh_s[kSweepThreads], sh_c[kSweepThreads];
     const int tid = (int)threadIdx.x;
     const int nf = d.fast(), ns = d.slow();
-    const int tf = (nf + T - 1) / T, tj = (d.ny + T - 1) / T, ts = (ns + T - 1) / T;
-    const int64_t ntiles = (int64_t)tf * tj * ts;
+    const int tf = (nf + T - 1) / T, tj = (d.ny + T - 1) / T;
     const bool done = e.status->done != 0;
     if (done && !e.copy) return;
     const int x = tid % I, y = (tid / I) % I, z0 = tid / (I * I);
     const int first = M - e.sweeps + 1;  // sweep m leaves a margin of M - m around the tile
     double s0 = 0.0, c0 = 0.0, s1 = 0.0, c1 = 0.0;
-    for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const int a0 = (int)(tile % tf) * T - M, b0 = (int)((tile / tf) % tj) * T - M,
-                  g0 = (int)(tile / ((int64_t)tf * tj)) * T - M;
-        float *in0 = s_phi[first & 1];
-        /* every load of the tile is under way before the first is waited for (a place outside the
-         * domain loads a cell of its face, which no sweep reads): a load per pass of a loop with
-         * the test inside took a trip to memory per pass, ten trips of 0.8 us */
-        constexpr int L = (W3 + kSweepThreads - 1) / kSweepThreads;
-        float v_in[L], v_sig[L], src[C];
-        uint8_t fl[C];
+    const int tile = (int)blockIdx.x;  // a workgroup each
+    const int a0 = (tile % tf) * T - M, b0 = ((tile / tf) % tj) * T - M,
+              g0 = (tile / (tf * tj)) * T - M;
+    float *in0 = s_phi[first & 1];
+    /* every load of the tile is under way before the first is waited for (a place outside the
+     * domain loads a cell of its face, which no sweep reads): a load per pass of a loop with
+     * the test inside took a trip to memory per pass, ten trips of 0.8 us */
+    constexpr int L = (W3 + kSweepThreads - 1) / kSweepThreads;
+    float v_in[L], v_sig[L], src[C];
+    uint8_t fl[C];
 #pragma unroll
-        for (int n = 0; n < L; ++n) {
-            const int l = imin(tid + n * kSweepThreads, W3 - 1);
-            const int a = imax(0, imin(a0 + l % W, nf - 1));
-            const int j = imax(0, imin(b0 + (l / W) % W, d.ny - 1));
-            const int b = imax(0, imin(g0 + l / (W * W), ns - 1));
-            const size_t c = ((size_t)b * d.ny + j) * nf + a;
-            v_in[n] = e.in[c];
-            v_sig[n] = e.sigma[c];
-        }
-        const int a = a0 + x + 1, j = b0 + y + 1;
-        const bool col = a >= 0 && a < nf && j >= 0 && j < d.ny;
+    for (int n = 0; n < L; ++n) {
+        const int l = imin(tid + n * kSweepThreads, W3 - 1);
+        const int a = imax(0, imin(a0 + l % W, nf - 1));
+        const int j = imax(0, imin(b0 + (l / W) % W, d.ny - 1));
+        const int b = imax(0, imin(g0 + l / (W * W), ns - 1));
+        const size_t c = ((size_t)b * d.ny + j) * nf + a;
+        v_in[n] = e.in[c];
+        v_sig[n] = e.sigma[c];
+    }
+    const int a = a0 + x + 1, j = b0 + y + 1;
+    const bool col = a >= 0 && a < nf && j >= 0 && j < d.ny;
 #pragma unroll
-        for (int n = 0; n < C; ++n) {
-            const int b = imax(0, imin(g0 + z0 + n * P + 1, ns - 1));
-            const size_t c = ((size_t)b * d.ny + imax(0, imin(j, d.ny - 1))) * nf +
-                             imax(0, imin(a, nf - 1));
-            fl[n] = e.flags[c];
-            src[n] = e.source[c];
-        }
+    for (int n = 0; n < C; ++n) {
+        const int b = imax(0, imin(g0 + z0 + n * P + 1, ns - 1));
+        const size_t c = ((size_t)b * d.ny + imax(0, imin(j, d.ny - 1))) * nf +
+                         imax(0, imin(a, nf - 1));
+        fl[n] = e.flags[c];
+        src[n] = e.source[c];
+    }
 #pragma unroll
-        for (int n = 0; n < L; ++n) {
-            const int l = tid + n * kSweepThreads;
-            if (l >= W3) break;
-            in0[l] = v_in[n];
-            s_sig[l] = v_sig[n];
-        }
-        bool zero[C];
+    for (int n = 0; n < L; ++n) {
+        const int l = tid + n * kSweepThreads;
+        if (l >= W3) break;
+        in0[l] = v_in[n];
+        s_sig[l] = v_sig[n];
+    }
+    bool zero[C];
 #pragma unroll
-        for (int n = 0; n < C; ++n) {
-            const int b = g0 + z0 + n * P + 1;
-            zero[n] = fl[n] == GAS || ((ZYX ? b : a) <= e.nz_solid && fl[n] == SOLID);
-            src[n] = src[n] * e.dx * e.dx;
-        }
-        __syncthreads();
-        /* the neighbours' places (the cell's own at the domain's faces) and conductivities */
-        const int ap = a + 1 < nf ? 1 : 0, am = a > 0 ? -1 : 0;
-        const int jp = j + 1 < d.ny ? W : 0, jm = j > 0 ? -W : 0;
-        int bp[C], bm[C];
-        float sp[C], sm[C], sn[C], ss[C], st[C], sb[C], denom[C];
+    for (int n = 0; n < C; ++n) {
+        const int b = g0 + z0 + n * P + 1;
+        zero[n] = fl[n] == GAS || ((ZYX ? b : a) <= e.nz_solid && fl[n] == SOLID);
+        src[n] = src[n] * e.dx * e.dx;
+    }
+    __syncthreads();
+    /* the neighbours' places (the cell's own at the domain's faces) and conductivities */
+    const int ap = a + 1 < nf ? 1 : 0, am = a > 0 ? -1 : 0;
+    const int jp = j + 1 < d.ny ? W : 0, jm = j > 0 ? -W : 0;
+    int bp[C], bm[C];
+    float sp[C], sm[C], sn[C], ss[C], st[C], sb[C], denom[C];
 #pragma unroll
-        for (int n = 0; n < C; ++n) {
-            const int zl = z0 + n * P, b = g0 + zl + 1;
-            const int l = ((zl + 1) * W + y + 1) * W + x + 1;
-            bp[n] = b + 1 < ns ? W * W : 0;
-            bm[n] = b > 0 ? -W * W : 0;
-            sp[n] = s_sig[l + (ZYX ? ap : bp[n])];
-            sm[n] = s_sig[l + (ZYX ? am : bm[n])];
-            sn[n] = s_sig[l + jp];
-            ss[n] = s_sig[l + jm];
-            st[n] = s_sig[l + (ZYX ? bp[n] : ap)];
-            sb[n] = s_sig[l + (ZYX ? bm[n] : am)];
-            const float eps = 1e-12f;
-            denom[n] = sp[n] + sm[n] + sn[n] + ss[n] + st[n] + sb[n] + eps;
-        }
-        for (int m = first; m <= M; ++m) {
-            const float *pin = s_phi[m & 1];
-            float *pout = s_phi[(m + 1) & 1];
-            const int lo = m - 1, hi = I - m;  // of the cells this sweep computes
-            if (col && x >= lo && x <= hi && y >= lo && y <= hi) {
+    for (int n = 0; n < C; ++n) {
+        const int zl = z0 + n * P, b = g0 + zl + 1;
+        const int l = ((zl + 1) * W + y + 1) * W + x + 1;
+        bp[n] = b + 1 < ns ? W * W : 0;
+        bm[n] = b > 0 ? -W * W : 0;
+        sp[n] = s_sig[l + (ZYX ? ap : bp[n])];
+        sm[n] = s_sig[l + (ZYX ? am : bm[n])];
+        sn[n] = s_sig[l + jp];
+        ss[n] = s_sig[l + jm];
+        st[n] = s_sig[l + (ZYX ? bp[n] : ap)];
+        sb[n] = s_sig[l + (ZYX ? bm[n] : am)];
+        const float eps = 1e-12f;
+        denom[n] = sp[n] + sm[n] + sn[n] + ss[n] + st[n] + sb[n] + eps;
+    }
+    for (int m = first; m <= M; ++m) {
+        const float *pin = s_phi[m & 1];
+        float *pout = s_phi[(m + 1) & 1];
+        const int lo = m - 1, hi = I - m;  // of the cells this sweep computes
+        if (col && x >= lo && x <= hi && y >= lo && y <= hi) {
 #pragma unroll
-                for (int n = 0; n < C; ++n) {
-                    const int zl = z0 + n * P, b = g0 + zl + 1;
-                    if (zl < lo || zl > hi || b < 0 || b >= ns) continue;
-                    const int l = ((zl + 1) * W + y + 1) * W + x + 1;
-                    const float *q = pin + l;
-                    const float old = q[0];
-                    float pn = sp[n] * q[ZYX ? ap : bp[n]] + sm[n] * q[ZYX ? am : bm[n]] +
-                               sn[n] * q[jp] + ss[n] * q[jm] + st[n] * q[ZYX ? bp[n] : ap] +
-                               sb[n] * q[ZYX ? bm[n] : am];
-                    float phi_new = (pn + src[n]) / denom[n];
-                    float now = (1.0f - e.omega) * old + e.omega * phi_new;
-                    if (zero[n]) now = 0.0f;
-                    if (m < M) {
-                        pout[l] = now;
-                        continue;
-                    }
-                    if (done) now = old;
-                    e.out[((size_t)b * d.ny + j) * nf + a] = now;
-                    if (e.parts) {
-                        double sum, er;
-                        two_sum(s0, (double)fabsf(now - old), sum, er);
-                        s0 = sum;
-                        c0 += er;
-                        two_sum(s1, (double)fabsf(old), sum, er);
-                        s1 = sum;
-                        c1 += er;
-                    }
+            for (int n = 0; n < C; ++n) {
+                const int zl = z0 + n * P, b = g0 + zl + 1;
+                if (zl < lo || zl > hi || b < 0 || b >= ns) continue;
+                const int l = ((zl + 1) * W + y + 1) * W + x + 1;
+                const float *q = pin + l;
+                const float old = q[0];
+                float pn = sp[n] * q[ZYX ? ap : bp[n]] + sm[n] * q[ZYX ? am : bm[n]] +
+                           sn[n] * q[jp] + ss[n] * q[jm] + st[n] * q[ZYX ? bp[n] : ap] +
+                           sb[n] * q[ZYX ? bm[n] : am];
+                float phi_new = (pn + src[n]) / denom[n];
+                float now = (1.0f - e.omega) * old + e.omega * phi_new;
+                if (zero[n]) now = 0.0f;
+                if (m < M) {
+                    pout[l] = now;
+                    continue;
+                }
+                if (done) now = old;
+                e.out[((size_t)b * d.ny + j) * nf + a] = now;
+                if (e.parts) {
+                    double sum, er;
+                    two_sum(s0, (double)fabsf(now - old), sum, er);
+                    s0 = sum;
+                    c0 += er;
+                    two_sum(s1, (double)fabsf(old), sum, er);
+                    s1 = sum;
+                    c1 += er;
                 }
             }
-            __syncthreads();
         }
+        __syncthreads();
     }
     if (!e.parts || done) return;
     block_reduce_pair(s0, c0, sh_s, sh_c);
@@ -859,12 +871,11 @@ int lorentz_run(const char *who, const waam_lorentz &q, const float *arc_k_dev, 
     float *in = q.phi, *other = q.phi_tmp;
     if (q.cold)
         hipLaunchKernelGGL(k_fill, dim3(grid_for(N)), dim3(kBlock), 0, st, in, 0.0f, N);
-    const int T = kSweepTile;
-    const int64_t tiles = (int64_t)((d.nx + T - 1) / T) * ((d.ny + T - 1) / T) *
-                          ((d.nz + T - 1) / T);
-    const int blocks = (int)(tiles < kReduceBlocks ? tiles : kReduceBlocks);
+    const int64_t tiles = sweep_tiles(d);
+    const bool tiled = tiles <= kTiledSweepTiles;
+    const int blocks = tiled ? (int)tiles : kLorentzSumBlocks;  // that leave L1 sums
 
-    auto sweep_chunk = [&](int n) {
+    auto sweeps = [&](int n) {
         for (int first = 1, m = n; m > 0; first = 0) {
             const int now = first ? (m + 1) / 2 : m;
             m -= now;
@@ -888,6 +899,19 @@ int lorentz_run(const char *who, const waam_lorentz &q, const float *arc_k_dev, 
                                    sw, d);
             std::swap(in, other);
         }
+    };
+    auto single_sweeps = [&](int n) {
+        for (int m = n; m > 0; --m) {
+            hipLaunchKernelGGL(k_elec_jacobi, grid3(d), block3(), 0, st, in, other, q.sigma,
+                               q.source, q.flags, q.dx, q.omega, q.nz_solid, d);
+            std::swap(in, other);
+        }
+        hipLaunchKernelGGL(k_elec_l1, dim3(blocks), dim3(kBlock), 0, st, (const float *)in,
+                           (const float *)other, l1_parts, N);
+    };
+    auto sweep_chunk = [&](int n) {
+        if (tiled) sweeps(n);
+        else single_sweeps(n);
         hipLaunchKernelGGL(k_elec_check, dim3(1), dim3(kBlock), 0, st, l1_parts, blocks, n, q.tol,
                            q.l1, status);
     };
@@ -927,7 +951,8 @@ int lorentz_run(const char *who, const waam_lorentz &q, const float *arc_k_dev, 
     /* A warm solve mostly converges in its first chunk: that one is read by itself, with the field
      * kernels queued behind it (they run only if it did). One that does not is likely to take the
      * rest of a usual limit of 40 sweeps: the chunks after it go out in groups, and a group whose
-     * early chunks converge leaves launches that end at once. */
+     * early chunks converge leaves launches that end at once. Single sweeps are read chunk by
+     * chunk: they do not look at the test. */
     ElecStatus h{};
     int launched = 0, group = 1;
     while (launched < q.max_sweeps && !h.done) {
@@ -944,7 +969,7 @@ int lorentz_run(const char *who, const waam_lorentz &q, const float *arc_k_dev, 
         if (rc != hipSuccess)
             return set_error(WAAM_ERR_HIP, "%s: %s", who, hipGetErrorString(rc));
         if (!(first && slabs && h.done) && (h.done || launched >= q.max_sweeps)) fields(nullptr);
-        group = first ? 3 : 4;
+        group = !tiled ? 1 : (first ? 3 : 4);
     }
     out.res = h.res;
     out.norm = h.norm;
