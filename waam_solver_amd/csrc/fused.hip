@@ -2874,23 +2874,31 @@ static void launch_k(bool capture, void (*k)(KArgs...), dim3 grid, dim3 block, h
  * device holds at once, or a quarter of them, were slower on 301x157x83: 34 us against 31) */
 constexpr int kSteadySurfaceBlocks = 512;
 constexpr int kSteadyWalkBlocks = 512;
-/* Steady steps on grids whose plate march has up to this many blocks (by the grid's x and y
- * extents, in either layout) run kernels 2, 2p and 3 in one launch.
- * Beside the surface cells' registers (five wavefronts a SIMD instead of seven) a larger plate
- * loses more than the overlap gives: the 3456 blocks of 768x384x192 take 147 us together and
- * 73 + 18 + 41 apart; the 1536 of 512x256x128 52 and 31 + 12 + 15, the 600 of 301x157x83 31 and
- * 19 + 9 + 18, the 30 of 64x40x32 16 and 8 + 7 + 15. */
+/* Which steady steps run kernels 2, 2p and 3 in one launch. Beside the surface cells' registers (five
+ * wavefronts a SIMD instead of seven) the sweeps lose more than the overlap gives once they fill the
+ * chip by themselves. With a plate march (ZYX, constant material) its blocks count, by the grid's x
+ * and y extents: the 3456 blocks of 768x384x192 take 147 us together and 73 + 18 + 41 apart; the
+ * 1536 of 512x256x128 52 and 31 + 12 + 15, the 600 of 301x157x83 31 and 19 + 9 + 18, the 30 of
+ * 64x40x32 16 and 8 + 7 + 15. */
 constexpr int kTogetherBlocks = 2048;
-/* With the tables there is no plate march, so the walk has the plate's segments too and fills the
- * chip sooner: up to this many row segments together (a step of 200x100x62, 24800 of them, 94 us
- * together and 105 apart; 256x128x64, 32768, 107 and 115; 320x160x72, 57600, 137 and 136;
- * 400x200x100, 140000, 223 and 203). */
+/* Elsewhere the walk has the plate's segments too and fills the chip sooner: the row segments count.
+ * us a step together and apart:
+ * tables, ZYX: 200x100x62, 24800 segments, 94 and 105; 256x128x64, 32768, 107 and 115; 320x160x72,
+ * 57600, 137 and 136; 400x200x100, 140000, 223 and 203;
+ * tables, XYZ: 128x96x64, 12288, 156 and 165; 160x80x64, 12800, 165 and 169; 200x100x62, 20000, 246
+ * and 243; 256x128x64, 32768, 368 and 350;
+ * constants, XYZ: 96x64x48, 6144, 99 and 107; 128x64x64, 8192, 118 and 122; 128x96x64, 12288, 147 and
+ * 147; 160x80x64, 12800, 154 and 151; 256x128x64, 32768, 340 and 312; 301x157x83, 94514, 816 and
+ * 693. */
 constexpr size_t kTogetherTableSegments = 40960;
+constexpr size_t kTogetherTableSegmentsXYZ = 16384;
+constexpr size_t kTogetherSegmentsXYZ = 10240;
 static bool thermal_together(const Dims &d, bool tab)
 {
+    if (d.layout == kLayoutXYZ)
+        return quiet_segments(d) <= (tab ? kTogetherTableSegmentsXYZ : kTogetherSegmentsXYZ);
     if (tab) return quiet_segments(d) <= kTogetherTableSegments;
-    return (d.nx + kTileFast - 1) / kTileFast * plate_row_blocks(d) * kPlateChunks <=
-           kTogetherBlocks;
+    return plate_blocks(d) <= kTogetherBlocks;
 }
 
 /* The step's launches in order: kernels 1 to 4 here, 5 to 7 in launch_flow. A steady step
