@@ -427,18 +427,19 @@ __device__ __forceinline__ bool segment_active(const QuietRec &q, int bx, int j,
  * neighbouring segment along the row pulls (the last cell for a direction of positive e_x, the
  * first for a negative one). A segment that holds a collided cell, or
  * whose stream flags differ from those two steps before, counts as changed in every direction
- * (kPullFull, set by kernel 7, which pulls the latter whole as well). A step that is not steady
- * leaves every word unknown (kPullUnknown): the next steady step pulls every segment and calls
+ * (kPullFull, set by kernel 4, which lists the latter whole as well). A step that is not steady
+ * keeps no words and only says so (`unknown`): the next steady step pulls every segment and calls
  * every one changed, since the destination it compares with may not be a pull of A(n-1)'s
- * predecessor; the one after pulls every segment and compares. The buffer at the lower address
+ * predecessor; the one after pulls every segment and compares. (Such a step once left a mark in
+ * every segment's four words: kernel 7 of 512x256x128 76 -> 87 us.) The buffer at the lower address
  * owns the first pair of words. */
 constexpr uint32_t kPullDirs = (1u << Q) - 1u;
 constexpr uint32_t kPullFull = 0x7fffffffu;  // bit 30: pull the segment itself whole as well
-constexpr uint32_t kPullUnknown = 0xffffffffu;
 
 struct PullRec {
     uint32_t *chg_src, *edge_src, *chg_dst, *edge_dst;
     int *count, *last, *next;  // as the segment list's
+    int *unknown;              // the step before kept no change words
     uint2 *list;               // (segment, directions)
 };
 
@@ -452,6 +453,7 @@ __device__ __forceinline__ PullRec pull_rec(const waam_step_fields &f, const Dim
     r.last = reinterpret_cast<int *>(base);
     r.count = r.last + 4 + p;
     r.next = r.last + 4 + (p ^ 1);
+    r.unknown = r.last + 8;
     r.chg_src = w + (p ? 2 : 0) * nseg;
     r.edge_src = r.chg_src + nseg;
     r.chg_dst = w + (p ? 0 : 2) * nseg;
@@ -571,6 +573,7 @@ __device__ __forceinline__ void quiet_list_quad(const waam_step_fields &f, const
     constexpr uint32_t kOnes = 0x01010101u;
     uint32_t sg[4], dirs[4] = {0u, 0u, 0u, 0u};
     bool act[4] = {false, false, false, false};
+    const bool unknown = *r.unknown != 0;
     if (s0 < nseg) {
         const int bx = (int)(s0 % (size_t)q.nbx);
         const size_t rowi = s0 / (size_t)q.nbx;
@@ -617,15 +620,14 @@ __device__ __forceinline__ void quiet_list_quad(const waam_step_fields &f, const
                 for (int v = 0; v < 4; ++v) dirs[v] |= (e[v] & up) | (e[v + 2] & dn);
             }
         }
-        uint32_t fresh[4];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
             sg[v] = (uint32_t)s0 + (uint32_t)v;
             act[v] = ((idle >> (8 * v)) & 1u) == 0u;
-            if ((ownc[v] & ~kPullDirs) != 0u) dirs[v] = kPullDirs;
-            fresh[v] = ownc[v] == kPullUnknown ? kPullFull : 0u;
+            if (unknown || (ownc[v] & ~kPullDirs) != 0u) dirs[v] = kPullDirs;
         }
-        const uint4 f4 = make_uint4(fresh[0], fresh[1], fresh[2], fresh[3]);
+        const uint32_t fresh = unknown ? kPullFull : 0u;
+        const uint4 f4 = make_uint4(fresh, fresh, fresh, fresh);
         *reinterpret_cast<uint4 *>(r.chg_dst + s0) = f4;
         *reinterpret_cast<uint4 *>(r.edge_dst + s0) = f4;
     }
@@ -657,8 +659,10 @@ __device__ __forceinline__ void quiet_list(const waam_step_fields &f, const Step
     if (sg < nseg && pulls_by_record(d)) {
         const int bx = (int)(sg % (size_t)q.nbx);
         const size_t row = sg / (size_t)q.nbx;
+        const bool unknown = *r.unknown != 0;
         dirs = pull_dirs(r, q, bx, (int)(row % (size_t)d.ny), (int)(row / (size_t)d.ny), d);
-        const uint32_t fresh = r.chg_src[sg] == kPullUnknown ? kPullFull : 0u;
+        if (unknown) dirs = kPullDirs;
+        const uint32_t fresh = unknown ? kPullFull : 0u;
         r.chg_dst[sg] = fresh;
         r.edge_dst[sg] = fresh;
     }
@@ -747,19 +751,13 @@ __device__ __forceinline__ void record_quiet(const QuietRec &q, size_t seg, bool
     }
 }
 
-/* kernel 7, one thread: the next step's counters start empty */
-__device__ __forceinline__ void empty_next_lists(const QuietRec &q, const PullRec &r)
+/* kernel 7, one thread: the next step's counters start empty, and the next step learns whether this
+ * one kept the pull's change words (a steady one does) */
+__device__ __forceinline__ void leave_lists(const QuietRec &q, const PullRec &r, bool steady)
 {
     q.next[0] = q.next[2] = 0;
     r.next[0] = 0;
-}
-
-/* a step that is not steady leaves the pull's record unknown for both buffers */
-__device__ __forceinline__ void forget_pull(const PullRec &r, size_t seg)
-{
-    if (threadIdx.x != 0) return;
-    r.chg_src[seg] = r.edge_src[seg] = kPullUnknown;
-    r.chg_dst[seg] = r.edge_dst[seg] = kPullUnknown;
+    *r.unknown = steady ? 0 : 1;
 }
 
 /* below the solidus and both HAZ thresholds: no freeze rule and no HAZ clock acts on the cell */
@@ -2144,7 +2142,7 @@ __global__ void __launch_bounds__(256) k_step_stream(waam_step_fields f, StepCon
     const QuietRec q = quiet_rec(f, d);
     if (blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && threadIdx.x == 0 &&
         threadIdx.y == 0)
-        empty_next_lists(q, pull_rec(f, d));
+        leave_lists(q, pull_rec(f, d), false);
     int i, j, k;
     if (PULL) {
         const bool in = d.cell(i, j, k);
@@ -2153,7 +2151,6 @@ __global__ void __launch_bounds__(256) k_step_stream(waam_step_fields f, StepCon
         if (in) quiet = stream_cell<E, true>(f, s, i, j, k);
         const size_t seg = seg_index(q, (int)blockIdx.x, j, (int)blockIdx.z, d);
         record_quiet(q, seg, quiet, false, false);
-        forget_pull(pull_rec(f, d), seg);
         return;
     }
     const int a = (int)(blockIdx.x * blockDim.x + threadIdx.x);
@@ -2190,7 +2187,6 @@ __global__ void __launch_bounds__(256) k_step_stream(waam_step_fields f, StepCon
                                      phi[t], fl[t]);
         const size_t seg = seg_index(q, (int)blockIdx.x, j, b, d);
         record_quiet(q, seg, quiet, false, false);
-        forget_pull(pull_rec(f, d), seg);
     }
 }
 
@@ -2205,7 +2201,7 @@ __global__ void __launch_bounds__(256) k_step_stream_seg(waam_step_fields f, Ste
         const PullRec r = pull_rec(f, d);
         *q.last = *q.count;
         *r.last = *r.count;
-        empty_next_lists(q, r);
+        leave_lists(q, r, true);
     }
     for_needed_segments(q, d, [&](size_t seg) {
         int i, j, k;
