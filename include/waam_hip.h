@@ -573,6 +573,8 @@ int waam_compute_vorticity_magnitude(const float *ux, const float *uy, const flo
  * physics/force_diagnostics.py:19-24) */
 int waam_max_norm3(const float *fx, const float *fy, const float *fz, float *out, int64_t n,
                    void *stream);
+/* y[e] = the exponential every kernel evaluates (waam_math.h, device form) of x[e] */
+int waam_expf_array(const float *x, float *y, int64_t n, void *stream);
 /* ProbeRecorder.record_step export/probes.py:95-113: out[2p], out[2p+1] = T, f_l at linear cell
  * cells[p] (in the fields' layout); a negative entry (probe outside the window) gives NaN. The
  * caller points out at a row of a device ring of samples and reads the ring back in one copy. */

@@ -129,6 +129,7 @@ SIGNATURES: dict[str, str] = {
     "waam_step_fused_lorentz": "ppppp",
     "waam_compute_vorticity_magnitude": "pppppffiiiip",
     "waam_max_norm3": "pppplp",
+    "waam_expf_array": "pplp",
     "waam_probe_gather": "pppilpp",
     "waam_cavity_step": "pppppppfffffiiiip",
     "waam_adj_arc_sums": "ppppiiiipp",

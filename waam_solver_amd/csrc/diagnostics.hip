@@ -1,7 +1,7 @@
 // diagnostics.hip — export-side fields and reductions: vorticity magnitude (reference
 // kernels.py:3380-3419, compute_vorticity_magnitude) and the max-norm of a vector field (the
 // reference physics/force_diagnostics.py:19-24 reads the three force fields back to the host
-// for it; here one device reduction leaves one float).
+// for it; here one device reduction leaves one float), and the kernels' exponential on an array.
 #include "waam_common.h"
 
 namespace waam {
@@ -72,6 +72,12 @@ __global__ void k_probe_gather(const float *__restrict__ T, const float *__restr
     out[2 * p + 1] = in ? fl[c] : __int_as_float(0x7fc00000);
 }
 
+__global__ void k_expf(const float *__restrict__ x, float *__restrict__ y, size_t n)
+{
+    const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e < n) y[e] = waam_expf(x[e]);
+}
+
 }  // namespace waam
 
 using namespace waam;
@@ -115,6 +121,15 @@ int waam_probe_gather(const float *T, const float *f_l, const int64_t *cells, in
     hipLaunchKernelGGL(k_probe_gather, dim3((unsigned)((n_probes + 63) / 64)), dim3(64), 0,
                        as_stream(stream), T, f_l, cells, n_probes, (size_t)n_cells, out);
     return check_launch("waam_probe_gather");
+}
+
+int waam_expf_array(const float *x, float *y, int64_t n, void *stream)
+{
+    if (n <= 0) return set_error(WAAM_ERR_INVALID, "waam_expf_array: n <= 0");
+    WAAM_RETURN_IF(check_ptrs("waam_expf_array", {x, y}));
+    hipLaunchKernelGGL(k_expf, dim3(grid_for((size_t)n)), dim3(kBlock), 0, as_stream(stream), x, y,
+                       (size_t)n);
+    return check_launch("waam_expf_array");
 }
 
 }  // extern "C"
