@@ -30,6 +30,14 @@ def _pulled(tw) -> tuple[int, int]:
     return int(rec[off:off + 4].view(np.int32)[0]), nseg
 
 
+def _bits(tw, bx: int, rows, k: int) -> list[int]:
+    """The record bytes of segment bx of the rows j in slice k (rows along x)."""
+    g = tw.grid
+    nbx = -(-g.nx // 64)
+    rec = g.quiet.to_numpy().view(np.uint8)
+    return [int(rec[(k * g.ny + j) * nbx + bx]) for j in rows]
+
+
 @pytest.mark.parametrize("nx,ny,nz,layout,pop", [
     (64, 40, 32, 1, "fp32"),     # one whole segment a row: it wraps onto itself
     (65, 24, 24, 1, "fp32"),     # the second segment is one cell: both its ends
@@ -65,10 +73,25 @@ def test_still_populations_are_left_alone(hip_device, nx, ny, nz, layout, pop):
         for f in ("f_src", "f_dst"):
             a, b = getattr(g, f).to_numpy(), getattr(ref.grid, f).to_numpy()
             assert bits_equal(a, b), f"step {done}: {mismatch_report(f, a, b)}"
-        if write:  # hot gas populations and a warm cell, as a host program may set them
+        if layout == 1:
+            # the warmed cell's row segments: cold plate before, not for some steps after, then again
+            bits = _bits(tw, nx // 2 // 64, (1, 2), 1)
+            print(f"[still] step {done}: record of the warmed rows {bits}", flush=True)
+            if done == 40:
+                assert all(b & 12 == 12 for b in bits)
+            if done == 44:
+                assert all(b & 4 == 0 for b in bits)
+            if done == 74:
+                assert bits[0] & 12 == 12  # the one that did not melt
+        if write:  # hot gas populations and warm plate cells, as a host program may set them: one
+            # above the record's limit (the lowest HAZ threshold), one that remelts
             for t in (tw, ref):
                 p = t.grid.f_src.to_numpy()
                 p[5, nx // 2, ny // 3, nz - 3] += np.float32(0.01)
                 t.grid.f_src.from_numpy(p)
-                T = t.grid.T.to_numpy()
+                T, H = t.grid.T.to_numpy(), t.grid.H.to_numpy()
+                for j, warm, latent in ((1, 1200.0, 0.0), (2, t.mat.T_liquidus + 50.0, t.L_rho)):
+                    T[nx // 2, j, 1] = warm
+                    H[nx // 2, j, 1] = t.cp_rho * warm + latent
                 t.grid.T.from_numpy(T)
+                t.grid.H.from_numpy(H)
