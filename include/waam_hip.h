@@ -518,7 +518,7 @@ int waam_cadj_thermal_step(const double *lam_next, double *lam_out, double *lam_
  * n steps of the rollouts above with frozen flags and phi in one call: the values of the
  * per-kernel entries, in fewer launches. The state lives in slots of N = nx*ny*nz cells (u: 3 N,
  * f: 19 N): step t reads slot t and writes slot t + 1 (stack 1), or the two slots in turn from
- * slot0 on (stack 0). arc_i, arc_j (host, n doubles): the arc centre of each step, in cells;
+ * slot0 on (stack 0; T always unless flow is 2, since only the flow's backward reads it). arc_i, arc_j (host, n doubles): the arc centre of each step, in cells;
  * c.arc_i and c.arc_j are not read. */
 typedef struct waam_rollout {
     waam_adj_consts c;

@@ -30,7 +30,7 @@ def _stream():
 def _saved(ro, adv: bool, flow: bool) -> dict:
     """The state and saved fields of all the steps, as the backward lays them out."""
     n = ro.n_steps
-    sv = {k: ro._new(n + 1) for k in ("H", "T", "fl")}
+    sv = {k: ro._new(2 if k == "T" and not flow else n + 1) for k in ("H", "T", "fl")}
     sv.update({k: ro._new(n) for k in (("A", "B", "E", "F") if adv else ("A", "E", "F"))})
     if flow:
         sv.update(u=ro._new(n + 1, 3), f=ro._new(n + 1, 19), Fr=ro._new(n, 3), Fc=ro._new(n, 3))
@@ -140,8 +140,9 @@ def test_coupled_rollback_equals_its_entries(hip_device, mode, nx, ny, nz, layou
     grads, sums = torch.zeros(3, **D64), torch.zeros(2, **D64)
     for t in reversed(range(n)):
         c = ro._consts(t)
-        T1, fl1, H1 = sv["T"][t + 1], sv["fl"][t + 1], sv["H"][t + 1]
+        fl1, H1 = sv["fl"][t + 1], sv["H"][t + 1]
         if flow:
+            T1 = sv["T"][t + 1]
             lam_fl1.zero_()
             lam_T1.zero_()
             Fc, Fr = sv["Fc"][t], sv["Fr"][t]

@@ -199,3 +199,29 @@ def test_a_bad_efficiency_is_not_swallowed(hip_device, mode, eta, monkeypatch):
     assert np.isnan(want[0]).any() == math.isnan(eta)  # the ceiling bounds an infinite one
     for name, a, b in zip(("H", "T", "f_l"), (ro.H_final, T, fl), want):
         assert bits_equal(a.cpu().numpy(), b), mismatch_report(name, a.cpu().numpy(), b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode,fields", [("thermal", 5), ("none", 5), ("frozen", 6), ("flow", 35)])
+def test_backward_memory(hip_device, mode, fields):
+    """The backward holds so many fields for each step between two checkpoints, and a few more
+    besides: two of each state and adjoint in turn, and work buffers in binary64."""
+    from waam_solver_amd.adjoint import CoupledRollout, ThermalRollout
+
+    tw, path = _twin(64, 40, 32, 1)
+    n, field = 40, 4 * tw.grid.n_cells
+    ro = (ThermalRollout(tw, n, path, checkpoint_every=n) if mode == "thermal" else
+          CoupledRollout(tw, n, path, checkpoint_every=n, advection=mode))
+    T, _ = ro.forward(THETA)
+    seed = torch.ones_like(T)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    base = torch.cuda.memory_allocated()
+    ro.backward(seed, seed)
+    held = (torch.cuda.max_memory_allocated() - base - n * 6 * 1024 * 8) / field
+    print(f"[rollout] {mode}: {held:.1f} fields over {n} steps", flush=True)
+    # H and f_l at the last step, two of T; binary64 counts twice: the two seeds and dL/dH, dL/du
+    # (three each), dL/df (nineteen), lamC, lamB, and the flow's T1, fl1 and G. The allocator may
+    # hand out blocks up to 1 MiB (three fields) larger than asked: eight fields for those
+    few = 8 + {"thermal": 6, "none": 16, "frozen": 28, "flow": 140}[mode]
+    assert held < fields * n + few

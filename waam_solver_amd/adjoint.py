@@ -199,8 +199,9 @@ class ThermalRollout:
         gfl = grad_fl.float().contiguous()
         lib().call("waam_adj_terminal", P(self.H_final), P(gT), P(gfl), P(self.flags),
                    ctypes.addressof(c_last), P(lam), g.n_cells, st)
-        # a segment's state and saved fields, one slot a step, reused from segment to segment
-        sv = {k: self._new(L + 1) for k in ("H", "T", "fl")}
+        # a segment's state and saved fields, one slot a step (T, which only the forward reads: two
+        # in turn), reused from segment to segment
+        sv = {k: self._new(2 if k == "T" else L + 1) for k in ("H", "T", "fl")}
         sv.update({k: self._new(L) for k in ("A", "E", "F")})
         sv["sums"] = torch.empty(2 * L, dtype=torch.float64, device=dev)
         slot = 0
@@ -486,7 +487,8 @@ class CoupledRollout:
         lib().call("waam_cadj_phase", P(self.H_final), P(self.flags), ctypes.addressof(c_last),
                    P(gT), P(gfl), P(lam["lam_H"]), g.n_cells, st)
         # a segment's state and saved fields, one slot a step, reused from segment to segment
-        sv = {k: self._new(L + 1) for k in ("H", "T", "fl")}
+        # (T: two in turn where only the forward reads it)
+        sv = {k: self._new(2 if k == "T" and not flow else L + 1) for k in ("H", "T", "fl")}
         sv.update({k: self._new(L) for k in (("A", "B", "E", "F") if adv else ("A", "E", "F"))})
         if flow:
             sv.update(u=self._new(L + 1, 3), f=self._new(L + 1, 19), Fr=self._new(L, 3),

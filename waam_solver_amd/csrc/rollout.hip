@@ -411,6 +411,8 @@ extern "C" int waam_rollout_forward(const waam_rollout *r, const double *arc_i,
     double *parts = reinterpret_cast<double *>((char *)r->scratch + kScratchTelemetryParts);
     float *tot = reinterpret_cast<float *>((char *)r->scratch + kScratchTelemetry);
     auto slot = [&](int t) { return (size_t)(r->stack ? t : (r->slot0 + t) & 1); };
+    /* only the flow's backward reads the steps' temperatures: two slots do elsewhere */
+    auto slot_T = [&](int t) { return r->flow == 2 ? slot(t) : (size_t)((r->slot0 + t) & 1); };
     for (int t = 0; t < n; ++t) {
         const size_t s0 = slot(t), s1 = slot(t + 1);
         a.ap.arc_i = (float)arc_i[t];
@@ -430,10 +432,10 @@ extern "C" int waam_rollout_forward(const waam_rollout *r, const double *arc_i,
         const size_t sv = (size_t)t * N;
         auto launch = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, dim3(kReduceBlocks), dim3(kBlock), 0, st,
-                               (const float *)r->H + s0 * N, (const float *)r->T + s0 * N,
+                               (const float *)r->H + s0 * N, (const float *)r->T + slot_T(t) * N,
                                (const float *)r->fl + s0 * N, u, u ? u + N : u, u ? u + 2 * N : u,
                                r->flags, (const float *)r->depth, (const float *)tot, a,
-                               r->H + s1 * N, r->T + s1 * N, r->fl + s1 * N,
+                               r->H + s1 * N, r->T + slot_T(t + 1) * N, r->fl + s1 * N,
                                r->A ? r->A + sv : nullptr, r->A && r->B ? r->B + sv : nullptr,
                                r->A ? r->E + sv : nullptr, r->A ? r->F + sv : nullptr, parts);
         };
