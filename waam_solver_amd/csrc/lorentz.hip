@@ -674,8 +674,15 @@ k_elec_J_bins(float *__restrict__ Jx, float *__restrict__ Jy, float *__restrict_
     const int64_t slab = (int64_t)d.ny * d.nx;
     const int64_t up = k + 1 < d.nz ? slab : 0, down = k > 0 ? -slab : 0;
     int n = 0;
-    auto compute = [&]() {
+    /* the list passes between lanes of one wavefront, whose LDS accesses keep their order: what
+     * must not happen is that the compiler moves them past each other */
+    auto handover = []() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    auto compute = [&]() {
+        handover();
         for (int q = lane; q < n; q += 64) {
             const uint32_t w = list[q];
             const int b = (int)(w % kJBinGroup), t = (int)(w / kJBinGroup);
@@ -702,7 +709,7 @@ k_elec_J_bins(float *__restrict__ Jx, float *__restrict__ Jy, float *__restrict_
                 }
         }
         n = 0;
-        __builtin_amdgcn_wave_barrier();
+        handover();
     };
     /* squared radii that the exact test need not see, a little wide; the last bin takes everything
      * beyond it */
