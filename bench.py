@@ -169,8 +169,9 @@ def cpu_baseline(w: dict, seconds: float, one_thread_steps: int) -> dict:
 # the listed row segments (on grids that do not fill the chip the surface cells share the launch).
 # Its algorithmic bytes per launch are those of the SOLID cells, each array element touched once
 # (neighbour re-reads and the listed GAS cells not counted):
-#   SOLID cell          H, T, T_prev, T_max read; H, T, T_prev, dT/dt written       32 B
-THERMAL_B_SOLID = 32
+#   SOLID cell          H, T, T_max read; H, T, T_prev, dT/dt written                28 B
+# (a cold plate cell's T_prev is the T it holds; the few warm ones, which are walked, read it too)
+THERMAL_B_SOLID = 28
 # What a whole step cannot do without: the SOLID cells' chain as above, and for each collided
 # (FLUID/IFACE) cell
 #   H T f_l phi r/w 32 B, u r/w 24 B, flags r/w 2 B, rho w 4 B, HAZ fields (T_max r/w, T_prev r/w,

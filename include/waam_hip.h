@@ -804,7 +804,11 @@ int waam_graph_destroy(waam_step_graph *g);
  * (one of WAAM_K_*); waam_timing_begin_every records only every `every`-th launch of it (the
  * events add a few microseconds around each recorded dispatch); waam_timing_end waits for the
  * recorded events, returns the summed duration and the number of timed launches, and disarms.
- * Process-wide, one kernel at a time; not for concurrent use from several threads. */
+ * Process-wide, one kernel at a time; not for concurrent use from several threads.
+ * A kernel that shares another's launch records none of its own: on steady steps
+ * (waam_step_params.quiet_skip) the tracers are part of WAAM_K_PULL in the ZYX layout, and the
+ * surface cells of WAAM_K_THERMAL on grids that do not fill the chip; WAAM_K_BEGIN then carries the
+ * segment list. WAAM_K_PULL records none where the pull runs inside kernel 7. */
 enum {
     WAAM_K_BEGIN = 0,
     WAAM_K_THERMAL = 1,

@@ -13,8 +13,8 @@
 namespace waam {
 
 /* A lane per cell of the linear index, so that rows of any length fill their wavefronts (64-lane
- * row tiles left half the wavefronts of the 66-cell rows two cells: 22.8 us a step, 64^3). The
- * populations and flags of the 19 sources load together; the cell's own populations, which only
+ * row tiles left half the wavefronts of the 66-cell rows of 64^3 two cells). The populations and
+ * flags of the 19 sources load together; the cell's own populations, which only
  * bounce back, load where a source is a wall. 64^3 fluid cells move 44 MB a step through the
  * Infinity Cache in 15.7 us (2.8 TB/s; 23.3 with the row tiles, every own population loaded and
  * 64-bit indices), 128^3 334 MB in 96 (3.5 TB/s; 143). Bound by the 38 loads a lane issues, half

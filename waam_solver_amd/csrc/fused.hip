@@ -324,7 +324,7 @@ __host__ __device__ inline size_t quiet_pull_offset(const Dims &d)
 }
 /* then, 256-aligned, the pull's own record (PullRec): its count on a line of its own, the change
  * and edge words of both population buffers, and its list (every segment once, and once more by
- * kernel 7) */
+ * kernel 4, ahead of the pull) */
 __host__ __device__ inline size_t quiet_still_offset(const Dims &d)
 {
     return (quiet_pull_offset(d) + (d.n() + 1) / 2 + 255) / 256 * 256;
@@ -1568,13 +1568,13 @@ __device__ __forceinline__ void thermal_walk(const waam_step_fields &f, const St
     });
 }
 
-/* the march in a launch of its own (a plate past kTogetherBlocks) */
+/* the march in a launch of its own (see thermal_together) */
 __global__ void __launch_bounds__(256) k_step_thermal_plate(waam_step_fields f, StepConsts s)
 {
     plate_march(f, s, stored_epw(f), (int)blockIdx.x);
 }
 
-/* the walk in a launch of its own (temperature-dependent material, or a plate of that size) */
+/* the walk in a launch of its own (see thermal_together) */
 template <bool TAB>
 __global__ void __launch_bounds__(256) k_step_thermal_seg(waam_step_fields f, StepConsts s)
 {

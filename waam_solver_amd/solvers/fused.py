@@ -1,13 +1,15 @@
 """The fused coupled step: one ``waam_step_fused`` call per timestep.
 
 Same results as ``coupled_step`` (the kernel-per-reference-kernel sequence) — the parity tests
-run both against the oracle — in seven launches and without host round trips on ordinary
+run both against the oracle — in six to nine launches and without host round trips on ordinary
 steps (arc_k is found and used on the device). The last kernel of a step lists the cells that
-end it FLUID/IFACE; the next step works through that list in the same launch as its thermal
-sweep, provided no host write (``field.write_epoch``) came in between; otherwise the sweep
-builds the list and one more launch consumes it. Steps on which a droplet detaches go through
-the standalone arc, deposition and impact kernels first (one host read of arc_k and of the
-placed volume), then the fused kernels with the arc marked as applied.
+end it FLUID/IFACE; the next step works through that list, on most grids in the same launch as its
+thermal sweep, provided no host write (``field.write_epoch``) came in between; otherwise the sweep
+builds the list and one more launch consumes it. Steps on which a droplet detaches run whole on
+the device as well (``waam_step_fused_droplet``); the conical source's go through the standalone
+arc, deposition and impact kernels first (host reads of arc_k and of the placed volume), then the
+fused kernels with the arc marked as applied. A step with the Lorentz force reads its solve's
+convergence test back.
 
 Buffer pairs: the grid holds H/H_tmp, T/T_tmp, f_l/fl_tmp, flags/flags_tmp and
 sflags/sflags_tmp; after each fused step every pair swaps, as do the population buffers. The

@@ -160,7 +160,7 @@ class WAAMTwin:
         self._interpass_cooling_steps = 0
         self.snapshot_forces = True
         self.tracer_seed = 0
-        # "fused": waam_step_fused (eight launches per step, the default); "reference": one
+        # "fused": waam_step_fused (six to nine launches per step, the default); "reference": one
         # launch per reference kernel in the reference's order. Both give identical fields.
         self.engine = "fused"
         # fused steps keep the populations as fp32 ("fp32") or as f - w_q in 16 bits ("fp16",
